@@ -311,29 +311,18 @@ HELIX_DEV unsigned pk_bf16(float a, float b) {
 HELIX_DEV float pk_lo(unsigned w) { return __builtin_bit_cast(float, w << 16); }
 HELIX_DEV float pk_hi(unsigned w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 
-// a - lo(w) and a - hi(w) for a packed bf16 pair w, each one v_dot2_f32_bf16:
-// w . (-1, 0) + a. Where w is a's own bf16 rounding (or that of a residual of
-// it) the difference is exactly representable in fp32, and the bf16 products
-// are exact, so the result is exact: the same value as unpacking the half and
-// subtracting, in one operation instead of two. The (-1, 0) and (0, -1) pairs
-// reach the instruction in a scalar register: the compiler would otherwise
-// encode the first as the inline constant -1.0, which the hardware applies as
-// the fp32 bit pattern 0xbf800000, i.e. the pair (0, -1) (measured).
-HELIX_DEV unsigned bf16_pair_reg(unsigned k) {
-    asm("" : "+s"(k));
-    return k;
-}
-HELIX_DEV float sub_lo(float a, unsigned w) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w),
-                                           __builtin_bit_cast(bf16x2, bf16_pair_reg(0x0000bf80u)), a, false);
-}
-HELIX_DEV float sub_hi(float a, unsigned w) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w),
-                                           __builtin_bit_cast(bf16x2, bf16_pair_reg(0xbf800000u)), a, false);
-}
+// a - lo(w) and a - hi(w) for a packed bf16 pair w; exact where w is a's own
+// bf16 rounding (or that of a residual of it). Unpacked and subtracted, two
+// operations: v_dot2_f32_bf16 does it in one, but a dot product shares the
+// matrix pipe. Behind each 16 x 16 x 32 MFMA (18 cycles alone, two waves per
+// SIMD) two dot products took the pair to 39 cycles and four to 48, two and
+// four subtractions to 18 and 27; at config 2's shape the fp32 path's walk took
+// 164 us with the dot products and 161 without.
+HELIX_DEV float sub_lo(float a, unsigned w) { return a - pk_lo(w); }
+HELIX_DEV float sub_hi(float a, unsigned w) { return a - pk_hi(w); }
 
 // Three-way bf16 split of the pair (a, b), each part packed as a pair:
-// 7 VALU operations for two values.
+// 11 VALU operations for two values.
 HELIX_DEV void split3_pair(float a, float b, unsigned& w0, unsigned& w1, unsigned& w2) {
     w0 = pk_bf16(a, b);
     const float ra = sub_lo(a, w0), rb = sub_hi(b, w0);
@@ -342,7 +331,7 @@ HELIX_DEV void split3_pair(float a, float b, unsigned& w0, unsigned& w1, unsigne
 }
 
 // Two-way bf16 split of the pair (a, b): v = v0 + v1 + e with |e| <= 2^-18 |v|,
-// 4 VALU operations for two values. Three products a0b0 + a0b1 + a1b0 leave
+// 6 VALU operations for two values. Three products a0b0 + a0b1 + a1b0 leave
 // out terms of at most 3 * 2^-18 of |ab| (about 1.1e-5).
 HELIX_DEV void split2_pair(float a, float b, unsigned& w0, unsigned& w1) {
     w0 = pk_bf16(a, b);
@@ -635,6 +624,12 @@ HELIX_DEV int vgpr_fresh(int v) {
     asm volatile("" : "+v"(v));
     return v;
 }
+
+// Scheduling fence for the vector memory instructions only: loads and stores
+// stay where the program puts them (so a refill never moves above the last use
+// of the registers it overwrites, and the in-order vmcnt waits keep their
+// distance), while ALU, MFMA and LDS work may still be interleaved across it.
+HELIX_DEV void vmem_fence() { __builtin_amdgcn_sched_barrier(0x0001 | 0x0002 | 0x0004 | 0x0008 | 0x0080 | 0x0400); }
 
 // Load of a wave-uniform element through the scalar unit (s_load, counted by
 // lgkmcnt): reading through the constant address space tells the compiler the

@@ -78,13 +78,13 @@ HELIX_DEV unsigned pk_f16(float a, float b) {
 }
 
 // Two-way fp16 split of the pair (a, b), 4 VALU operations: the residuals
-// a - v0 are exact in fp32, each one v_dot2_f32_f16 of the packed pair with
-// (-1, 0) or (0, -1), held in a scalar register (bf16_pair_reg).
+// a - v0 are exact in fp32, each one v_fma_mix_f32 (not a dot product, which
+// would share the matrix pipe: see sub_lo).
 HELIX_DEV void split2h_pair(float a, float b, unsigned& w0, unsigned& w1) {
     w0 = pk_f16(a, b);
     const f16x2 h = __builtin_bit_cast(f16x2, w0);
-    const float ra = __builtin_amdgcn_fdot2(h, __builtin_bit_cast(f16x2, bf16_pair_reg(0x0000bc00u)), a, false);
-    const float rb = __builtin_amdgcn_fdot2(h, __builtin_bit_cast(f16x2, bf16_pair_reg(0xbc000000u)), b, false);
+    const float ra = __builtin_fmaf((float)h[0], -1.0f, a);
+    const float rb = __builtin_fmaf((float)h[1], -1.0f, b);
     w1 = pk_f16(ra, rb);
 }
 
@@ -221,12 +221,6 @@ HELIX_DEV float hb_load_dt(const HelixScanParams& p, const float* __restrict__ d
     const helix_rsrc rdt = make_rsrc(dt_h + (long long)t0 * p.s_dt[0], ((tlen - 1) * sdt + 1) * 4u);
     return buf_f32(rdt, min(lane, tlen - 1) * sdt * 4, 0);
 }
-
-// Scheduling fence for the vector memory instructions only: loads and stores
-// stay where the program puts them (so a refill never moves above the last use
-// of the registers it overwrites, and the in-order vmcnt waits keep their
-// distance), while ALU, MFMA and LDS work may still be interleaved across it.
-HELIX_DEV void vmem_fence() { __builtin_amdgcn_sched_barrier(0x0001 | 0x0002 | 0x0004 | 0x0008 | 0x0080 | 0x0400); }
 
 // B rows (and C rows, for a copying wave) of chunk c. Rows clamp to the last
 // valid token and state indices to d_state, so every load is in bounds; a wave

@@ -136,9 +136,8 @@ __device__ __forceinline__ void store_y_tile(const f32x16& acc, const HelixScanP
 // y[t = 16 tb + 4 q + r][pp]. Rows past tlen and columns past the slab width
 // are dropped by the range check; with tlen <= 0 nothing is stored. AUX: the
 // stores' cache policy (HELIX_NT, or HELIX_NT_L2 for the walk on Pass A's
-// bf16 copies of B and C). RT_ACC: add what y holds when p.y_acc is set (off
-// for a caller that loaded it ahead with load_y16 and added it to acc).
-template <typename IO, int AUX = HELIX_NT, bool RT_ACC = true>
+// bf16 copies of B and C).
+template <typename IO, int AUX = HELIX_NT>
 __device__ __forceinline__ void store_y16(const f32x4 (&acc)[4], const HelixScanParams& p,
                                           const HelixScanBuffers& b, int seq, int h, int t0, int tlen,
                                           int p0, int pw, int pp, int q) {
@@ -149,21 +148,14 @@ __device__ __forceinline__ void store_y16(const f32x4 (&acc)[4], const HelixScan
                                         (long long)t0 * p.s_y[0] + (long long)p0 * p.s_y[2],
                                     bytes);
     const int voff = (4 * q * sy0 + pp * sy2) * ES;
-    auto put = [&](auto acc_on) {
 #pragma unroll
-        for (int tb = 0; tb < 4; ++tb)
+    for (int tb = 0; tb < 4; ++tb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 16 * tb + 4 * q + r;
-                const float v = acc[tb][r];
-                y_store<IO, decltype(acc_on)::value, AUX>(ry, v, store_off_if_lt(voff, t, tlen, pp, pw),
-                                                          (16 * tb + r) * sy0 * ES);
-            }
-    };
-    if constexpr (RT_ACC)
-        with_y_acc(p, put);
-    else
-        put(std::false_type{});
+        for (int r = 0; r < 4; ++r) {
+            const int t = 16 * tb + 4 * q + r;
+            const float v = acc[tb][r];
+            y_store<IO, false, AUX>(ry, v, store_off_if_lt(voff, t, tlen, pp, pw), (16 * tb + r) * sy0 * ES);
+        }
 }
 
 // What y holds at the elements store_y16 would store (fp32 storage), 0 where
@@ -191,9 +183,8 @@ __device__ __forceinline__ void load_y16(f32x4 (&yv)[4], const HelixScanParams& 
 // = S[16 nb + 4 q + r][p0 + pp] (q = lane / 16, pp = 16 w4 + c16). Without
 // p.fuse_b it is Pass B's S_seg tile of the Pass A segment the walk segment
 // starts at; with p.fuse_b the tiles hold Pass A's segment aggregates and the
-// workgroup runs Pass B's recurrence here. YT: the single pass without
-// scratch (HelixScanParams::ytile, never with fuse_b): the tile is in y.
-template <int NP, bool YT = false>
+// workgroup runs Pass B's recurrence here.
+template <int NP>
 __device__ __forceinline__ void walk_start_state(f32x4 (&R)[NP / 16], const HelixScanParams& p,
                                                  const HelixScanBuffers& b, int seq, int h, int slab, int seg,
                                                  int p0, int pw, int pp, int q, int w4, int c16, bool head_ok) {
@@ -203,25 +194,9 @@ __device__ __forceinline__ void walk_start_state(f32x4 (&R)[NP / 16], const Heli
     // tile's unit layout that is unit ((pt NT32 + nb/2) 4 + r4) 64 + lane'
     // with pt = w4/2, r4 = 2 (nb%2) + q/2, lane' = 32 (q%2) + 16 (w4%2) + c16.
     {
-        const float* tiles = YT ? nullptr : b.s_seg + seq * p.sg_seq + state_tile_off(p, h, slab);
+        const float* tiles = b.s_seg + seq * p.sg_seq + state_tile_off(p, h, slab);
         const int vunit = 64 * (q >> 1) + 32 * (q & 1) + 16 * (w4 & 1) + c16;
         const int pt = w4 >> 1;
-        if constexpr (YT) {
-            // The tile of the walk's first Pass A segment, in y's rows of that
-            // segment and the slab's columns (ytile_unit); the range covers
-            // the rows the tile and its log-decay take.
-            const int s = seg * (p.walk_len / p.seg_len);
-            const int upr = pw >> 2;
-            const unsigned rows = (unsigned)((16 * NP + 1 + upr - 1) / upr);
-            const helix_rsrc ry = make_rsrc(b.y + ytile_base(p, seq, h, slab, s), rows * (unsigned)p.s_y[0] * 4u);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                const int u = vunit + ((pt * NT32 + (nb >> 1)) * 4 + 2 * (nb & 1)) * 64;
-                R[nb] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                      ry, (int)ytile_unit(p, u, pw) * 4, 0, 0));
-            }
-            return;
-        }
         auto load_tile = [&](int s, f32x4 (&T)[NB]) {
             const helix_rsrc rg = make_rsrc(tiles + (long long)s * p.sg_seg, 64u * NP * sizeof(float));
 #pragma unroll

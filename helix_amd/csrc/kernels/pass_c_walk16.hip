@@ -472,10 +472,8 @@ __device__ __forceinline__ void scan_walk16_impl(const HelixScanParams& p, const
         if constexpr (YACC) {
 #pragma unroll
             for (int tb = 0; tb < 4; ++tb) acc[tb] += yprev[tb];
-            store_y16<IO, YAUX, false>(acc, p, b, seq, h, t0, head_ok ? tlen : 0, p0, pw, pp, q);
-        } else {
-            store_y16<IO, YAUX>(acc, p, b, seq, h, t0, head_ok ? tlen : 0, p0, pw, pp, q);
         }
+        store_y16<IO, YAUX>(acc, p, b, seq, h, t0, head_ok ? tlen : 0, p0, pw, pp, q);
 
         if constexpr (M_IN_B) __syncthreads();
     }

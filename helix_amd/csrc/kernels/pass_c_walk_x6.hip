@@ -1,63 +1,108 @@
-// pass_c_walk_x6.hip -- the fp32 path's Pass C: the chunk walk on bf16x6 products.
+// pass_c_walk_x6.hip -- the fp32 path's Pass C: the chunk walk on bf16x6 products,
+// four (head, P slab) items of one B/C group per workgroup.
 //
 // Reference counterpart: helix_chunk_out_f32 (src/kernels/
-// helix_scan_multipass.metal:225-361). Like the bf16 path's walk
-// (pass_c_walk16.hip), one workgroup walks a segment of chunks from the
-// segment's start state S_seg (Pass B) and forms every chunk's own start
-// state R on the way, producing per chunk
+// helix_scan_multipass.metal:225-361). One workgroup walks a run of chunks
+// from its start state S_seg (Pass B) and forms every chunk's own start state R
+// on the way, producing per chunk
 //     y = tril(C B^T . decay) (dt x) + exp(Lcum) . (C R)        (G1, G2, G3)
 //     R <- exp(L_end) R + B^T . (decay . dt . x)                  (G4)
-// Here every product keeps fp32 accuracy: v_mfma_f32_16x16x32_bf16 over
-// operands split into three bf16 parts (six products, fp32 accumulation),
-// and R stays in fp32 registers. Against the chunk-parallel bf16x6 Pass C
-// (pass_c_x6.hip), whose per-chunk start states Pass A writes and Pass C
-// reads back, the walk moves half the bytes.
+// Every product keeps fp32 accuracy: bf16 MFMA over operands split into three
+// bf16 parts (six products, fp32 accumulation), R in fp32 registers. Against
+// the chunk-parallel bf16x6 Pass C (pass_c_x6.hip), whose per-chunk start
+// states Pass A writes and Pass C reads back, the walk moves half the bytes.
 //
-// Workgroup: (seq, walk segment, two heads of one B/C group, 64-wide P slab),
-// eight waves; wave (hw, w4) owns P columns 16 w4 .. 16 w4 + 15 of head hw:
-//   - R[n][p] for its 16 columns: NP/16 result tiles, register r of tile nb
-//     holding R[16 nb + 4 (lane/16) + r][p];
-//   - G3 and G4 on those tiles, G2 on its columns;
-//   - G1 (C B^T, the same for both heads) split over the eight waves by
-//     16 x 16 block; each head's M = C B^T . decay shared through LDS.
-// K order: within each group of 32 state indices, index 16 h + 4 q + r sits at
-// K position 8 q + 4 h + r (perm32) in the C and B rows, so R's registers are
-// G3's operand as they stand (the layout of the bf16 walk).
+// What bounds it is the sum of its matrix and vector work: under bf16 MFMA load
+// the part runs at 1.8-2.0 GHz, not 2.4, and vector instructions add to the
+// matrix time (44 of them for every 12 products of 32 x 32 x 16: 470 -> 600 cycles
+// a wave pair, whatever their order; reordering this kernel's phases, mixing
+// them by scheduling groups or giving a SIMD's two waves opposite orders
+// changed nothing or cost time). So the layout does less of both per head:
+//   - Wave w owns item w % 4 and its P columns 32 (w / 4) .. + 31 for all 64
+//     tokens and every state index: G2, G3 and G4 run on 32 x 32 tiles, and a
+//     C or B^T fragment read from LDS feeds 32 columns.
+//   - B and C are split once per workgroup, for four items.
+//   - x goes straight from memory into the operand layout (lane = column,
+//     tokens 16 s + 8 hi + e), as in Pass A, and never touches LDS.
+//   - G1 (C B^T, the same for the four items) runs on ten 16 x 16 blocks over
+//     the eight waves and is shared as fp32; each wave forms its own M = C B^T
+//     . decay operand in registers. The heads' M planes would not fit the LDS.
+//   - The run's last chunk leaves no state (Pass B has it): no G4.
+// The fp32 path's scan at L=8192 H=64 P=64 N=128 G=8 went from 237 to 199 us, at
+// L=2048 from 75 to 69, at 4 x 1000 tokens of 32 heads of 128 from 128 to 109,
+// against waves of 16 columns, two heads per workgroup, M planes in LDS.
 //
-// LDS, three bf16 planes per operand in the x6_off layout (no padding):
-//   C    [64 t][NP n]   perm32 n order             G1, G3
-//   B    [64 j][NP n]   perm32 n order             G1; afterwards the region
-//   M    [64 t][64 j]   one per head               holds the heads' M (G2)
-//   B^T  [NP n][64 j]   natural n order            G4
-// and the heads' decay records: 145 KiB at d_state 128 (one workgroup per
-// CU), 98 KiB at d_state 64.
-// The B operands of G2 and G4 (dt x and decay dt x at the lane's own column
-// and K tokens) and of G3 (R) are split in registers.
+// K order: index 16 s + 8 a + 4 b + r of a group of 16 state indices (a, b in
+// {0, 1}) sits at K position 8 b + 4 a + r in the C rows (perm16), so R's result
+// registers (lane hi = b) are G3's operand as they stand.
+//
+// LDS, rows padded by 8 elements (16 consecutive operand rows start on 16
+// distinct groups of four banks, and every access of the chunk loop is a
+// per-lane base plus an immediate offset; an XOR swizzle spent a quarter of the
+// vector instructions on addresses):
+//   C    [64 t][NP n]   three bf16 planes, perm16 n order      G1, G3
+//   B^T  [NP n][64 j]   three bf16 planes, natural order       G1, G4
+//   CB   [64 t][64 j]   fp32, blocks on or below the diagonal  G2
+// and the decay records of two chunks: 132 KiB at d_state 128, one workgroup
+// per CU.
 #include "helix_common.h"
 
-#include "pass_c_stage.h"
+// Split planes of a caller's B and C value: three bf16 parts of fp32, one of a
+// bf16 value, two of an f16 value (11 significant bits: both exact).
+template <typename IO> struct WX6Planes { static constexpr int value = 3; };
+template <> struct WX6Planes<__bf16> { static constexpr int value = 1; };
+template <> struct WX6Planes<_Float16> { static constexpr int value = 2; };
 
-// Six 16 x 16 x 32 products of split operands a[3] x b[3], smallest terms first.
-HELIX_DEV f32x4 wx6_mfma(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x4 acc) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], acc, 0, 0, 0);
+// The pair (a, b) as NPL packed bf16 parts (NPL 1 and 2: exact for values of
+// that many parts).
+template <int NPL>
+HELIX_DEV void wx6_split(float a, float b, unsigned (&w)[NPL]) {
+    if constexpr (NPL == 3)
+        split3_pair(a, b, w[0], w[1], w[2]);
+    else if constexpr (NPL == 2)
+        split2_pair(a, b, w[0], w[1]);
+    else
+        w[0] = pk_bf16(a, b);
+}
+// Eight values as the planes of one MFMA operand.
+template <int NPL>
+HELIX_DEV void wx6_split8(const float (&v)[8], bf16x8 (&o)[NPL]) {
+    u32x4 q[NPL];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        unsigned w[NPL];
+        wx6_split<NPL>(v[2 * e], v[2 * e + 1], w);
+#pragma unroll
+        for (int k = 0; k < NPL; ++k) q[k][e] = w[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NPL; ++k) o[k] = __builtin_bit_cast(bf16x8, q[k]);
+}
+
+// Products of split operands a[NA] x b[NB], smallest terms first: those of the
+// parts (i, j) with i + j <= 2 (six for three parts of each).
+template <int NA, int NB>
+HELIX_DEV f32x16 wx6_mfma(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x16 acc) {
+#pragma unroll
+    for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+        for (int i = sum; i >= 0; --i)
+            if (i < NA && sum - i < NB) acc = mfma_bf16(a[i], b[sum - i], acc);
+    return acc;
+}
+template <int NA, int NB>
+HELIX_DEV f32x4 wx6_mfma16(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x4 acc) {
+#pragma unroll
+    for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+        for (int i = sum; i >= 0; --i)
+            if (i < NA && sum - i < NB) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[sum - i], acc, 0, 0, 0);
     return acc;
 }
 
-// v, opaque to the optimizer (it stays in a VGPR and is not known to be
-// loop-invariant).
-HELIX_DEV int vgpr_opaque(int v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
-// K position of state index i inside its group of 32: 16 h + 4 q + r -> 8 q + 4 h + r.
-HELIX_DEV int wx6_perm32(int i) {
-    return (i & ~31) | (8 * ((i >> 2) & 3) + 4 * ((i >> 4) & 1) + (i & 3));
+// K position of state index i inside its group of 16: 8 a + 4 b + r -> 8 b + 4 a + r.
+HELIX_DEV int wx6_perm16(int i) {
+    return (i & ~12) | ((i & 4) << 1) | ((i & 8) >> 1);
 }
 
 // G1 block idx (0..9) of the lower triangle of the 4 x 4 grid of 16 x 16
@@ -68,132 +113,273 @@ HELIX_DEV int wx6_jb(int idx) {
     return idx - tb * (tb + 1) / 2;
 }
 
-// This lane's B and C runs of one chunk (fp32) of rows j0 and j0 + 1: NH
-// 16-byte words per row, state indices 8u + 4 hh .. + 3 for hh = 0 .. NH - 1
-// (d_state 128: NH = 2, the whole run 8u .. 8u + 7) or for hh = hf alone
-// (d_state 64: NH = 1, lanes 8 apart take the run's two halves).
-template <int NH>
-struct RunsWX6 {
-    u32x4 b[2][NH], c[2][NH];
+constexpr int WX6_RSJ = HELIX_CS + 8;              // B^T rows (elements)
+constexpr int WX6_RSM = HELIX_CS + 4;              // CB rows (floats)
+template <int NP> constexpr int WX6_RSC = NP + 8;  // C rows (elements)
+
+// A thread's C rows of a chunk: rows 8 wave + 2 (lane / 16) and the next, a run
+// of NP / 16 state indices each (eight at d_state 128, half of such a run at 64).
+template <int NP>
+HELIX_DEV void wx6_c_run(int lane, int wave, int& j, int& n, int& pos) {
+    const int c16 = lane & 15;
+    const int u = NP == 128 ? c16 : (c16 & 7), hf = NP == 128 ? 0 : (c16 >> 3);
+    j = 8 * wave + 2 * (lane >> 4);
+    n = 8 * u + 4 * hf;
+    pos = wx6_perm16(n);    // n + 4 sits 8 further
+}
+// Its B rows: NP / 32 consecutive tokens of four state indices, lane bits
+// placed so that a load instruction reads runs of 256 bytes and 16 consecutive
+// lanes write 16 distinct bank pairs of B^T.
+template <int NP>
+HELIX_DEV void wx6_b_rows(int lane, int wave, int& n, int& t) {
+    if constexpr (NP == 128) {
+        n = 64 * (wave >> 2) + 4 * ((lane & 3) | ((lane >> 4) << 2));
+        t = 16 * (wave & 3) + 4 * ((lane >> 2) & 3);
+    } else {
+        n = 4 * (lane & 15);
+        t = 8 * wave + 2 * (lane >> 4);
+    }
+}
+
+// NE consecutive elements of IO at byte offset off, in storage form.
+template <typename IO, int NE>
+struct WX6Run {
+    static constexpr int W = NE * (int)sizeof(IO) / 4;
+    unsigned w[W];
+    __device__ __forceinline__ void load(helix_rsrc rs, int off) {
+        if constexpr (W == 2) {
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
+            w[0] = v[0];
+            w[1] = v[1];
+        } else {
+#pragma unroll
+            for (int k = 0; k < W; k += 4) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 4 * k, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[k + e] = v[e];
+            }
+        }
+    }
+    __device__ __forceinline__ float at(int e) const {
+        if constexpr (sizeof(IO) == 4)
+            return as_f32(w[e]);
+        else
+            return io_f32<IO>((unsigned short)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu)));
+    }
 };
 
-template <int NH>
-__device__ __forceinline__ void load_runs_x6(RunsWX6<NH>& r, const HelixScanParams& p, const float* __restrict__ B_g,
-                                             const float* __restrict__ C_g, int c, int N, int j0, int u, int hf) {
-    const int t0   = (p.chunk_base + c) * HELIX_CS;
-    const int tlen = min(HELIX_CS, p.n_tok - t0);
-    const int sb0 = sgpr_fresh((int)p.s_b[0]), sc0 = sgpr_fresh((int)p.s_c[0]);
-    const helix_rsrc rb = make_rsrc(B_g + (long long)t0 * p.s_b[0], ((tlen - 1) * sb0 + N) * 4u);
-    const helix_rsrc rc = make_rsrc(C_g + (long long)t0 * p.s_c[0], ((tlen - 1) * sc0 + N) * 4u);
-    const int n0 = min(8 * u, N - 8);   // d_state % 8 == 0: a run is all in or out
+// A walk's y tiles of one chunk and item (32 x 32 MFMA layout, lane (hi, lo) of
+// P column pp): tile tb's register 4 r4 + r is y[t = 32 tb + 8 r4 + 4 hi +
+// r][pp]. f(rsrc, byte offset, scalar byte offset, tb, register) for each; rows
+// past tlen and columns past the slab width get an offset past the resource's
+// range, which drops a store and reads 0; with tlen <= 0 everything is out of
+// range. Where a token row of y is longer than the slab (every layout with
+// channels innermost) rows past tlen are out of range by themselves and one
+// offset serves every row.
+template <int ES, typename Buf, typename F>
+__device__ __forceinline__ void wx6_for_y(Buf* y, const HelixScanParams& p, int seq, int h, int t0, int tlen, int p0,
+                                        int pw, int pp, int hi, F&& f) {
+    const int sy0 = sgpr_fresh((int)p.s_y[0]), sy2 = (int)p.s_y[2];
+    const unsigned bytes = tlen > 0 ? ((tlen - 1) * sy0 + (pw - 1) * sy2 + 1) * (unsigned)ES : 0u;
+    const helix_rsrc ry = make_rsrc_u(y + seq * p.seq_y + h * p.s_y[1] + (long long)t0 * p.s_y[0] +
+                                          (long long)p0 * p.s_y[2],
+                                      bytes);
+    const int voff = (4 * hi * sy0 + pp * sy2) * ES;
+    if (sy0 > (pw - 1) * sy2) {
+        const int v = store_off_if_lt(voff, pp, pw, 0, 1);
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int jr = min(j0 + k, tlen - 1);
+        for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-        for (int w = 0; w < NH; ++w) {
-            const int hh = NH == 2 ? w : hf;
-            r.b[k][w] = __builtin_amdgcn_raw_buffer_load_b128(rb, (n0 + jr * sb0) * 4 + 16 * hh, 0, 0);
-            r.c[k][w] = __builtin_amdgcn_raw_buffer_load_b128(rc, (n0 + jr * sc0) * 4 + 16 * hh, 0, 0);
+            for (int r = 0; r < 16; ++r) f(ry, v, (32 * tb + 8 * (r >> 2) + (r & 3)) * sy0 * ES, tb, r);
+    } else {
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                f(ry, store_off_if_lt(voff, 32 * tb + acc_row(r, hi), tlen, pp, pw),
+                  (32 * tb + 8 * (r >> 2) + (r & 3)) * sy0 * ES, tb, r);
+    }
+}
+template <typename IO, int AUX>
+__device__ __forceinline__ void wx6_store_y(const f32x16 (&acc)[2], const HelixScanParams& p,
+                                               const HelixScanBuffers& b, int seq, int h, int t0, int tlen, int p0,
+                                               int pw, int pp, int hi) {
+    wx6_for_y<(int)sizeof(IO)>(reinterpret_cast<IO*>(b.y), p, seq, h, t0, tlen, p0, pw, pp, hi,
+                             [&](helix_rsrc ry, int voff, int soff, int tb, int r) {
+                                 const float v = acc[tb][r];
+                                 y_store<IO, false, AUX>(ry, v, voff, soff);
+                             });
+}
+// What y holds at the elements wx6_store_y would store (fp32 storage), 0
+// where it would store nothing: for a walk that adds into y, loaded a chunk's
+// work ahead of the stores.
+__device__ __forceinline__ void wx6_load_y(f32x16 (&yv)[2], const HelixScanParams& p, const HelixScanBuffers& b,
+                                              int seq, int h, int t0, int tlen, int p0, int pw, int pp, int hi) {
+    wx6_for_y<4>(b.y, p, seq, h, t0, tlen, p0, pw, pp, hi,
+               [&](helix_rsrc ry, int voff, int soff, int tb, int r) { yv[tb][r] = buf_f32(ry, voff, soff); });
+}
+
+// The start state R of a walk segment: R[nt] register 4 r4 + r = S[32 nt + 8 r4
+// + 4 hi + r][p0 + 32 pt + lo], a lane's units of the state tile as they stand
+// (helix_params.h). Without p.fuse_b it is Pass B's S_seg tile of the Pass A
+// segment the walk segment starts at; with p.fuse_b the tiles hold Pass A's
+// segment aggregates and the wave runs Pass B's recurrence here. YT: the single
+// pass without scratch (HelixScanParams::ytile, never with fuse_b): the tile is
+// in y.
+template <int NP, bool YT>
+__device__ __forceinline__ void wx6_start_state(f32x16 (&R)[NP / 32], const HelixScanParams& p,
+                                                   const HelixScanBuffers& b, int seq, int h, int slab, int seg,
+                                                   int p0, int pw, int pt, int lane, bool item_ok) {
+    constexpr int NT = NP / 32;
+    const int lo = lane & 31, hi = lane >> 5;
+    const int N = p.d_state, pp = 32 * pt + lo;
+    auto put = [](f32x16& t, int r4, f32x4 v) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[4 * r4 + r] = v[r];
+    };
+    if constexpr (YT) {
+        // The tile of the walk's first Pass A segment, in y's rows of that
+        // segment and the slab's columns (ytile_unit); the range covers the
+        // rows the tile and its log-decay take.
+        const int s = seg * (p.walk_len / p.seg_len);
+        const int upr = pw >> 2;
+        const unsigned rows = (unsigned)((16 * NP + 1 + upr - 1) / upr);
+        const helix_rsrc ry = make_rsrc_u(b.y + ytile_base(p, seq, h, slab, s), rows * (unsigned)p.s_y[0] * 4u);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+                put(R[nt], r4, __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                            ry, (int)ytile_unit(p, tile_unit(NT, pt, nt, r4, lane), pw) * 4, 0, 0)));
+        return;
+    }
+    const float* tiles = b.s_seg + seq * p.sg_seq + state_tile_off(p, h, slab);
+    auto load_tile = [&](int s, f32x16 (&T)[NT]) {
+        const helix_rsrc rg = make_rsrc_u(tiles + (long long)s * p.sg_seg, 64u * NP * sizeof(float));
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) put(T[nt], r4, buf_unit<float>(rg, lane, tile_unit(NT, pt, nt, r4, 0)));
+    };
+    if (!p.fuse_b) {
+        load_tile(seg * (p.walk_len / p.seg_len), R);
+        return;
+    }
+    // Pass B's recurrence (helix_state_scan_f32, same operation order) up to
+    // this walk's segment:
+    //   carry = s0[ids[seq]];  carry = exp(segld_s) carry + D_s,  s < seg
+    // The last segment's workgroup takes one more step and stores s1. Tile
+    // padding (pp >= pw, n >= d_state) starts from zero, as in Pass B. ids and
+    // the segment log-decays come through the scalar unit, so using them does
+    // not wait for the first chunk's vector loads.
+    const int src = p.has_ids ? sload_i32(b.ids, seq) : seq;
+    const long long hs = (long long)h * p.s_s[0];
+    const unsigned sbytes = (unsigned)(((long long)(p.head_dim - 1) * p.s_s[1] + N) * 4);
+    const int soff = (int)((p0 + pp) * p.s_s[1] + 4 * hi) * 4;
+    auto state_off = [&](int nt, int r4) {   // byte offset of the lane's four state values
+        return store_off_if_lt(soff + 4 * (32 * nt + 8 * r4), pp, pw, 32 * nt + 8 * r4 + 4 * hi, N);
+    };
+    const helix_rsrc r0 = make_rsrc_u(b.s0 + src * p.seq_s + hs, sbytes);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+            put(R[nt], r4, __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r0, state_off(nt, r4), 0, 0)));
+    const float* __restrict__ sd = b.segld + seq * p.sd_seq + h;
+    const bool last = seg == p.n_seg - 1;
+    const int nd = seg + (last ? 1 : 0);
+    constexpr int BLK = 2;   // tiles in flight
+    for (int sb = 0; sb < nd; sb += BLK) {
+        f32x16 T[BLK][NT];
+        float a[BLK];
+#pragma unroll
+        for (int k = 0; k < BLK; ++k) {
+            const int s = min(sb + k, nd - 1);
+            load_tile(s, T[k]);
+            a[k] = expf(sload_f32(sd, (long long)s * p.n_head));
+        }
+#pragma unroll
+        for (int k = 0; k < BLK; ++k) {
+            if (sb + k >= nd) break;
+            if (sb + k < seg) {
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) R[nt] = a[k] * R[nt] + T[k][nt];
+            } else if (item_ok) {
+                // s1[seq] = exp(segld_seg) S_seg(seg) + D_seg
+                const helix_rsrc r1 = make_rsrc_u(b.s1 + seq * p.seq_s + hs, sbytes);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    const f32x16 v = a[k] * R[nt] + T[k][nt];
+#pragma unroll
+                    for (int r4 = 0; r4 < 4; ++r4) {
+                        const u32x4 w = {as_u32(v[4 * r4]), as_u32(v[4 * r4 + 1]), as_u32(v[4 * r4 + 2]),
+                                         as_u32(v[4 * r4 + 3])};
+                        __builtin_amdgcn_raw_buffer_store_b128(w, r1, state_off(nt, r4), 0, 0);
+                    }
+                }
+            }
         }
     }
 }
 
-// The decay record of token lane (store_decay_record64: dt, exp(Lcum), Lcum
-// in fp64) and x at this lane's P column for its K tokens j = 32 s + 8 q + e
-// (s = 0, 1; e = 0..7), prefetched a chunk ahead. YT (no records): the raw dt
-// of token lane instead.
-struct StageWX6 {
-    u32x4 rec;
-    float dtraw;
-    float x[16];
-};
-
-template <bool YT>
-__device__ __forceinline__ void load_stage_x6(StageWX6& st, const HelixScanParams& p, const float* __restrict__ rec_h,
-                                              const float* __restrict__ dt_h, const float* __restrict__ x_h, int c,
-                                              int lane, int q, int pp, int pw) {
-    const int t0   = (p.chunk_base + c) * HELIX_CS;
-    const int tlen = min(HELIX_CS, p.n_tok - t0);
-    const int sx0 = sgpr_fresh((int)p.s_x[0]), sx2 = (int)p.s_x[2];
-    const helix_rsrc rx = make_rsrc(x_h + (long long)t0 * p.s_x[0], ((tlen - 1) * sx0 + (pw - 1) * sx2 + 1) * 4u);
-    if constexpr (YT) {
-        const int sdt = (int)p.s_dt[0];
-        const helix_rsrc rdt = make_rsrc(dt_h + (long long)t0 * p.s_dt[0], ((tlen - 1) * sdt + 1) * 4u);
-        st.dtraw = buf_f32(rdt, min(lane, tlen - 1) * sdt * 4, 0);
-    } else {
-        const helix_rsrc rr = make_rsrc(rec_h + (long long)c * p.n_head * (HELIX_CS * 4), HELIX_CS * 16u);
-        st.rec = __builtin_amdgcn_raw_buffer_load_b128(rr, lane * 16, 0, 0);
-    }
-    // Rows past tlen read 0 (past the resource's range) or, with strides under
-    // which a token row is shorter than the slab, another element of the
-    // chunk: dt is 0 for them either way.
-    const int xv = min(pp, pw - 1) * sx2 + 8 * q * sx0;
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) st.x[8 * s + e] = buf_elem<float>(rx, xv, (32 * s + e) * sx0);
-}
-
+// IO: the caller's storage type of x, B, C and y.
 // YT: the single pass run as the three passes without scratch
-// (HelixScanParams::ytile): the start state comes from y (walk_start_state)
-// and the decay preamble is formed here from dt, as Pass A forms its records
-// (softplus, fp64 wave scan), since there are no records.
+// (HelixScanParams::ytile): the start state comes from y and the decay
+// preamble is formed here from dt, as Pass A forms its records (softplus, fp64
+// wave scan), since there are no records.
 // YACC: the walk of a block of state indices after the first (p.y_acc): y of
 // each chunk is loaded with the next chunk's inputs and added to the chunk's
 // result.
-template <int NP, bool YT = false, bool YACC = false>
-__device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, const HelixScanBuffers& b) {
+template <int NP, typename IO = float, bool YT = false, bool YACC = false>
+__device__ __forceinline__ void scan_wx6_impl(const HelixScanParams& p, const HelixScanBuffers& b) {
     static_assert(NP == 64 || NP == 128, "d_state 64 or 128");
-    // Staging lanes: 16 per pair of rows; a run of eight state indices per
-    // lane at d_state 128 (NH = 2 words per row), half a run at 64 (NH = 1).
-    constexpr int NH = NP / 64;
-    constexpr int HPW = 2;                     // heads per workgroup, four waves each
-    constexpr int NB  = NP / 16;               // 16-row state tiles of R
-    constexpr int KS  = NP / 32;               // K steps over the state
-    constexpr int NT32 = NP / 32;              // 32 x 32 tiles of the slab tile layout
-    constexpr int NCH = NP / 8;                // 16-byte chunks per C / B row
-    constexpr int PL_CB = 3 * HELIX_CS * NP;   // C (or B) planes, elements
-    constexpr int PL_M  = 3 * HELIX_CS * HELIX_CS;
-    constexpr int PF = 2;                      // products an operand read runs ahead
-    __shared__ __attribute__((aligned(16))) __bf16 sC[PL_CB];
-    __shared__ __attribute__((aligned(16))) __bf16 sBt[3 * NP * HELIX_CS];   // B^T[n][j] planes
-    __shared__ __attribute__((aligned(16))) __bf16 sM[HPW * PL_M];     // each head's M[t][j] planes
-    __shared__ __attribute__((aligned(16))) float sDt[HPW][HELIX_CS];    // dt_j (0 past tlen)
-    __shared__ __attribute__((aligned(16))) float sSd[HPW][HELIX_CS];    // exp(L_end - Lcum_j)
-    __shared__ __attribute__((aligned(16))) float sE[HPW][HELIX_CS];     // exp(Lcum_t)
-    __shared__ __attribute__((aligned(16))) double sL[HPW][HELIX_CS];    // Lcum_t
+    static_assert(sizeof(IO) == 4 || !(YT || YACC), "state tiles in y and sums into y: fp32 storage");
+    constexpr int HB  = HELIX_HB;              // items per workgroup, two waves each
+    constexpr int NT  = NP / 32;               // 32-row state tiles of R
+    constexpr int KS  = NP / 16;               // K steps over the state (G3)
+    constexpr int NPL = WX6Planes<IO>::value;  // planes of B and C
+    constexpr int RSC = WX6_RSC<NP>, RSJ = WX6_RSJ, RSM = WX6_RSM;
+    constexpr int PL_C = HELIX_CS * RSC, PL_B = NP * RSJ;   // one plane, elements
+    constexpr int L = NP / 32;                 // B tokens per thread
+    constexpr int CE = NP / 16;                // C state indices per row and thread
+    __shared__ __attribute__((aligned(16))) __bf16 sC[NPL * PL_C];
+    __shared__ __attribute__((aligned(16))) __bf16 sBt[NPL * PL_B];
+    __shared__ __attribute__((aligned(16))) float sCB[HELIX_CS * RSM];
+    // Decay records of the chunk's and the next chunk's tokens, by parity: dt
+    // (0 past tlen), exp(L_end - Lcum) dt, exp(Lcum), and Lcum log2(e) as the
+    // sum of two floats (differences of Lcum keep fp32's precision at any
+    // magnitude of Lcum).
+    __shared__ __attribute__((aligned(16))) float sDt[2][HB][HELIX_CS], sW[2][HB][HELIX_CS], sE[2][HB][HELIX_CS];
+    __shared__ __attribute__((aligned(16))) float sLh[2][HB][HELIX_CS], sLl[2][HB][HELIX_CS];
 
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = wave_uniform();
-    const int hw = wave >> 2, w4 = wave & 3;   // head slot, P block within it
-    const int N = p.d_state, P = p.head_dim;
-    const int hpg = p.heads_per_group;
-    const int npair = (hpg + HPW - 1) / HPW;
+    const int lane = threadIdx.x & 63, wave = wave_uniform(), lo = lane & 31, hi = lane >> 5;
+    const int N = p.d_state;
 
-    // 1-D grid in the logical order (head block, group, slab, walk segment,
-    // sequence). An XCD's share of the logical ids then covers whole walk
-    // segments over every group: a group's head blocks share the XCD (and the
-    // chunk's B and C in its L2), and the XCD's x reads and y writes are whole
-    // token rows of one stretch of a sequence. With the walk segment as the
-    // fastest index after the group (an XCD per group, 2 KiB of every 16 KiB
-    // token row at config 2) the fp32 path took 212-215 us; 207-210 us in this
-    // order. The walk segment sits below the sequence, as in the bf16 walk,
-    // so that an XCD's share stays within one sequence of a batch.
-    const unsigned total = (unsigned)p.n_walk * (unsigned)p.n_group * (unsigned)npair *
-                           (unsigned)p.n_pslab * (unsigned)p.n_seq;
+    // 1-D grid in the logical order (item block, group, walk segment,
+    // sequence), as Pass A's: an XCD's share is whole token rows of one stretch
+    // of a sequence, and a group's item blocks share the XCD's L2.
+    const int ipg = p.heads_per_group * p.n_pslab;
+    const int nib = (ipg + HB - 1) / HB;
+    const unsigned total = (unsigned)p.n_walk * (unsigned)p.n_group * (unsigned)nib * (unsigned)p.n_seq;
     unsigned wid = xcd_logical_id(blockIdx.x, total);
-    const int pair = (int)(wid % (unsigned)npair);    wid /= (unsigned)npair;
-    const int g    = (int)(wid % (unsigned)p.n_group); wid /= (unsigned)p.n_group;
-    const int slab = (int)(wid % (unsigned)p.n_pslab); wid /= (unsigned)p.n_pslab;
-    const int seg  = (int)(wid % (unsigned)p.n_walk); wid /= (unsigned)p.n_walk;
-    const int seq  = (int)wid;
-    // A workgroup of the last pair may have one head: its spare waves walk
-    // that head again and store nothing.
-    const int hslot = HPW * pair + hw;
-    const bool head_ok = hslot < hpg;
-    const int h  = g * hpg + min(hslot, hpg - 1);
+    const int ib  = (int)(wid % (unsigned)nib);       wid /= (unsigned)nib;
+    const int g   = (int)(wid % (unsigned)p.n_group); wid /= (unsigned)p.n_group;
+    const int seg = (int)(wid % (unsigned)p.n_walk);  wid /= (unsigned)p.n_walk;
+    const int seq = (int)wid;
+    // This wave's item and 32-column block of its slab. Each SIMD (waves s and
+    // s + 4) holds one item; in a block of at most two items their four waves
+    // take a SIMD each instead. The other waves only stage B and C and take
+    // their share of G1.
+    const int n_live = min(HB, ipg - ib * HB);
+    const int is = n_live > 2 ? wave % HB : (wave % HB) >> 1;
+    const int pt = n_live > 2 ? wave / HB : wave & 1;
+    const bool item_ok = is < n_live && (n_live > 2 || wave < HB);
+    const int ii = ib * HB + min(is, n_live - 1);
+    const int h = g * p.heads_per_group + ii / p.n_pslab;
+    const int slab = ii % p.n_pslab;
     const int p0 = slab * HELIX_HD;
-    const int pw = min(HELIX_HD, P - p0);
+    const int pw = min(HELIX_HD, p.head_dim - p0);
+    const int pp = 32 * pt + lo;               // this lane's column in the slab
 
     const int c_begin = seg * p.walk_len;
     const int c_end   = min(c_begin + p.walk_len, p.n_cg);
@@ -202,374 +388,380 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
     const float* __restrict__ rec_h = YT ? nullptr : b.pre + ((long long)seq * p.cpg * p.n_head + h) * (HELIX_CS * 4);
     const float* __restrict__ dt_h = b.dt + seq * p.seq_dt + h * p.s_dt[1];
     const float A_h = YT ? b.A[(long long)h * p.s_a] : 0.0f;
-    const float* __restrict__ x_h = b.x + seq * p.seq_x + h * p.s_x[1] + p0 * p.s_x[2];
-    const float* __restrict__ B_g = b.B + seq * p.seq_b + g * p.s_b[1];
-    const float* __restrict__ C_g = b.C + seq * p.seq_c + g * p.s_c[1];
+    const IO* __restrict__ x_h = reinterpret_cast<const IO*>(b.x) + seq * p.seq_x + h * p.s_x[1] + p0 * p.s_x[2];
+    const IO* __restrict__ B_g = reinterpret_cast<const IO*>(b.B) + seq * p.seq_b + g * p.s_b[1];
+    const IO* __restrict__ C_g = reinterpret_cast<const IO*>(b.C) + seq * p.seq_c + g * p.s_c[1];
 
-    // Staging: lane (c16, rr) holds its run's state indices (RunsWX6) of rows
-    // j0 and j0 + 1 (the wave's eight rows, 16 lanes per pair). A chunk's planes are staged
-    // while the previous chunk's products run: C once G1 and G3 are done with
-    // it, B once G4 is. C is zeroed past tlen and d_state, which is all G1 and
-    // G3 need; B rows past tlen only meet dt = 0 columns in G4.
-    // Word w of a run holds state indices 8u + 4 hh .. + 3, at K position
-    // cpos + 8 hh (perm32 keeps each group of four together).
-    auto half_of = [&](int w, int hf) { return NH == 2 ? w : hf; };
-    auto stage_c = [&](const RunsWX6<NH>& rn, int tl, int j0, int u, int hf, int cpos) {
+    auto tlen_of = [&](int c) { return min(HELIX_CS, p.n_tok - (p.chunk_base + c) * HELIX_CS); };
+
+    // Rows past tlen and state indices past d_state take an offset past the
+    // resource's range and read 0.
+    WX6Run<IO, 4> rb[L];
+    WX6Run<IO, CE> rc[2];
+    auto load_b = [&](int c, int ln) {
+        constexpr int ES = (int)sizeof(IO);
+        int bn, bt;
+        wx6_b_rows<NP>(ln, wave, bn, bt);
+        const int tl = tlen_of(c);
+        const int sb0 = sgpr_fresh((int)p.s_b[0]);
+        const helix_rsrc rs = make_rsrc(B_g + (long long)(p.chunk_base + c) * HELIX_CS * p.s_b[0],
+                                        ((tl - 1) * sb0 + N) * (unsigned)ES);
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int j = j0 + k;
-            const unsigned keep = ~(unsigned)(((tl - 1 - j) | (N - 1 - 8 * u)) >> 31);
+        for (int i = 0; i < L; ++i) rb[i].load(rs, store_off_if_lt(((bt + i) * sb0 + bn) * ES, bt + i, tl, bn, N));
+    };
+    auto load_c = [&](int c, int ln) {
+        constexpr int ES = (int)sizeof(IO);
+        int cj, cn0, cpos;
+        wx6_c_run<NP>(ln, wave, cj, cn0, cpos);
+        const int tl = tlen_of(c);
+        const int sc0 = sgpr_fresh((int)p.s_c[0]);
+        const helix_rsrc rs = make_rsrc(C_g + (long long)(p.chunk_base + c) * HELIX_CS * p.s_c[0],
+                                        ((tl - 1) * sc0 + N) * (unsigned)ES);
 #pragma unroll
-            for (int w = 0; w < NH; ++w) {
-                u32x2 cq[3];
+        for (int k = 0; k < 2; ++k) rc[k].load(rs, store_off_if_lt(((cj + k) * sc0 + cn0) * ES, cj + k, tl, cn0, N));
+    };
+    // K step s (tokens 16 s + 8 hi + e) of chunk c's x, in storage form. Rows
+    // past tlen read 0 (past the resource's range) or, with strides under which
+    // a token row is shorter than the slab, another element of the chunk: dt is
+    // 0 for them either way.
+    typename IoWord<IO>::type xs[4][8];
+    auto load_x = [&](int c, int s) {
+        const int tl = tlen_of(c);
+        const int sx0 = sgpr_fresh((int)p.s_x[0]), sx2 = (int)p.s_x[2];
+        const helix_rsrc rx = make_rsrc(x_h + (long long)(p.chunk_base + c) * HELIX_CS * p.s_x[0],
+                                        ((tl - 1) * sx0 + (pw - 1) * sx2 + 1) * (unsigned)sizeof(IO));
+        const int xv = min(pp, pw - 1) * sx2 + 8 * hi * sx0;
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    unsigned c0, c1, c2;
-                    split3_pair(as_f32(rn.c[k][w][2 * e] & keep), as_f32(rn.c[k][w][2 * e + 1] & keep), c0, c1, c2);
-                    cq[0][e] = c0;
-                    cq[1][e] = c1;
-                    cq[2][e] = c2;
-                }
-                const int pos = cpos + 8 * half_of(w, hf);
-#pragma unroll
-                for (int pl = 0; pl < 3; ++pl)
-                    *reinterpret_cast<u32x2*>(&sC[x6_off<HELIX_CS, NCH>(pl, j, pos >> 3) + (pos & 7)]) = cq[pl];
-            }
+        for (int e = 0; e < 8; ++e) xs[s][e] = io_load_word<IO>(rx, xv, (16 * s + e) * sx0);
+    };
+    // The decay record of token lane (store_decay_record64: dt, exp(Lcum), Lcum
+    // in fp64), or with YT the token's dt.
+    u32x4 rec;
+    float dtraw;
+    auto load_rec = [&](int c) {
+        if constexpr (YT) {
+            const int tl = tlen_of(c), sdt = (int)p.s_dt[0];
+            const helix_rsrc rs = make_rsrc(dt_h + (long long)(p.chunk_base + c) * HELIX_CS * p.s_dt[0],
+                                            ((tl - 1) * sdt + 1) * 4u);
+            dtraw = buf_f32(rs, min(lane, tl - 1) * sdt * 4, 0);
+        } else {
+            const helix_rsrc rs = make_rsrc(rec_h + (long long)c * p.n_head * (HELIX_CS * 4), HELIX_CS * 16u);
+            rec = __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, 0, 0);
         }
     };
-    // B's split planes, bw[row k][plane][pair e] (state indices 8u + 4 hh +
-    // 2 (e % 2), +1 for word w = e / 2).
-    auto split_b = [&](const RunsWX6<NH>& rn, unsigned (&bw)[2][3][2 * NH]) {
+    // A chunk's records into buffer par, by one wave of each item.
+    auto stage_rec = [&](int tl, int par) {
+        if (pt != 1 || !item_ok) return;
+        float dtv, e;
+        double lcum;
+        if constexpr (YT) {
+            // As Pass A's hb_preamble forms the records.
+            dtv = keep_if_lt(helix_dt(p, dtraw), lane, tl);
+            lcum = wave_incl_sum((double)A_h * (double)dtv);
+            e = expf((float)lcum);
+        } else {
+            dtv = as_f32(rec[0]);
+            e = as_f32(rec[1]);
+            lcum = __builtin_bit_cast(double, (unsigned long long)rec[2] | ((unsigned long long)rec[3] << 32));
+        }
+        const double l2 = lcum * 1.4426950408889634074;
+        const float l2h = (float)l2;
+        sDt[par][is][lane] = dtv;
+        sW[par][is][lane] = exp2_diff(bcast(lcum, 63), lcum) * dtv;
+        sE[par][is][lane] = e;
+        sLh[par][is][lane] = l2h;
+        sLl[par][is][lane] = (float)(l2 - (double)l2h);
+    };
+    auto stage_c = [&](int ln) {
+        int cj, cn0, cpos;
+        wx6_c_run<NP>(ln, wave, cj, cn0, cpos);
+        __bf16* const wC = sC + cj * RSC + cpos;
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int e = 0; e < 2 * NH; ++e)
-                split3_pair(as_f32(rn.b[k][e >> 1][2 * (e & 1)]), as_f32(rn.b[k][e >> 1][2 * (e & 1) + 1]),
-                            bw[k][0][e], bw[k][1][e], bw[k][2][e]);
-    };
-    // B^T[n][j0 .. j0 + 1] (natural n order): the halves of rows j0 and
-    // j0 + 1 as one 4-byte store.
-    auto write_bt = [&](const unsigned (&bw)[2][3][2 * NH], int j0, int u, int hf) {
+            for (int m = 0; m < CE / 4; ++m) {   // four state indices at K position cpos + 8 m
+                unsigned w[2][NPL];
 #pragma unroll
-        for (int pl = 0; pl < 3; ++pl)
+                for (int e = 0; e < 2; ++e) {
+                    if constexpr (NPL == 1)
+                        w[e][0] = rc[k].w[2 * m + e];   // bf16 pairs as they are
+                    else
+                        wx6_split<NPL>(rc[k].at(4 * m + 2 * e), rc[k].at(4 * m + 2 * e + 1), w[e]);
+                }
 #pragma unroll
-            for (int e = 0; e < 4 * NH; ++e) {
-                const unsigned wa = bw[0][pl][e >> 1], wb = bw[1][pl][e >> 1];
-                const unsigned v = (e & 1) ? ((wa >> 16) | (wb & 0xffff0000u)) : ((wa & 0xffffu) | (wb << 16));
-                const int n = 8 * u + 4 * half_of(e >> 2, hf) + (e & 3);
-                *reinterpret_cast<unsigned*>(&sBt[x6_off<NP, 8>(pl, n, j0 >> 3) + (j0 & 7)]) = v;
+                for (int pl = 0; pl < NPL; ++pl)
+                    *reinterpret_cast<u32x2*>(wC + pl * PL_C + k * RSC + 8 * m) = u32x2{w[0][pl], w[1][pl]};
             }
     };
-    auto tlen_of = [&](int c) { return min(HELIX_CS, p.n_tok - (p.chunk_base + c) * HELIX_CS); };
-
-    RunsWX6<NH> runs;
-    unsigned bw[2][3][2 * NH];
-    StageWX6 st;
-    {
-        const int c16 = lane & 15, rr = lane >> 4, j0 = 8 * wave + 2 * rr;
-        const int u = NH == 2 ? c16 : (c16 & 7), hf = NH == 2 ? 0 : (c16 >> 3);
-        load_runs_x6<NH>(runs, p, B_g, C_g, c_begin, N, j0, u, hf);
-        load_stage_x6<YT>(st, p, rec_h, dt_h, x_h, c_begin, lane, rr, 16 * w4 + c16, pw);
-        stage_c(runs, tlen_of(c_begin), j0, u, hf, wx6_perm32(8 * u));
-        split_b(runs, bw);
-        load_runs_x6<NH>(runs, p, B_g, C_g, min(c_begin + 1, c_end - 1), N, j0, u, hf);
-    }
-
-    // The segment's start state: S_seg from Pass B, or Pass B's recurrence
-    // over Pass A's aggregates run here (p.fuse_b).
-    f32x4 R[NB];
-    {
-        const int q = lane >> 4, c16 = lane & 15;
-        walk_start_state<NP, YT>(R, p, b, seq, h, slab, seg, p0, pw, 16 * w4 + c16, q, w4, c16, head_ok);
-        if constexpr (YT) {
-            // The start state lies in y's rows that this workgroup's waves
-            // overwrite from the first chunk on: every wave has it in
-            // registers before the first barrier, which comes before any y
-            // store.
+    // B's planes as B^T wants them: tokens bt .. bt + L - 1 of state index bn + k.
+    auto stage_b = [&](int ln) {
+        int bn, bt;
+        wx6_b_rows<NP>(ln, wave, bn, bt);
+        __bf16* const wB = sBt + bn * RSJ + bt;
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-                asm volatile("" ::"v"(R[nb][0]), "v"(R[nb][1]), "v"(R[nb][2]), "v"(R[nb][3]));
+        for (int k = 0; k < 4; ++k) {
+            unsigned w[L / 2][NPL];
+#pragma unroll
+            for (int i = 0; i < L / 2; ++i) {
+                if constexpr (NPL == 1)   // the halves k % 2 of the two tokens' words as one pair
+                    w[i][0] = __builtin_amdgcn_perm(rb[2 * i + 1].w[k >> 1], rb[2 * i].w[k >> 1],
+                                                    (k & 1) ? 0x07060302u : 0x05040100u);
+                else
+                    wx6_split<NPL>(rb[2 * i].at(k), rb[2 * i + 1].at(k), w[i]);
+            }
+#pragma unroll
+            for (int pl = 0; pl < NPL; ++pl) {
+                __bf16* dst = wB + pl * PL_B + k * RSJ;
+                if constexpr (L == 4)
+                    *reinterpret_cast<u32x2*>(dst) = u32x2{w[0][pl], w[1][pl]};
+                else
+                    *reinterpret_cast<unsigned*>(dst) = w[0][pl];
+            }
         }
-    }
+    };
 
-    __bf16* const sMh = sM + hw * PL_M;
+    load_c(c_begin, lane);
+    load_b(c_begin, lane);
+    load_rec(c_begin);
+
+    // The segment's start state, R[nt] register 4 r4 + r = S[32 nt + 8 r4 + 4 hi
+    // + r][pp]: a lane's units of the state tile as they stand (helix_params.h).
+    f32x16 R[NT];
+    wx6_start_state<NP, YT>(R, p, b, seq, h, slab, seg, p0, pw, pt, lane, item_ok);
+    if constexpr (YT) {
+        // The start state lies in y's rows that this workgroup's waves
+        // overwrite from the first chunk on: every wave has it in registers
+        // before the first barrier, which comes before any y store.
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float v = R[nt][r];
+                asm volatile("" ::"v"(v));
+            }
+    }
+    stage_c(lane);
+    stage_rec(tlen_of(c_begin), 0);
+    // x is first used after the chunk's second barrier.
+#pragma unroll
+    for (int s = 0; s < 4; ++s) load_x(c_begin, s);
+    load_c(min(c_begin + 1, c_end - 1), lane);
+    load_rec(min(c_begin + 1, c_end - 1));
 
     // Three barriers per chunk: (1) the chunk's planes and records are staged;
-    // (2) M is written and G1 and G3 are done with C (the next chunk's C
-    // planes are staged behind it); (3) G1 and G4 are done with B^T (the next
-    // chunk's B^T planes are written at the top of the loop). G2 reads M after
-    // (2); the next chunk writes M only after its (1).
+    // (2) CB is written and G1 and G3 are done with C (the next chunk's C
+    // planes and records are staged behind it); (3) G4 is done with B^T, G2
+    // with CB (the next chunk's B^T planes are written at the top of the loop).
+#pragma unroll 1
     for (int c = c_begin; c < c_end; ++c) {
         const int t0   = (p.chunk_base + c) * HELIX_CS;
         const int tlen = tlen_of(c);
-        // On the last chunk the next chunk is this one again: no branch.
-        const int cn = min(c + 1, c_end - 1);
-        // Lane-derived indices, formed anew in every chunk: hoisted out of the
-        // loop, the LDS addresses made from them would not fit the registers.
-        const int ln = vgpr_opaque(lane);
-        const int c16 = ln & 15, q = ln >> 4;  // MFMA operand row, K slot group
-        const int u = NH == 2 ? c16 : (c16 & 7), hf = NH == 2 ? 0 : (c16 >> 3);   // staging run, its half
-        const int rr = q;                      // staging row pair
-        const int j0 = 8 * wave + 2 * rr;
-        const int cpos = wx6_perm32(8 * u);    // K position of 8u; 8u + 4 sits 8 further
-        const int pp = 16 * w4 + c16;          // this lane's P column in the slab
+        const int par  = (c - c_begin) & 1;
+        // The segment's last chunk leaves no state (Pass B has it): no G4, and
+        // nothing staged or loaded for a next one.
+        const bool last = c + 1 == c_end;
+        const int cnn = min(c + 2, c_end - 1);
 
-        write_bt(bw, j0, u, hf);
+        // Lane-derived addresses are formed anew in every chunk: hoisted out of
+        // the loop they would not fit the registers, and a spilled address is
+        // reloaded behind the loads in flight.
+        const int ln = vgpr_fresh(lane);
+        const int lo = ln & 31, hi = ln >> 5, c16 = ln & 15, q = ln >> 4;
 
-        // ---- decay records of the two heads --------------------------------
-        float a_c = 0.0f;
-        if constexpr (YT) {
-            // dt (0 past tlen), Lcum in fp64 and its exponentials, as Pass A's
-            // hb_preamble forms the records, by one wave of each head: wave
-            // w4 == hw, so the two heads' preambles run on different SIMDs.
-            // The others read exp(L_end) (token 63's exp(Lcum)) from sE after
-            // the barrier below.
-            if (w4 == hw) {
-                const float dtv = keep_if_lt(helix_dt(p, st.dtraw), lane, tlen);
-                const double lcum = wave_incl_sum((double)A_h * (double)dtv);
-                const double lend = bcast(lcum, 63);
-                sDt[hw][lane] = dtv;
-                sE[hw][lane] = expf((float)lcum);
-                sSd[hw][lane] = exp2_diff(lend, lcum);
-                sL[hw][lane] = lcum;
-            }
-        } else {
-            if (w4 == 0) {
-                const double lcum = __builtin_bit_cast(double, (unsigned long long)st.rec[2] |
-                                                                   ((unsigned long long)st.rec[3] << 32));
-                const double lend = __builtin_bit_cast(
-                    double, (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)st.rec[2], 63) |
-                                ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)st.rec[3], 63) << 32));
-                sDt[hw][lane] = as_f32(st.rec[0]);
-                sE[hw][lane] = as_f32(st.rec[1]);
-                sSd[hw][lane] = exp2_diff(lend, lcum);
-                sL[hw][lane] = lcum;
-            }
-            // exp(L_end) = exp(Lcum) of token 63.
-            a_c = __builtin_bit_cast(float, __builtin_amdgcn_readlane((int)st.rec[1], 63));
-        }
+        stage_b(ln);
+        if (!last) load_b(c + 1, ln);
         __syncthreads();   // (1)
-        if constexpr (YT) a_c = sE[hw][HELIX_CS - 1];
+        f32x16 yprev[2];
+        if constexpr (YACC) wx6_load_y(yprev, p, b, seq, h, t0, item_ok ? tlen : 0, p0, pw, pp, hi);
 
-        // dt x at (K token j = 32 s + 8 q + e, column pp); G4 scales it by the
-        // decay when it needs it.
-        float xb[2][8];
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int h4 = 0; h4 < 2; ++h4) {
-                const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sDt[hw][32 * s + 8 * q + 4 * h4]);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) xb[s][4 * h4 + k] = d4[k] * st.x[8 * s + 4 * h4 + k];
-            }
-        // The scheduling fences keep each prefetch's loads after the last use
-        // of the registers they fill, and each staging step after the barrier
-        // that frees its LDS: hoisted, they wait on loads still in flight.
-        __builtin_amdgcn_sched_barrier(0);
-        load_stage_x6<YT>(st, p, rec_h, dt_h, x_h, cn, lane, q, pp, pw);
-        f32x4 yprev[4];
-        if constexpr (YACC) load_y16(yprev, p, b, seq, h, t0, head_ok ? tlen : 0, p0, pw, pp, q);
+        const __bf16* const rC16 = sC + c16 * RSC + 8 * q;    // operand row c16 of C
+        const __bf16* const rBt = sBt + (16 * (q >> 1) + 4 * (q & 1) + (c16 >> 2)) * RSJ + 4 * (c16 & 3);
 
         // ---- G1: D[j][t] = (B C^T) of blocks idx = wave, wave + 8 -----------
         // Block idx: D[j = 16 jb + 4 q + r][t = 16 tb + c16].
-        f32x4 d[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int idx = wave + 8 * i;
-            d[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             if (idx < 10) {
                 const int tb = wx6_tb(idx), jb = wx6_jb(idx);
+                const __bf16* const ra = rBt + 16 * jb;
+                const __bf16* const rcb = rC16 + 16 * tb * RSC;
+                f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int s = 0; s < KS; ++s) {
+                for (int s = 0; s < NP / 32; ++s) {
                     // B rows j = 16 jb + c16 by transpose reads of B^T: K slot
-                    // 4 h + r of lane group q is C's column 32 s + 8 q + 4 h + r,
-                    // state index 32 s + 16 h + 4 q + r (perm32); lane 4 r + v
-                    // names that row of B^T and tokens 16 jb + 4 v .. + 3.
-                    bf16x8 av[3], bv[3];
-                    {
-                        const int jc = 16 * jb + 4 * (c16 & 3);
-                        const int nr = 32 * s + 4 * q + (c16 >> 2);
+                    // 4 a + r of lane group q is C's position 32 s + 8 q + 4 a
+                    // + r, state index 32 s + 16 (q / 2) + 8 a + 4 (q % 2) + r
+                    // (perm16); lane 4 r + v names that row of B^T and tokens
+                    // 16 jb + 4 v .. + 3.
+                    bf16x8 av[NPL], bv[NPL];
 #pragma unroll
-                        for (int pl = 0; pl < 3; ++pl) {
-                            const u32x2 lo = lds_read_tr16(&sBt[x6_off<NP, 8>(pl, nr, jc >> 3) + (jc & 7)]);
-                            const u32x2 hi = lds_read_tr16(&sBt[x6_off<NP, 8>(pl, nr + 16, jc >> 3) + (jc & 7)]);
-                            av[pl] = __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
-                        }
+                    for (int pl = 0; pl < NPL; ++pl) {
+                        const u32x2 a0 = lds_read_tr16(ra + pl * PL_B + 32 * s * RSJ);
+                        const u32x2 a1 = lds_read_tr16(ra + pl * PL_B + (32 * s + 8) * RSJ);
+                        av[pl] = __builtin_bit_cast(bf16x8, u32x4{a0[0], a0[1], a1[0], a1[1]});
+                        bv[pl] = *reinterpret_cast<const bf16x8*>(rcb + pl * PL_C + 32 * s);
                     }
-                    x6_read<HELIX_CS, NCH>(sC, 16 * tb + c16, 4 * s + q, bv);
-                    d[i] = wx6_mfma(av, bv, d[i]);
+                    d = wx6_mfma16(av, bv, d);
                 }
-            }
-        }
-
-        // ---- M[t][j] = (C B^T)[t][j] exp(Lcum_t - Lcum_j), j <= t, per head --
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int idx = wave + 8 * i;
-            if (idx < 10) {
-                const int tb = wx6_tb(idx), jb = wx6_jb(idx);
-                const int t = 16 * tb + c16;
-                const int jq = 16 * jb + 4 * q;
-#pragma unroll
-                for (int hh = 0; hh < HPW; ++hh) {
-                    const double lt = sL[hh][t];
-                    float m[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        m[r] = keep_if_le(d[i][r] * exp2_diff(lt, sL[hh][jq + r]), jq + r, t);
-                    u32x2 mq[3];
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        unsigned w0, w1, w2;
-                        split3_pair(m[2 * e], m[2 * e + 1], w0, w1, w2);
-                        mq[0][e] = w0;
-                        mq[1][e] = w1;
-                        mq[2][e] = w2;
-                    }
-#pragma unroll
-                    for (int pl = 0; pl < 3; ++pl)
-                        *reinterpret_cast<u32x2*>(&sM[hh * PL_M + x6_off<HELIX_CS, 8>(pl, t, jq >> 3) + (jq & 7)]) =
-                            mq[pl];
-                }
+                *reinterpret_cast<f32x4*>(&sCB[(16 * tb + c16) * RSM + 16 * jb + 4 * q]) = d;
             }
         }
 
         // ---- G3: y = exp(Lcum_t) . (C R), R the state before this chunk -----
-        // Products (s, tb) in order; the C planes of a product are read PF
-        // products ahead, and R's split for the next K step during this one.
-        f32x4 acc[4];
-#pragma unroll
-        for (int tb = 0; tb < 4; ++tb) acc[tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        {
+        const __bf16* const rC = sC + lo * RSC + 8 * hi;      // operand row lo of C
+        f32x16 acc[2];
+        acc[0] = zero16();
+        acc[1] = zero16();
+        if (item_ok) {
             auto split_r = [&](int s, bf16x8 (&rp)[3]) {
                 float rv[8];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    rv[e] = R[2 * s][e];
-                    rv[4 + e] = R[2 * s + 1][e];
-                }
-                x6_split8(rv, rp);
+                for (int e = 0; e < 8; ++e) rv[e] = R[s >> 1][8 * (s & 1) + e];
+                wx6_split8<3>(rv, rp);
             };
-            constexpr int NI = 4 * KS;
-            bf16x8 cv[PF + 1][3], rp[2][3];
+            auto read_c = [&](int s, bf16x8 (&cv)[2][NPL]) {
 #pragma unroll
-            for (int k = 0; k < PF; ++k) x6_read<HELIX_CS, NCH>(sC, 16 * (k % 4) + c16, 4 * (k / 4) + q, cv[k]);
+                for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                    for (int pl = 0; pl < NPL; ++pl)
+                        cv[tb][pl] = *reinterpret_cast<const bf16x8*>(rC + pl * PL_C + 32 * tb * RSC + 16 * s);
+            };
+            bf16x8 cv[2][2][NPL], rp[2][3];
+            read_c(0, cv[0]);
             split_r(0, rp[0]);
 #pragma unroll
-            for (int it = 0; it < NI; ++it) {
-                const int s = it / 4, tb = it % 4;
-                const int nx = it + PF;
-                if (nx < NI) x6_read<HELIX_CS, NCH>(sC, 16 * (nx % 4) + c16, 4 * (nx / 4) + q, cv[nx % (PF + 1)]);
-                if (tb == 1 && s + 1 < KS) split_r(s + 1, rp[(s + 1) & 1]);
-                __builtin_amdgcn_sched_barrier(0);
-                acc[tb] = wx6_mfma(cv[it % (PF + 1)], rp[s & 1], acc[tb]);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int s = 0; s < KS; ++s) {
+                if (s + 1 < KS) {
+                    read_c(s + 1, cv[(s + 1) & 1]);
+                    split_r(s + 1, rp[(s + 1) & 1]);
+                }
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) acc[tb] = wx6_mfma(cv[s & 1][tb], rp[s & 1], acc[tb]);
             }
-        }
 #pragma unroll
-        for (int tb = 0; tb < 4; ++tb) {
-            const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sE[hw][16 * tb + 4 * q]);
+            for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[tb][r] *= e4[r];
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    const f32x4 e4 = *reinterpret_cast<const f32x4*>(&sE[par][is][32 * tb + 8 * r4 + 4 * hi]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[tb][4 * r4 + r] *= e4[r];
+                }
         }
         __syncthreads();   // (2)
 
-        __builtin_amdgcn_sched_barrier(0);
-        stage_c(runs, tlen_of(cn), j0, u, hf, cpos);
-
-        // ---- G4: R <- exp(L_end) R + B^T . (decay dt x) (after G3 used R) ---
-        // Products (s, nb) in order, B^T's planes read PF products ahead.
+        // ---- G2: y += M . dtX, K step by K step of 16 tokens ----------------
+        const float* const rCB = sCB + lo * RSM + 8 * hi;     // row lo of a tile of CB
+        const __bf16* const rB = sBt + lo * RSJ + 8 * hi;     // operand row lo of B^T
+        auto g2 = [&] {
+            float lth[2], ltl[2];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) R[nb] *= a_c;
-        {
-            auto split_x = [&](int s, bf16x8 (&xp)[3]) {
-                float xs[8];
-#pragma unroll
-                for (int h4 = 0; h4 < 2; ++h4) {
-                    const f32x4 s4 = *reinterpret_cast<const f32x4*>(&sSd[hw][32 * s + 8 * q + 4 * h4]);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) xs[4 * h4 + k] = s4[k] * xb[s][4 * h4 + k];
-                }
-                x6_split8(xs, xp);
-            };
-            auto read_bt = [&](int s, int nb, bf16x8 (&bt)[3]) {
-                x6_read<NP, 8>(sBt, 16 * nb + c16, 4 * s + q, bt);
-            };
-            constexpr int NI = 2 * NB;
-            bf16x8 bt[PF + 1][3], xp[2][3];
-#pragma unroll
-            for (int k = 0; k < PF; ++k) read_bt(k / NB, k % NB, bt[k]);
-            split_x(0, xp[0]);
-#pragma unroll
-            for (int it = 0; it < NI; ++it) {
-                const int s = it / NB, nb = it % NB;
-                const int nx = it + PF;
-                if (nx < NI) read_bt(nx / NB, nx % NB, bt[nx % (PF + 1)]);
-                if (nb == 1 && s == 0) split_x(1, xp[1]);
-                __builtin_amdgcn_sched_barrier(0);
-                R[nb] = wx6_mfma(bt[it % (PF + 1)], xp[s], R[nb]);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int tb = 0; tb < 2; ++tb) {
+                lth[tb] = sLh[par][is][32 * tb + lo];
+                ltl[tb] = sLl[par][is][32 * tb + lo];
             }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                float v[8];
+#pragma unroll
+                for (int a = 0; a < 2; ++a) {
+                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sDt[par][is][16 * s + 8 * hi + 4 * a]);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[4 * a + k] = d4[k] * io_widen<IO>(xs[s][4 * a + k]);
+                }
+                bf16x8 x2[3];
+                wx6_split8<3>(v, x2);
+                // M[t][j] = CB[t][j] exp(Lcum_t - Lcum_j), j <= t, of t tile tb
+                // at tokens j = 16 s + 8 hi + e.
+                const int lim = vgpr_fresh(lo - 8 * hi);
+#pragma unroll
+                for (int tb = s >> 1; tb < 2; ++tb) {
+                    float m[8];
+#pragma unroll
+                    for (int a = 0; a < 2; ++a) {
+                        const f32x4 cb = *reinterpret_cast<const f32x4*>(rCB + 32 * tb * RSM + 16 * s + 4 * a);
+                        const f32x4 jh = *reinterpret_cast<const f32x4*>(&sLh[par][is][16 * s + 8 * hi + 4 * a]);
+                        const f32x4 jl = *reinterpret_cast<const f32x4*>(&sLl[par][is][16 * s + 8 * hi + 4 * a]);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const int e = 4 * a + k;
+                            const float d = cb[k] * __builtin_amdgcn_exp2f((lth[tb] - jh[k]) + (ltl[tb] - jl[k]));
+                            m[e] = (s >> 1) == tb ? (lim >= 16 * (s & 1) + e ? d : 0.0f) : d;
+                        }
+                    }
+                    bf16x8 mp[3];
+                    wx6_split8<3>(m, mp);
+                    acc[tb] = wx6_mfma(mp, x2, acc[tb]);
+                }
+            }
+        };
+        // ---- G4: R <- exp(L_end) R + B^T . (w x), w = exp(L_end - Lcum) dt ---
+        auto g4 = [&] {
+            const float a_c = sE[par][is][HELIX_CS - 1];   // exp(L_end)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) R[nt] *= a_c;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                float v[8];
+#pragma unroll
+                for (int a = 0; a < 2; ++a) {
+                    const f32x4 w4 = *reinterpret_cast<const f32x4*>(&sW[par][is][16 * s + 8 * hi + 4 * a]);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[4 * a + k] = w4[k] * io_widen<IO>(xs[s][4 * a + k]);
+                }
+                bf16x8 x4[3];
+                wx6_split8<3>(v, x4);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    bf16x8 bp[NPL];
+#pragma unroll
+                    for (int pl = 0; pl < NPL; ++pl)
+                        bp[pl] = *reinterpret_cast<const bf16x8*>(rB + pl * PL_B + 32 * nt * RSJ + 16 * s);
+                    R[nt] = wx6_mfma(bp, x4, R[nt]);
+                }
+            }
+        };
+        if (!last) {
+            __builtin_amdgcn_sched_barrier(0);
+            stage_c(ln);
+            load_c(cnn, ln);
+            stage_rec(tlen_of(c + 1), par ^ 1);
+            load_rec(cnn);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        split_b(runs, bw);
-        __builtin_amdgcn_sched_barrier(0);
-        load_runs_x6<NH>(runs, p, B_g, C_g, min(c + 2, c_end - 1), N, j0, u, hf);
-
-        // ---- G2: y += M . dtX (t block tb needs j < 16 (tb + 1)) -----------
-        // K step s covers j blocks 2s and 2s + 1; for tb = 0 and 2 the second
-        // lies above the diagonal (lanes q >= 2), where M was not written.
+        if (item_ok) g2();
+        if (!last && item_ok) {
+            g4();
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            bf16x8 xp[3];
-            x6_split8(xb[s], xp);
-#pragma unroll
-            for (int tb = 2 * s; tb < 4; ++tb) {
-                bf16x8 mv[3];
-                x6_read<HELIX_CS, 8>(sMh, 16 * tb + c16, 4 * s + q, mv);
-                if (tb == 2 * s) {
-                    const unsigned keep = q < 2 ? ~0u : 0u;
-#pragma unroll
-                    for (int pl = 0; pl < 3; ++pl)
-                        mv[pl] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, mv[pl]) & keep);
-                }
-                acc[tb] = wx6_mfma(mv, xp, acc[tb]);
-            }
+            for (int s = 0; s < 4; ++s) load_x(c + 1, s);
+            __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (YACC) {
-#pragma unroll
-            for (int tb = 0; tb < 4; ++tb) acc[tb] += yprev[tb];
-            store_y16<float, HELIX_NT, false>(acc, p, b, seq, h, t0, head_ok ? tlen : 0, p0, pw, pp, q);
-        } else {
-            store_y16<float>(acc, p, b, seq, h, t0, head_ok ? tlen : 0, p0, pw, pp, q);
+            acc[0] += yprev[0];
+            acc[1] += yprev[1];
         }
+        if (item_ok) wx6_store_y<IO, HELIX_NT>(acc, p, b, seq, h, t0, tlen, p0, pw, pp, hi);
+        if (last) break;
         __syncthreads();   // (3)
     }
 }
 
-#define HELIX_PASS_C_WALK_X6(NP)                                                                \
-    extern "C" __global__ __launch_bounds__(HELIX_WG * 2) void helix_scan_walk_x6_n##NP(         \
+#define HELIX_PASS_C_WALK_X6(NP)                                                                 \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_n##NP(   \
         HelixScanParams p, HelixScanBuffers b) {                                                \
-        scan_walk_x6_impl<NP>(p, b);                                                            \
-    }
-
-// The single pass without scratch (HelixScanParams::ytile).
-#define HELIX_PASS_C_WALK_X6_Y(NP)                                                              \
-    extern "C" __global__ __launch_bounds__(HELIX_WG * 2) void helix_scan_walk_x6_y_n##NP(       \
+        scan_wx6_impl<NP>(p, b);                                                             \
+    }                                                                                           \
+    /* The single pass without scratch (HelixScanParams::ytile). */                             \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_y_n##NP( \
         HelixScanParams p, HelixScanBuffers b) {                                                \
-        scan_walk_x6_impl<NP, true>(p, b);                                                      \
-    }
-
-// The walks of the second and later blocks of state indices.
-#define HELIX_PASS_C_WALK_X6_ACC(NP)                                                            \
-    extern "C" __global__ __launch_bounds__(HELIX_WG * 2) void helix_scan_walk_x6_acc_n##NP(     \
+        scan_wx6_impl<NP, float, true>(p, b);                                                \
+    }                                                                                           \
+    /* The walks of the second and later blocks of state indices. */                            \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_acc_n##NP( \
         HelixScanParams p, HelixScanBuffers b) {                                                \
-        scan_walk_x6_impl<NP, false, true>(p, b);                                               \
+        scan_wx6_impl<NP, float, false, true>(p, b);                                         \
     }
 
 HELIX_PASS_C_WALK_X6(64)
 HELIX_PASS_C_WALK_X6(128)
-HELIX_PASS_C_WALK_X6_ACC(64)
-HELIX_PASS_C_WALK_X6_ACC(128)
-HELIX_PASS_C_WALK_X6_Y(64)
-HELIX_PASS_C_WALK_X6_Y(128)

@@ -126,10 +126,10 @@ struct TraitTable {
                 t.k_state_scan = kernel("helix_state_scan_y_f32");
                 t.k_chunk_out = kernel("helix_scan_walk_x6_y_n" + np);
                 t.mfma_a = "v_mfma_f32_32x32x16_bf16 (bf16x6 split operands)";
-                t.mfma_c = "v_mfma_f32_16x16x32_bf16 (bf16x6 split operands)";
+                t.mfma_c = "v_mfma_f32_32x32x16_bf16 (bf16x6 split operands)";
                 t.np = kNps[k];
                 t.walk = true;
-                t.walk_hpw = 2;
+                t.walk_hb = true;
                 t.a_hb = true;
             }
             if (k < 2) {
@@ -168,7 +168,7 @@ struct TraitTable {
                 t.k_chunk_out_acc = kernel("helix_scan_walk_x6_acc_n" + np);
                 t.mfma_c = "v_mfma_f32_16x16x32_bf16 (bf16x6 split operands)";
                 t.walk = true;
-                t.walk_hpw = 2;
+                t.walk_hb = true;
                 t.walk_fuse_b = true;
                 t.rec_kind = 2;
             }
@@ -436,6 +436,13 @@ constexpr long kMaxSegLen = 16;
 // two chunks of split B planes): ~256 workgroups fill the chip.
 constexpr long kTargetWgHb = 256;
 
+// Workgroups of HELIX_HB (head, P slab) items of a B/C group, per segment.
+long item_blocks(const helix_scan_desc& d) {
+    const long n_pslab = (d.head_dim + HELIX_HD - 1) / HELIX_HD;
+    const long ipg = (long)(d.n_head / d.n_group) * n_pslab;
+    return (long)d.n_seq * d.n_group * ((ipg + HELIX_HB - 1) / HELIX_HB);
+}
+
 int choose_walk_len(const helix_scan_desc& d, int cpg) {
     const long n_pslab = (d.head_dim + HELIX_HD - 1) / HELIX_HD;
     const long items = (long)d.n_seq * d.n_head * n_pslab;
@@ -464,6 +471,10 @@ struct DispatchCost {
 };
 constexpr DispatchCost kCostA{3.0, 0.009, 2.0, 0.0};
 constexpr DispatchCost kCostWalk{2.25, 0.007, 0.5, 0.5};
+// The fp32 path's walk of HELIX_HB items: 13.5 us a chunk step over the whole
+// chip at L=8192 H=64 P=64 N=128 G=8 (256 workgroups), with the bf16 walk's
+// proportions.
+constexpr DispatchCost kCostWalkHb{7.5, 0.0235, 0.5, 0.5};
 constexpr int kXcds = 8, kEnginesPerXcd = 4, kCusPerEngine = 8;
 
 // Microseconds for workgroups given in logical-id order as (chunk steps,
@@ -510,7 +521,14 @@ double fused_lengths_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, i
                     wg.emplace_back(seg_steps(s) + kCostA.o,
                                     (double)std::min(HELIX_HB, ipg - HELIX_HB * ib) / HELIX_HB);
     const double a = dispatch_us(wg, kCostA);
-    // Walk: (head block, group, slab, walk, sequence).
+    // Walk: (item block, group, walk, sequence), or (head block, group, slab, walk, sequence).
+    if (tr.walk_hb) {
+        for (size_t i = 0, n = wg.size(); i < n; ++i) {
+            const int s = (int)(i / ((size_t)nib * d.n_group) % nseg);
+            wg[i].first += kCostWalkHb.o - kCostA.o + kCostWalkHb.g * s;
+        }
+        return a + dispatch_us(wg, kCostWalkHb);
+    }
     const int hpw = tr.walk_hpw ? tr.walk_hpw : HELIX_WALK_HPW(tr.np);
     const int npair = (hpg + hpw - 1) / hpw;
     wg.clear();
@@ -539,7 +557,7 @@ int fused_walk_len(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cp
     using Key = std::tuple<int, int, int, int, int, int, int, int>;
     static std::mutex mu;
     static std::map<Key, int> memo;
-    const Key key{d.n_seq, d.n_head, d.head_dim, d.n_group, tr.np, tr.walk_hpw, cpg, shortest};
+    const Key key{d.n_seq, d.n_head, d.head_dim, d.n_group, tr.np, tr.walk_hb ? -1 : tr.walk_hpw, cpg, shortest};
     {
         std::lock_guard<std::mutex> lk(mu);
         const auto it = memo.find(key);
@@ -573,9 +591,7 @@ void choose_lengths(const helix_tuning& tu, const helix_scan_desc& d, const Heli
         a = std::min(tu.seg_len, cpg);
         w = std::max(a, (w / a) * a);
     } else if (tr.a_hb) {
-        const long n_pslab = (d.head_dim + HELIX_HD - 1) / HELIX_HD;
-        const long ipg = (long)(d.n_head / d.n_group) * n_pslab;
-        const long per_seg = (long)d.n_seq * d.n_group * ((ipg + HELIX_HB - 1) / HELIX_HB);
+        const long per_seg = item_blocks(d);
         a = 1;
         for (int cand = w; cand >= 1; --cand) {
             if (w % cand) continue;
@@ -612,6 +628,25 @@ void layout(const helix_tuning& tu, const helix_scan_desc& d, const HelixMatmulT
     choose_lengths(tu, d, tr, cpg, &pl->seg_len, &pl->walk_len);
     pl->segs_per_group = (cpg + pl->seg_len - 1) / pl->seg_len;
     pl->walks_per_group = (cpg + pl->walk_len - 1) / pl->walk_len;
+    pl->run_len = pl->walk_len;
+    if (tr.walk_hb) {
+        // The walk with HELIX_HB items per workgroup, one workgroup per CU, has
+        // half the workgroups of the two-head walks that walk_len is chosen
+        // for: the run of whole Pass A segments with the fewest chunk steps
+        // over its rounds of workgroups, each costing about 0.6 of a step more
+        // (its start state and first loads). At 24 heads x 2 x 1500 tokens
+        // runs of 1, 2 and 3 chunks are 288, 144 and 96 workgroups.
+        const long wg = item_blocks(d);
+        double best = 0.0;
+        for (int run = pl->seg_len; run <= pl->walk_len; run += pl->seg_len) {
+            const long rounds = (wg * ((cpg + run - 1) / run) + kTargetWgHb - 1) / kTargetWgHb;
+            const double cost = (double)rounds * (run + 0.6);
+            if (run == pl->seg_len || cost <= best) {
+                best = cost;
+                pl->run_len = run;
+            }
+        }
+    }
     pl->sl_elem_bytes = bf16_state ? 2 : 4;
     pl->sl_elems = (pl->seg_len > 1 && !walk) ? state * (size_t)cpg : 0;
     pl->sg_elems = state * (size_t)pl->segs_per_group;

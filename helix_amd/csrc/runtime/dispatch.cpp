@@ -19,7 +19,9 @@
 //   Pass C  grid (chunks * n_group * n_hblk * n_seq)    x 256 threads (1-D,
 //           decoded XCD-aware in the kernel); the walking variant runs one
 //           workgroup of 256 * HELIX_WALK_HPW(np) threads per (walk segment,
-//           block of that many heads of a group, P slab, seq) instead
+//           block of that many heads of a group, P slab, seq) instead (bf16
+//           path), or of 512 threads per (run of chunks, item block of a
+//           group, seq) (fp32 path)
 // The ragged-tail padding and the bf16 staging of B and C that the reference
 // runs as separate passes (dispatch.mm:218-245) happen inside the Pass A/C
 // staging here, so there is nothing to launch before the group loop.
@@ -235,7 +237,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
     const long long HT = (long long)d->n_head * params.n_pslab * 64 * tr.np;
     params.np      = tr.np;
     params.seg_len = plan.seg_len;
-    params.walk_len = plan.walk_len;
+    params.walk_len = plan.run_len;
     params.hblk    = plan.hblk;
     params.n_hblk  = plan.n_hblk;
     params.sl_cg   = HT;
@@ -278,17 +280,18 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
     const unsigned hpg = (unsigned)(d->n_head / d->n_group);
     const unsigned hpw = tr.walk_hpw > 0 ? (unsigned)tr.walk_hpw : HELIX_WALK_HPW(tr.np);
     const unsigned pairs = (hpg + hpw - 1) / hpw;
+    // Head-block Pass A and walk: item blocks of HELIX_HB (head, P slab) pairs per group.
+    const long long ipg = (long long)hpg * params.n_pslab;
+    const long long nib = (ipg + HELIX_HB - 1) / HELIX_HB;
     auto pass_c_groups = [&](int n_cg, int n_walk) -> long long {
+        if (tr.walk_hb) return (long long)d->n_seq * d->n_group * nib * n_walk;
         return tr.walk ? (long long)n_walk * d->n_group * pairs * params.n_pslab * d->n_seq
                        : (long long)n_cg * d->n_group * plan.n_hblk * d->n_seq;
     };
-    // Head-block Pass A: item blocks of HELIX_HB (head, P slab) pairs per group.
-    const long long ipg = (long long)hpg * params.n_pslab;
-    const long long nib = (ipg + HELIX_HB - 1) / HELIX_HB;
     auto pass_a_groups = [&](int n_seg) -> long long { return (long long)d->n_seq * d->n_group * nib * n_seg; };
     {
         const int n_cg = std::min(plan.chunks_per_group, plan.n_chunks);
-        const long long wg_c = pass_c_groups(n_cg, (n_cg + plan.walk_len - 1) / plan.walk_len);
+        const long long wg_c = pass_c_groups(n_cg, (n_cg + plan.run_len - 1) / plan.run_len);
         const long long wg_a = tr.a_hb ? pass_a_groups((n_cg + plan.seg_len - 1) / plan.seg_len) : 0;
         if (wg_c > 0xffffffffLL || wg_a > 0xffffffffLL) {
             set_error(ctx, "launch grid exceeds 2^32 workgroups");
@@ -322,7 +325,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         params.chunk_base  = base;
         params.n_cg        = std::min(plan.chunks_per_group, plan.n_chunks - base);
         params.n_seg       = (params.n_cg + plan.seg_len - 1) / plan.seg_len;
-        params.n_walk      = (params.n_cg + plan.walk_len - 1) / plan.walk_len;
+        params.n_walk      = (params.n_cg + plan.run_len - 1) / plan.run_len;
         params.first_group = base == 0 ? 1 : 0;
 
         hipError_t e = hipSuccess;
@@ -338,7 +341,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
                                       (unsigned)d->n_seq, HELIX_WG, 1, 1, 0, stream, args, nullptr);
         if (e == hipSuccess && do_c) {
             const unsigned n_wg = (unsigned)pass_c_groups(params.n_cg, params.n_walk);
-            const unsigned threads = tr.walk ? HELIX_WG * hpw : HELIX_WG;
+            const unsigned threads = tr.walk_hb ? HELIX_HB_THREADS : tr.walk ? HELIX_WG * hpw : HELIX_WG;
             // With bf16 copies, Pass C reads B and C from them: dense
             // [seq][t][group][n] rows counted from the group's first token.
             // The base is moved back by that token so that the kernel's

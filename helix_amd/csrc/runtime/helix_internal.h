@@ -83,6 +83,9 @@ struct HelixMatmulTraits {
     int           single_threads;  // its workgroup size (64 x waves)
     // Heads per workgroup of a walking Pass C; 0 means HELIX_WALK_HPW(np).
     int           walk_hpw;
+    // The walk runs HELIX_HB (head, P slab) items per workgroup, as the
+    // head-block Pass A does, over MultipassPlan::run_len chunks.
+    bool          walk_hb;
     // Pass A writes bf16 copies of B and C that the walking Pass C reads.
     bool          bccopy;
     // The walking Pass C can run Pass B's segment scan in its prologue
@@ -132,6 +135,8 @@ struct MultipassPlan {
     int    segs_per_group   = 0;
     int    walk_len         = 0;   // chunks per walking Pass C segment (multiple of seg_len)
     int    walks_per_group  = 0;
+    int    run_len          = 0;   // chunks per workgroup of the walking Pass C: walk_len, or with walk_hb the
+                                   // part of it (whole Pass A segments) that still fills the chip
     int    hblk             = 0;
     int    n_hblk           = 0;
     size_t sl_elems         = 0;   // s_local elements (0 when seg_len == 1)
