@@ -293,7 +293,8 @@ HELIX_DEV int hb_off(int k, int r, int c) {
 
 // Split the L consecutive tokens' values v[0..L-1] of state index n into NS
 // planes and store them at tokens t .. t + L - 1 of row n (hb_off layout).
-// H16: two fp16 planes, or one where the scaled values are exact in fp16.
+// H16: two fp16 planes, or one where the scaled values are exact in fp16; one
+// bf16 plane of bf16 values.
 template <int NP, int NS, int L, bool H16 = false>
 HELIX_DEV void hb_stage_run(__bf16* planes, int n, int t, const float* v) {
     static_assert(L == 2 || L == 4, "runs of two or four tokens");
@@ -301,8 +302,8 @@ HELIX_DEV void hb_stage_run(__bf16* planes, int n, int t, const float* v) {
 #pragma unroll
     for (int e = 0; e < L / 2; ++e) {
         unsigned w[3];
-        if constexpr (H16 && NS == 1)
-            w[0] = pk_f16(v[2 * e], v[2 * e + 1]);
+        if constexpr (NS == 1)
+            w[0] = H16 ? pk_f16(v[2 * e], v[2 * e + 1]) : pk_bf16(v[2 * e], v[2 * e + 1]);
         else if constexpr (H16)
             split2h_pair(v[2 * e], v[2 * e + 1], w[0], w[1]);
         else if constexpr (NS == 3)
@@ -373,8 +374,9 @@ __device__ __forceinline__ void chunk_state_hb_impl(const HelixScanParams& p, co
     // B's planes. With fp16 planes and 16-bit storage one: a bf16 or f16 value
     // (8 or 11 significant bits) scaled by a power of two is exact in fp16
     // wherever it stays a normal number, so B's low plane would be zero and
-    // the products are a1 b0 + a0 b0.
-    constexpr int NSB = (H16 && sizeof(IO) == 2) ? 1 : NS;
+    // the products are a1 b0 + a0 b0. On bf16 planes a bf16 value is one plane
+    // and an f16 value two, exactly: three and five products in place of six.
+    constexpr int NSB = sizeof(IO) == 4 ? NS : (H16 || __is_same(IO, __bf16)) ? 1 : 2;
     constexpr int PLANES = NSB * NP * HB_RS;
     __shared__ __attribute__((aligned(16))) __bf16 sB[2 * PLANES];   // two chunks' planes
     // Per chunk parity and item: w_j of the chunk's 64 tokens, and L_end (fp64
@@ -599,20 +601,15 @@ __device__ __forceinline__ void chunk_state_hb_impl(const HelixScanParams& p, co
             for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_f16(bp[i][0], xp[0], acc[i0 + i]);
             return;
         }
-        if constexpr (NS == 3) {
+        // The parts (k, l) of B and x with k + l < NS.
 #pragma unroll
-            for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_bf16(bp[i][2], xp[0], acc[i0 + i]);
+        for (int sum = NS - 1; sum >= 0; --sum)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_bf16(bp[i][1], xp[1], acc[i0 + i]);
+            for (int k = sum; k >= 0; --k)
+                if (k < NSB) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_bf16(bp[i][0], xp[2], acc[i0 + i]);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_bf16(bp[i][1], xp[0], acc[i0 + i]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_bf16(bp[i][0], xp[1], acc[i0 + i]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_bf16(bp[i][0], xp[0], acc[i0 + i]);
+                    for (int i = 0; i < 2; ++i) acc[i0 + i] = mfma_bf16(bp[i][k], xp[sum - k], acc[i0 + i]);
+                }
     };
     // The x operand planes of K step s of the chunk in xs, weighted by w0, w1.
     auto split_x = [&](int s, const f32x4& w0, const f32x4& w1, bf16x8 (&xp)[NS]) {
@@ -896,6 +893,14 @@ __device__ __forceinline__ void chunk_state_hb_impl(const HelixScanParams& p, co
     extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_chunk_state_hb_x6agg_r64_n##NP( \
         HelixScanParams p, HelixScanBuffers b) {                                                      \
         chunk_state_hb_impl<NP, 2, float, false, 3, true>(p, b);                                      \
+    }                                                                                                 \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_chunk_state_hb_x6agg_r64_bf16io_n##NP( \
+        HelixScanParams p, HelixScanBuffers b) {                                                      \
+        chunk_state_hb_impl<NP, 2, __bf16, false, 3, true>(p, b);                                     \
+    }                                                                                                 \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_chunk_state_hb_x6agg_r64_f16io_n##NP( \
+        HelixScanParams p, HelixScanBuffers b) {                                                      \
+        chunk_state_hb_impl<NP, 2, _Float16, false, 3, true>(p, b);                                   \
     }                                                                                                 \
     extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_chunk_state_hb_x6agg_bf16io_n##NP( \
         HelixScanParams p, HelixScanBuffers b) {                                                      \

@@ -331,7 +331,7 @@ __device__ __forceinline__ void wx6_start_state(f32x16 (&R)[NP / 32], const Heli
 // each chunk is loaded with the next chunk's inputs and added to the chunk's
 // result.
 template <int NP, typename IO = float, bool YT = false, bool YACC = false>
-__device__ __forceinline__ void scan_wx6_impl(const HelixScanParams& p, const HelixScanBuffers& b) {
+__device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, const HelixScanBuffers& b) {
     static_assert(NP == 64 || NP == 128, "d_state 64 or 128");
     static_assert(sizeof(IO) == 4 || !(YT || YACC), "state tiles in y and sums into y: fp32 storage");
     constexpr int HB  = HELIX_HB;              // items per workgroup, two waves each
@@ -750,17 +750,25 @@ __device__ __forceinline__ void scan_wx6_impl(const HelixScanParams& p, const He
 #define HELIX_PASS_C_WALK_X6(NP)                                                                 \
     extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_n##NP(   \
         HelixScanParams p, HelixScanBuffers b) {                                                \
-        scan_wx6_impl<NP>(p, b);                                                             \
+        scan_walk_x6_impl<NP>(p, b);                                                             \
+    }                                                                                           \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_bf16io_n##NP( \
+        HelixScanParams p, HelixScanBuffers b) {                                                \
+        scan_walk_x6_impl<NP, __bf16>(p, b);                                                        \
+    }                                                                                           \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_f16io_n##NP( \
+        HelixScanParams p, HelixScanBuffers b) {                                                \
+        scan_walk_x6_impl<NP, _Float16>(p, b);                                                      \
     }                                                                                           \
     /* The single pass without scratch (HelixScanParams::ytile). */                             \
     extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_y_n##NP( \
         HelixScanParams p, HelixScanBuffers b) {                                                \
-        scan_wx6_impl<NP, float, true>(p, b);                                                \
+        scan_walk_x6_impl<NP, float, true>(p, b);                                                \
     }                                                                                           \
     /* The walks of the second and later blocks of state indices. */                            \
     extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk_x6_acc_n##NP( \
         HelixScanParams p, HelixScanBuffers b) {                                                \
-        scan_wx6_impl<NP, float, false, true>(p, b);                                         \
+        scan_walk_x6_impl<NP, float, false, true>(p, b);                                         \
     }
 
 HELIX_PASS_C_WALK_X6(64)

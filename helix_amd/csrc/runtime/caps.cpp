@@ -74,9 +74,10 @@ int io_index(helix_dtype io) { return io == HELIX_BF16 ? 1 : io == HELIX_F16 ? 2
 // long as the process.
 struct TraitTable {
     // [io][k]: single pass; [k]: diagonal A; [k]: fp32 path; [k]: the fp32
-    // path's walk (d_state <= 128); [io][split6][bccopy][k]: bf16 path (bccopy
+    // path's walk (d_state <= 128); [io][k]: the same with 16-bit storage (io
+    // 1, 2); [io][split6][bccopy][k]: bf16 path (bccopy
     // only with fp32 storage).
-    HelixMatmulTraits single[3][3], diag[2], f32[3], f32walk[2], bf16[3][2][2][3], ysingle[2];
+    HelixMatmulTraits single[3][3], diag[2], f32[3], f32walk[2], f32io[3][2], bf16[3][2][2][3], ysingle[2];
     // [io][bccopy][k]: bf16 path with Pass A on scaled fp16 planes (d_state
     // <= 128; bccopy only with fp32 storage).
     HelixMatmulTraits h3[3][2][2];
@@ -171,6 +172,19 @@ struct TraitTable {
                 t.walk_hb = true;
                 t.walk_fuse_b = true;
                 t.rec_kind = 2;
+            }
+            for (int io = 1; io < 3 && k < 2; ++io) {
+                HelixMatmulTraits& t = f32io[io][k];
+                t = f32walk[k];
+                t.name = keep(std::string("mfma fp32, passes A and C bf16x6, ") + (io == 1 ? "bf16" : "f16") + " storage" + upto);
+                t.k_chunk_state = kernel(std::string("helix_chunk_state_hb_x6agg_r64_") + kIoTag[io] + "n" + np);
+                t.k_chunk_out = kernel(std::string("helix_scan_walk_x6_") + kIoTag[io] + "n" + np);
+                t.k_chunk_out_acc = nullptr;
+                t.mfma_a = io == 1 ? "v_mfma_f32_32x32x16_bf16 (one exact plane of B, three of x)"
+                                   : "v_mfma_f32_32x32x16_bf16 (two exact planes of B, three of x)";
+                t.mfma_c = io == 1 ? "v_mfma_f32_32x32x16_bf16 (one exact plane of B and C, three of the rest)"
+                                   : "v_mfma_f32_32x32x16_bf16 (two exact planes of B and C, three of the rest)";
+                t.fallback = &single[io][k];
             }
             for (int io = 0; io < 3; ++io)
                 for (int s6 = 0; s6 < 2; ++s6)
@@ -295,6 +309,21 @@ thread_local const helix_ctx* t_last_ctx = nullptr;
 
 namespace helix::rt {
 
+// Whether a short scan is faster as one launch of the single pass than as the
+// passes. The single pass runs one workgroup per CU, four per (seq, head, P
+// slab), each over the whole sequence: with u = rounds of 256 workgroups x
+// (chunks + 1) it takes 3.7 u + 1 us (fp32 storage, d_state 65..128; 2.8 u + 1.5
+// up to 64), 5.0 u + 1.5 (16-bit storage; 3.5 u + 1.5). The passes take 25-32 us
+// at d_state 65..128 and 17-20 up to 64 before the length shows, the fp32 path's
+// a little more than the bf16 path's. Measured at 64..640 tokens x 1..8
+// sequences of 8..80 heads, 27 heads of 192: at the limits below 18-31 us
+// against 18-42, one step past them 18-38 against 17-44.
+bool one_launch_scan(const helix_scan_desc& d, bool fp32_path) {
+    const long wg = (long)d.n_seq * d.n_head * ((d.head_dim + HELIX_HD - 1) / HELIX_HD) * 4;
+    const long u = (wg + 255) / 256 * ((d.n_tok + HELIX_CS - 1) / HELIX_CS + 1);
+    return u <= (d.io_dtype == HELIX_F32 ? 5 : 4) + (d.d_state > 64 ? 1 : 0) + (fp32_path ? 1 : 0);
+}
+
 helix_tuning tuning_from_env() {
     helix_tuning t;
     t.scratch_mb = env_long("HELIX_SCRATCH_MB", t.scratch_mb);
@@ -389,7 +418,12 @@ const HelixMatmulTraits& select_traits_unblocked(const helix_ctx* ctx, const hel
     // HELIX_FORCE_BACKEND=s... pins the fp32 path (reference caps.mm:82-86).
     const bool bf16 = (d.backend == HELIX_BACKEND_AUTO || d.backend == HELIX_BACKEND_MPP) && !tu.force_fp32;
     if (!bf16) {
-        if (io) return tt.single[io][k];
+        // 16-bit storage: Pass A and the walk up to d_state 128, on B and C as
+        // one (bf16) or two (f16) exact bf16 planes. At L=2048 H=64 P=64 N=128
+        // G=8 in bf16 storage 54 us against 168 for the one-launch single pass
+        // (HELIX_F32_WALK=0, at d_state 256, and for short scans), whose fp32
+        // MFMA walks the whole sequence in each workgroup.
+        if (io) return k < 2 && tu.f32_walk != 0 && !one_launch_scan(d, true) ? tt.f32io[io][k] : tt.single[io][k];
         // A walk of one chunk carries no state between chunks: where the plan
         // gives one-chunk walks (short sequences of few heads), the
         // chunk-parallel Pass C is the faster form (config 0: 23.0 against
@@ -882,7 +916,7 @@ extern "C" bool helix_scan_supported(helix_ctx* ctx, const helix_scan_desc* d) {
 
 extern "C" size_t helix_scan_scratch_size(helix_ctx* ctx, const helix_scan_desc* d) {
     // The single-pass walks (multipass = false, diagonal A, 16-bit storage off
-    // the bf16 path) use none.
+    // the bf16 path at d_state 256) use none.
     if (!d || !d->multipass) return 0;
     const HelixMatmulTraits& tr = helix::rt::select_traits(ctx, *d);
     if (tr.k_single) return 0;

@@ -65,16 +65,17 @@ ByteRange byte_range(const void* base, long long n_seq, long long seq_stride,
 bool y_overlaps_others(const helix_scan_desc& d, const void* y, const void* x, const void* dt, const void* A,
                        const void* B, const void* C, const void* s0, const void* ids, const void* s1) {
     const long long T = d.n_tok, S = d.n_seq;
-    const ByteRange ry = byte_range(y, S, d.seq_y, {{T, d.s_y[0]}, {d.n_head, d.s_y[1]}, {d.head_dim, d.s_y[2]}}, 4);
+    const size_t es = d.io_dtype == HELIX_F32 ? 4 : 2;   // x, B, C and y
+    const ByteRange ry = byte_range(y, S, d.seq_y, {{T, d.s_y[0]}, {d.n_head, d.s_y[1]}, {d.head_dim, d.s_y[2]}}, es);
     auto state = [&](const void* p) {
         return byte_range(p, S, d.seq_s, {{d.n_head, d.s_s[0]}, {d.head_dim, d.s_s[1]}, {d.d_state, d.s_s[2]}}, 4);
     };
     const ByteRange others[] = {
-        byte_range(x, S, d.seq_x, {{T, d.s_x[0]}, {d.n_head, d.s_x[1]}, {d.head_dim, d.s_x[2]}}, 4),
+        byte_range(x, S, d.seq_x, {{T, d.s_x[0]}, {d.n_head, d.s_x[1]}, {d.head_dim, d.s_x[2]}}, es),
         byte_range(dt, S, d.seq_dt, {{T, d.s_dt[0]}, {d.n_head, d.s_dt[1]}}, 4),
         byte_range(A, 1, 0, {{d.n_head, d.s_a}}, 4),
-        byte_range(B, S, d.seq_b, {{T, d.s_b[0]}, {d.n_group, d.s_b[1]}, {d.d_state, d.s_b[2]}}, 4),
-        byte_range(C, S, d.seq_c, {{T, d.s_c[0]}, {d.n_group, d.s_c[1]}, {d.d_state, d.s_c[2]}}, 4),
+        byte_range(B, S, d.seq_b, {{T, d.s_b[0]}, {d.n_group, d.s_b[1]}, {d.d_state, d.s_b[2]}}, es),
+        byte_range(C, S, d.seq_c, {{T, d.s_c[0]}, {d.n_group, d.s_c[1]}, {d.d_state, d.s_c[2]}}, es),
         state(s1),
         ids ? byte_range(ids, S, 1, {}, 4) : state(s0),
     };
@@ -157,6 +158,17 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         if (ytile) trp = ytr;
     }
     const HelixMatmulTraits& tr = *trp;
+    // 16-bit storage on the fp32 path: the one-launch single pass where the
+    // passes have no scratch (none was needed before they served it) or y
+    // overlaps an input.
+    auto run_fallback = [&] {
+        return encode_one(ctx, stream, d, s0, x, dt, A, B, C, ids, y, s1, scratch, scratch_sized, budget_cap, inner,
+                          y_acc, dry, *tr.fallback);
+    };
+    if (tr.fallback && ((!scratch.buf && !scratch_sized) ||
+                        y_overlaps_others(*d, dptr(y), dptr(x), dptr(dt), dptr(A), dptr(B), dptr(C), dptr(s0),
+                                          dptr(ids), dptr(s1))))
+        return run_fallback();
     if (tr.k_single) {
         hipFunction_t f1 = fn(y_acc && tr.k_single_acc ? tr.k_single_acc : tr.k_single);
         if (!f1) {
@@ -217,6 +229,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         void* sp = dptr(scratch);
         if (hipMemGetAddressRange(&base, &size, sp) == hipSuccess) {
             const size_t avail = (size_t)((char*)base + size - (char*)sp);
+            if (avail < plan.total_bytes && tr.fallback) return run_fallback();
             if (avail < plan.total_bytes) {
                 set_error(ctx, "scratch buffer smaller than helix_scan_scratch_size()");
                 return HELIX_ERR_SCRATCH_TOO_SMALL;
@@ -546,6 +559,7 @@ extern "C" helix_status helix_scan_plan_info(helix_ctx* ctx, const helix_scan_de
         out->state_in_y = 1;
         out->kernel_1pass = tr.k_single;
     }
+    if (tr.fallback) out->kernel_1pass = tr.fallback->k_single;   // without scratch
     const HelixMatmulTraits& tp = ytr ? *ytr : tr;
     const helix::rt::MultipassPlan pl = ytr ? yplan : helix::rt::plan_multipass(ctx, pd, tr);
     out->n_chunks = pl.n_chunks;

@@ -81,6 +81,10 @@ struct HelixMatmulTraits {
     // y with y loaded ahead (null: k_single adds through y_acc itself).
     const char*   k_single_acc;
     int           single_threads;  // its workgroup size (64 x waves)
+    // The single-pass kernels the encoder runs instead where the caller lends
+    // no scratch or too little, or y overlaps an input (null: none; 16-bit
+    // storage on the fp32 path).
+    const HelixMatmulTraits* fallback;
     // Heads per workgroup of a walking Pass C; 0 means HELIX_WALK_HPW(np).
     int           walk_hpw;
     // The walk runs HELIX_HB (head, P slab) items per workgroup, as the
@@ -154,6 +158,10 @@ struct MultipassPlan {
 // (helix_scan_encode_noalloc plans for its fixed array).
 MultipassPlan plan_multipass(const helix_ctx* ctx, const helix_scan_desc& d, const HelixMatmulTraits& tr,
                              size_t budget_cap = SIZE_MAX);
+
+// Whether a scan is short enough to run as one launch of the single pass
+// instead of the fp32 path's passes, or the bf16 path's.
+bool one_launch_scan(const helix_scan_desc& d, bool fp32_path);
 
 // Whether the walking Pass C runs Pass B's segment scan itself (no Pass B
 // launch): a single-group plan of at most four segments on a kernel that can;

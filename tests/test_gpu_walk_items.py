@@ -9,10 +9,12 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from oracle import pyoracle as po
-from helix_amd.desc import HELIX_BACKEND_SGMMA
-from gpu_harness import F32_ABS, F32_REL, ctx_for, run
+from helix_amd.desc import HELIX_BACKEND_SGMMA, HELIX_BF16, HELIX_F16, HELIX_OK, HELIX_TENSOR_NULL
+from gpu_harness import F32_ABS, F32_REL, T, ctx_for, run
+from test_gpu_io import TORCH, U, rounded
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +42,49 @@ def test_item_blocks(gpu, shape, knobs):
     _, y, s1 = run(ctx, p, d)
     assert po.allclose_ratio(y, y_ref, F32_REL, F32_ABS) <= 1.0
     assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
+
+
+# 16-bit storage on the fp32 path: Pass A and the walk on one (bf16) or two
+# (f16) exact planes of B and C past the lengths that run as one launch.
+IO_SHAPES = [
+    ((513, 1, 5, 72, 120, 1), 0),       # ten items, an 8-channel last slab, one token last
+    ((449, 2, 6, 64, 64, 2), 0),        # three items per group, d_state 64
+    ((450, 1, 64, 64, 128, 8), 6),      # B and C inside wider rows
+]
+
+
+@pytest.mark.parametrize("io", [HELIX_BF16, HELIX_F16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape,pad", IO_SHAPES, ids=["x".join(map(str, s)) for s, _ in IO_SHAPES])
+def test_16bit_storage(gpu, shape, pad, io):
+    """Against the oracle fed the rounded inputs: y within the fp32 bound plus
+    its own rounding to the storage type, s1 within the fp32 bound. Without
+    scratch, or with y in x's place, the one-launch single pass serves the
+    call, to the same bounds."""
+    p = rounded(po.problem_harness(*shape, 616, "long"), io)
+    p.s0 = (np.random.default_rng(6).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
+    y_ref, s_ref = po.scan(p, use_ids=False)
+    L, S, H, P, N, G = shape
+    d = p.d.copy()
+    d.io_dtype, d.backend, d.multipass = io, HELIX_BACKEND_SGMMA, True
+    for k in (d.s_b, d.s_c):
+        k[0], k[1] = G * (N + pad), N + pad
+    d.seq_b = d.seq_c = L * G * (N + pad)
+    info = gpu.plan_info(d)
+    assert b"helix_scan_walk_x6_" in info.kernel_c and info.total_bytes == gpu.scratch_size(d) > 0
+
+    def up(a, width=0):
+        t = torch.from_numpy(np.ascontiguousarray(a)).cuda()
+        return torch.nn.functional.pad(t, (0, width))
+
+    x, B, C = up(p.x).to(TORCH[io]), up(p.B, pad).to(TORCH[io]), up(p.C, pad).to(TORCH[io])
+    dt, A, s0 = up(p.dt), up(p.A), up(p.s0)
+    scratch = torch.empty(info.total_bytes, dtype=torch.uint8, device="cuda")
+    for route in ("passes", "no scratch", "in place"):
+        y = x.clone() if route == "in place" else torch.full_like(x, float("nan"))
+        s1 = torch.full_like(s0, float("nan"))
+        rc = gpu.encode(torch.cuda.current_stream().cuda_stream, d, T(s0), T(y if route == "in place" else x), T(dt), T(A),
+                        T(B), T(C), HELIX_TENSOR_NULL, T(y), T(s1), T(None if route == "no scratch" else scratch))
+        assert rc == HELIX_OK, gpu.last_error()
+        torch.cuda.synchronize()
+        assert po.allclose_ratio(y.float().cpu().numpy(), y_ref, F32_REL + U[io], F32_ABS) <= 1.0, route
+        assert po.allclose_ratio(s1.cpu().numpy(), s_ref, F32_REL, F32_ABS) <= 1.0, route
