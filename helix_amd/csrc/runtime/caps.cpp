@@ -344,6 +344,10 @@ helix_tuning tuning_from_env() {
     if (yt >= 0) t.ytile = yt > 0 ? 1 : 0;
     const int sb = env_switch("HELIX_STATE_BLOCKS");
     if (sb >= 0) t.state_blocks = sb > 0 ? 1 : 0;
+    for (const char* k : {"HELIX_SCRATCH_MB", "HELIX_PASSA_SPLIT", "HELIX_PASSA_F16", "HELIX_FUSE_B",
+                          "HELIX_WALK_BCCOPY", "HELIX_SEG_LEN", "HELIX_WALK_LEN", "HELIX_HBLK", "HELIX_F32_WALK",
+                          "HELIX_1PASS_Y", "HELIX_STATE_BLOCKS"})
+        if (std::getenv(k)) t.planned = false;
     return t;
 }
 
@@ -439,6 +443,14 @@ const HelixMatmulTraits& select_traits_unblocked(const helix_ctx* ctx, const hel
     // keeps the six.
     if (k < 2 && tu.passa_split != 3 && tu.passa_f16 != 0) return tt.h3[io][bc][k];
     return tt.bf16[io][tu.passa_split == 3 ? 0 : 1][bc][k];
+}
+
+const HelixMatmulTraits* short_scan_traits(const helix_ctx* ctx, const helix_scan_desc& d,
+                                           const HelixMatmulTraits& tr) {
+    if (!tuning_of(ctx).planned || d.a_form != HELIX_A_SCALAR_PER_HEAD || d.d_state > HELIX_N_BLOCK ||
+        !one_launch_scan(d, tr.backend == HELIX_BACKEND_SGMMA))
+        return nullptr;
+    return &table().single[io_index(d.io_dtype)][np_index(d.d_state)];
 }
 
 // The walk's prologue loads up to segs_per_group segment aggregates per

@@ -8,8 +8,8 @@
 // first group of a multi-group plan leaves the earlier groups enqueued.) Stream order sequences the passes; there are no barriers to
 // insert.
 //
-// multipass = false, or a diagonal A: one launch of the single-pass kernel, grid
-// (n_seq * n_head * n_pslab) x 256 threads, no scratch.
+// multipass = false, a diagonal A, or a short scan (one_launch_scan): one launch
+// of the single-pass kernel, grid n_seq * n_head * n_pslab * 4, no scratch.
 //
 // Otherwise, per super-chunk group, in stream order:
 //   Pass A  grid (n_seq * n_group * item blocks * segments) x 512 threads (the
@@ -131,7 +131,35 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         return HELIX_ERR_INVALID_ARG;
     }
 
-    const HelixMatmulTraits* trp = &sel;
+    // A short scan runs as one launch of the single pass, whatever its plan
+    // (HELIX_ONLY_PASS times the plan's passes).
+    // Whether the caller's scratch holds `need` bytes. The reference checks the
+    // MTLBuffer length (dispatch.mm:150-153); the HIP analogue is the allocation
+    // containing the pointer.
+    auto scratch_fits = [&](size_t need) {
+        if (need == 0 || scratch_sized) return true;
+        if (!scratch.buf) return false;
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        void* sp = dptr(scratch);
+        if (hipMemGetAddressRange(&base, &size, sp) != hipSuccess) {
+            (void)hipGetLastError();  // not a hipMalloc allocation: cannot verify, trust the caller
+            return true;
+        }
+        return (size_t)((char*)base + size - (char*)sp) >= need;
+    };
+    auto no_scratch = [&] {
+        set_error(ctx, scratch.buf ? "scratch buffer smaller than helix_scan_scratch_size()"
+                                   : "multipass requires a scratch buffer of helix_scan_scratch_size() bytes");
+        return HELIX_ERR_SCRATCH_TOO_SMALL;
+    };
+    const HelixMatmulTraits* const one =
+        std::getenv("HELIX_ONLY_PASS") ? nullptr : helix::rt::short_scan_traits(ctx, *d, sel);
+    const HelixMatmulTraits* trp = one ? one : &sel;
+    // It needs no scratch, but the caller's contract is the plan's.
+    if (one && !sel.k_single && !sel.fallback &&
+        !scratch_fits(helix::rt::plan_multipass(ctx, *d, sel, budget_cap).total_bytes))
+        return no_scratch();
     auto fn = [&](const char* name) -> hipFunction_t {
         if (!name) return nullptr;
         auto it = ctx->kernels.find(name);
@@ -149,7 +177,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
     // Not for a block that adds into y (y holds the sum so far); the first
     // block of a single pass may keep its tiles in y, which it then
     // overwrites with its share.
-    if (trp->k_single && !y_acc) {
+    if (trp->k_single && !y_acc && !one) {
         const HelixMatmulTraits* ytr = nullptr;
         yplan = helix::rt::plan_ytile(ctx, *d, *trp, &ytr);
         ytile = ytr && (reinterpret_cast<uintptr_t>(dptr(y)) & 15) == 0 &&
@@ -217,26 +245,9 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         set_error(ctx, "empty problem");
         return HELIX_ERR_INVALID_ARG;
     }
-    if (plan.total_bytes > 0 && !scratch_sized) {
-        if (!scratch.buf) {
-            set_error(ctx, "multipass requires a scratch buffer of helix_scan_scratch_size() bytes");
-            return HELIX_ERR_SCRATCH_TOO_SMALL;
-        }
-        // The reference checks the MTLBuffer length (dispatch.mm:150-153);
-        // the HIP analogue is the allocation containing the pointer.
-        hipDeviceptr_t base = nullptr;
-        size_t size = 0;
-        void* sp = dptr(scratch);
-        if (hipMemGetAddressRange(&base, &size, sp) == hipSuccess) {
-            const size_t avail = (size_t)((char*)base + size - (char*)sp);
-            if (avail < plan.total_bytes && tr.fallback) return run_fallback();
-            if (avail < plan.total_bytes) {
-                set_error(ctx, "scratch buffer smaller than helix_scan_scratch_size()");
-                return HELIX_ERR_SCRATCH_TOO_SMALL;
-            }
-        } else {
-            (void)hipGetLastError();  // not a hipMalloc allocation: cannot verify, trust the caller
-        }
+    if (!scratch_fits(plan.total_bytes)) {
+        if (tr.fallback) return run_fallback();
+        return no_scratch();
     }
 
     hipFunction_t fA = fn(tr.k_chunk_state), fB = fn(tr.k_state_scan),

@@ -36,6 +36,8 @@ struct helix_tuning {
     int  f32_walk    = -1;     // HELIX_F32_WALK=0 / 1: the fp32 path's chunk-parallel Pass C / walk
                                // (on per-chunk states stored by Pass A) at d_state 128
     int  ytile       = -1;     // HELIX_1PASS_Y=0: the single pass in its one-launch form only
+    bool planned     = true;   // none of the overrides (this struct, FORCE_BACKEND aside) is set:
+                               // a short scan may run as one launch (one_launch_scan)
     int  state_blocks = -1;    // HELIX_STATE_BLOCKS=0|1: d_state 129..256 (fp32 storage,
                                // scalar A) as blocks of at most 128 state indices, or not
 };
@@ -162,6 +164,12 @@ MultipassPlan plan_multipass(const helix_ctx* ctx, const helix_scan_desc& d, con
 // Whether a scan is short enough to run as one launch of the single pass
 // instead of the fp32 path's passes, or the bf16 path's.
 bool one_launch_scan(const helix_scan_desc& d, bool fp32_path);
+
+// The one-launch single pass where the encoder runs a descriptor (or block of
+// state indices) planned on `tr` as that: a short scan with scalar A, d_state <=
+// 128 and no tuning override. Null otherwise.
+const HelixMatmulTraits* short_scan_traits(const helix_ctx* ctx, const helix_scan_desc& d,
+                                           const HelixMatmulTraits& tr);
 
 // Whether the walking Pass C runs Pass B's segment scan itself (no Pass B
 // launch): a single-group plan of at most four segments on a kernel that can;

@@ -72,6 +72,10 @@ typedef struct {
 #define HELIX_PASS_B_LAUNCHED 0   /* kernel_b, between Pass A and Pass C         */
 #define HELIX_PASS_B_IN_C     1   /* the walking Pass C's prologue               */
 
+/* The plan of the passes. A scan of a few chunks is encoded as one launch of
+ * the single pass instead, whatever its plan, where that is faster (scalar A,
+ * d_state up to 128 or blocks of it, no tuning variable set); its scratch then
+ * stays unused. */
 /* Returns HELIX_ERR_UNSUPPORTED_SHAPE when the descriptor is declined. */
 helix_status helix_scan_plan_info(helix_ctx* ctx, const helix_scan_desc* d,
                                   helix_plan_info* out);

@@ -88,3 +88,33 @@ def test_16bit_storage(gpu, shape, pad, io):
         torch.cuda.synchronize()
         assert po.allclose_ratio(y.float().cpu().numpy(), y_ref, F32_REL + U[io], F32_ABS) <= 1.0, route
         assert po.allclose_ratio(s1.cpu().numpy(), s_ref, F32_REL, F32_ABS) <= 1.0, route
+
+
+# Short scans: at the limit of the one-launch route on each path (caps.cpp,
+# one_launch_scan) and one chunk past it, with the passes that a tuning
+# override keeps (HELIX_STATE_BLOCKS=1, the default's value).
+SHORT = [
+    ((257, 1, 8, 64, 64, 1), True), ((321, 1, 8, 64, 64, 1), False),     # d_state 64: 5 / 6 chunks, fp32 path
+    ((384, 1, 64, 64, 128, 8), True), ((385, 1, 64, 64, 128, 8), False),
+    ((64, 3, 40, 72, 96, 1), False),                                     # four rounds of workgroups of one chunk
+    ((40, 3, 27, 72, 96, 1), True),                                      # three rounds of a ragged chunk
+    ((200, 1, 4, 64, 256, 1), True),                                     # two blocks of state indices
+]
+
+
+@pytest.mark.parametrize("shape,one", SHORT, ids=["x".join(map(str, s)) for s, _ in SHORT])
+def test_short_scan(gpu, shape, one):
+    p = po.problem_harness(*shape, 717, "long")
+    p.s0 = (np.random.default_rng(7).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
+    y_ref, s_ref = po.scan(p, use_ids=False)
+    d = p.d.copy()
+    d.backend, d.multipass = HELIX_BACKEND_SGMMA, True
+    results = {}
+    for name, ctx, multipass in (("default", gpu, True), ("passes", ctx_for(gpu, HELIX_STATE_BLOCKS="1"), True),
+                                 ("one launch", ctx_for(gpu, HELIX_1PASS_Y="0"), False)):
+        d.multipass = multipass
+        _, y, s1 = results[name] = run(ctx, p, d)
+        assert po.allclose_ratio(y, y_ref, F32_REL, F32_ABS) <= 1.0, name
+        assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0, name
+    same = all(np.array_equal(a, b) for a, b in zip(results["default"][1:], results["one launch" if one else "passes"][1:]))
+    assert same
