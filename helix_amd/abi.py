@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from ctypes import POINTER, c_bool, c_char_p, c_int, c_int32, c_size_t, c_uint64, c_void_p
 
 from .desc import (HELIX_OK, STATUS_NAMES, HelixScanDesc, HelixTensor)
@@ -26,7 +27,7 @@ ABI_SYMBOLS = (
     "helix_scan_encode",
     "helix_scan_encode_into",
 )
-HOST_SYMBOLS = ("helix_ctx_create_host", "helix_scan_plan_info", "helix_scan_encode_noalloc")
+HOST_SYMBOLS = ("helix_ctx_create_host", "helix_scan_plan_info", "helix_scan_run", "helix_scan_encode_noalloc")
 # include/helix/helix_host.h HELIX_PASS_B_*: where Pass B's segment scan runs
 PASS_B_LAUNCHED, PASS_B_IN_C = 0, 1
 # include/helix/helix_host.h HELIX_NOALLOC_SCRATCH_BYTES
@@ -60,6 +61,13 @@ class HelixPlanInfo(ctypes.Structure):
         ("state_in_y", c_int32),
         ("state_blocks", c_int32),
     ]
+
+
+# helix_scan_desc and helix_scan_args (include/helix/helix_host.h) for
+# struct.pack: filling ctypes fields one by one cost more than the launches.
+DESC_STRUCT = struct.Struct("=6i24q5i?3x2f")
+ARGS_STRUCT = struct.Struct("=11Q")
+assert DESC_STRUCT.size == ctypes.sizeof(HelixScanDesc)
 
 
 class HelixError(RuntimeError):
@@ -106,6 +114,9 @@ def lib():
     L.helix_scan_encode_into.restype = c_int
     L.helix_scan_encode_noalloc.argtypes = [c_void_p, c_void_p, dp] + [T] * 9
     L.helix_scan_encode_noalloc.restype = c_int
+    # The descriptor and the arguments as packed bytes (DESC_STRUCT, ARGS_STRUCT).
+    L.helix_scan_run.argtypes = [c_void_p, c_void_p, c_char_p, c_char_p, POINTER(c_size_t)]
+    L.helix_scan_run.restype = c_int
     L.helix_scan_plan_info.argtypes = [c_void_p, dp, POINTER(HelixPlanInfo)]
     L.helix_scan_plan_info.restype = c_int
     _lib = L
@@ -169,6 +180,12 @@ class Context:
         if st != HELIX_OK:
             raise HelixError(st, "descriptor declined")
         return info
+
+    def run(self, stream: int, desc: bytes, args: bytes) -> tuple[int, int]:
+        """helix_scan_run on a packed descriptor and arguments: (status, scratch bytes needed)."""
+        need = c_size_t()
+        rc = _lib.helix_scan_run(self.handle, stream, desc, args, ctypes.byref(need))
+        return rc, need.value
 
     def encode_noalloc(self, stream: int, d: HelixScanDesc, s0, x, dt, A, B, C, ids, y, s1) -> int:
         """helix_scan_encode_noalloc: the scan on the library's fixed scratch."""

@@ -146,7 +146,7 @@ typedef struct HelixScanParams {
 /* Device pointers for one encode. s_local is float* on the fp32 path and a
  * bf16 array on the bf16 path. */
 typedef struct HelixScanBuffers {
-    const float* s0;
+    const float* s0;      /* null: a zero state enters */
     const float* x;
     const float* dt;
     const float* A;

@@ -49,7 +49,7 @@ __device__ __forceinline__ void state_scan_impl(const HelixScanParams& p, const 
     const int src = p.has_ids ? b.ids[seq] : seq;
     const long long soff = h * p.s_s[0] + (long long)pr * p.s_s[1] + n;
     f32x4 carry = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (valid) {
+    if (valid && (b.s0 || !p.first_group)) {   // without s0 a zero state enters
         const float* cs = p.first_group ? b.s0 + src * p.seq_s + soff : b.s1 + seq * p.seq_s + soff;
 #pragma unroll
         for (int k = 0; k < 4; ++k) carry[k] = cs[k];

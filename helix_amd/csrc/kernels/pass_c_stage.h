@@ -222,7 +222,7 @@ __device__ __forceinline__ void walk_start_state(f32x4 (&R)[NP / 16], const Heli
             const long long hs = (long long)h * p.s_s[0];
             const unsigned sbytes = (unsigned)(((long long)(P - 1) * p.s_s[1] + N) * 4);
             const int soff = (int)((p0 + pp) * p.s_s[1]) * 4;
-            const helix_rsrc r0 = make_rsrc(b.s0 + src * p.seq_s + hs, sbytes);
+            const helix_rsrc r0 = make_rsrc_u(b.s0 + src * p.seq_s + hs, b.s0 ? sbytes : 0u);   // none: reads 0
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 const int n = 16 * nb + 4 * q;

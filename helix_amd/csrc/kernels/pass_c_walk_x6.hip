@@ -279,7 +279,7 @@ __device__ __forceinline__ void wx6_start_state(f32x16 (&R)[NP / 32], const Heli
     auto state_off = [&](int nt, int r4) {   // byte offset of the lane's four state values
         return store_off_if_lt(soff + 4 * (32 * nt + 8 * r4), pp, pw, 32 * nt + 8 * r4 + 4 * hi, N);
     };
-    const helix_rsrc r0 = make_rsrc_u(b.s0 + src * p.seq_s + hs, sbytes);
+    const helix_rsrc r0 = make_rsrc_u(b.s0 + src * p.seq_s + hs, b.s0 ? sbytes : 0u);   // none: reads 0
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll

@@ -246,7 +246,7 @@ __device__ __forceinline__ void scan_1pass_impl(const HelixScanParams& p, const 
     f32x4 R[NTW];
     {
         const helix_rsrc rs = make_rsrc(b.s0 + src * p.seq_s + h * p.s_s[0] + (long long)p0 * sN,
-                                        swave ? srow_bytes : 0u);
+                                        swave && b.s0 ? srow_bytes : 0u);   // without s0 a zero state
 #pragma unroll
         for (int i = 0; i < NTW; ++i)
 #pragma unroll

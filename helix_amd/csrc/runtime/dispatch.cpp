@@ -77,7 +77,7 @@ bool y_overlaps_others(const helix_scan_desc& d, const void* y, const void* x, c
         byte_range(B, S, d.seq_b, {{T, d.s_b[0]}, {d.n_group, d.s_b[1]}, {d.d_state, d.s_b[2]}}, es),
         byte_range(C, S, d.seq_c, {{T, d.s_c[0]}, {d.n_group, d.s_c[1]}, {d.d_state, d.s_c[2]}}, es),
         state(s1),
-        ids ? byte_range(ids, S, 1, {}, 4) : state(s0),
+        ids ? byte_range(ids, S, 1, {}, 4) : s0 ? state(s0) : ByteRange{},
     };
     for (const ByteRange& r : others)
         if (ry.overlaps(r)) return true;
@@ -95,12 +95,13 @@ bool y_overlaps_others(const helix_scan_desc& d, const void* y, const void* x, c
 // budget_cap: the plan's scratch budget is at most this many bytes (the fixed
 // array of helix_scan_encode_noalloc).
 // dry: run every check, enqueue nothing.
+// A null s0 is a zero state where the entry point allows it (encode_core).
 helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_desc* d,
                         helix_tensor s0, helix_tensor x, helix_tensor dt, helix_tensor A,
                         helix_tensor B, helix_tensor C, helix_tensor ids, helix_tensor y,
                         helix_tensor s1, helix_tensor scratch, bool scratch_sized, size_t budget_cap,
                         bool inner, bool y_acc, bool dry, const HelixMatmulTraits& sel) {
-    if (!s0.buf || !x.buf || !dt.buf || !A.buf || !B.buf || !C.buf || !y.buf || !s1.buf) {
+    if (!x.buf || !dt.buf || !A.buf || !B.buf || !C.buf || !y.buf || !s1.buf) {
         set_error(ctx, "null tensor (s0, x, dt, A, B, C, y and s1 are required)");
         return HELIX_ERR_INVALID_ARG;
     }
@@ -410,7 +411,11 @@ helix_status encode_core(helix_ctx* ctx, hipStream_t stream, const helix_scan_de
                          helix_tensor s0, helix_tensor x, helix_tensor dt, helix_tensor A,
                          helix_tensor B, helix_tensor C, helix_tensor ids, helix_tensor y,
                          helix_tensor s1, helix_tensor scratch, bool scratch_sized = false,
-                         size_t budget_cap = SIZE_MAX) {
+                         size_t budget_cap = SIZE_MAX, bool zero_state = false) {
+    if (!s0.buf && !zero_state) {
+        set_error(ctx, "null tensor (s0, x, dt, A, B, C, y and s1 are required)");
+        return HELIX_ERR_INVALID_ARG;
+    }
     const int nb = helix::rt::n_state_blocks(ctx, *d);
     if (nb == 1)
         return encode_one(ctx, stream, d, s0, x, dt, A, B, C, ids, y, s1, scratch, scratch_sized, budget_cap,
@@ -433,7 +438,7 @@ helix_status encode_core(helix_ctx* ctx, hipStream_t stream, const helix_scan_de
                           /*inner=*/true, /*y_acc=*/false, /*dry=*/false,
                           helix::rt::select_traits_unblocked(ctx, one));
     }
-    if (!s0.buf || !x.buf || !dt.buf || !A.buf || !B.buf || !C.buf || !y.buf || !s1.buf) {
+    if (!x.buf || !dt.buf || !A.buf || !B.buf || !C.buf || !y.buf || !s1.buf) {
         set_error(ctx, "null tensor (s0, x, dt, A, B, C, y and s1 are required)");
         return HELIX_ERR_INVALID_ARG;
     }
@@ -533,6 +538,25 @@ extern "C" helix_status helix_scan_encode_noalloc(helix_ctx* ctx, void* stream, 
     }
     return encode_core(ctx, static_cast<hipStream_t>(stream), d, s0, x, dt, A, B, C, ids, y, s1, scratch,
                        /*scratch_sized=*/true, HELIX_NOALLOC_SCRATCH_BYTES);
+}
+
+extern "C" helix_status helix_scan_run(helix_ctx* ctx, void* stream, const helix_scan_desc* d,
+                                       const helix_scan_args* a, size_t* need) {
+    if (!ctx || !d || !a || !need) return HELIX_ERR_INVALID_ARG;
+    *need = 0;
+    if (!helix_scan_supported(ctx, d)) {
+        set_error(ctx, "descriptor not supported (see helix_ctx_backend_desc)");
+        return HELIX_ERR_UNSUPPORTED_SHAPE;
+    }
+    *need = helix_scan_scratch_size(ctx, d);
+    if (a->scratch_bytes < *need) {
+        set_error(ctx, "scratch buffer smaller than helix_scan_scratch_size()");
+        return HELIX_ERR_SCRATCH_TOO_SMALL;
+    }
+    auto t = [](const void* p) { return helix_tensor{const_cast<void*>(p), 0}; };
+    return encode_core(ctx, static_cast<hipStream_t>(stream), d, t(a->s0), t(a->x), t(a->dt), t(a->A), t(a->B), t(a->C),
+                       t(a->ids), t(a->y), t(a->s1), t(a->scratch), /*scratch_sized=*/a->scratch != nullptr, SIZE_MAX,
+                       /*zero_state=*/true);
 }
 
 extern "C" helix_status helix_scan_plan_info(helix_ctx* ctx, const helix_scan_desc* d,

@@ -10,12 +10,14 @@ from __future__ import annotations
 
 import math
 import threading
+from ctypes import c_float
 
 import torch
 
-from .abi import Context, HelixError
-from .desc import (HELIX_BACKEND_AUTO, HELIX_BACKEND_MPP, HELIX_BACKEND_SGMMA, HELIX_BF16, HELIX_F16,
-                   HELIX_F32, HELIX_OK, HELIX_TENSOR_NULL, HelixScanDesc, HelixTensor)
+from .abi import ARGS_STRUCT, DESC_STRUCT, Context, HelixError
+from .desc import (HELIX_A_SCALAR_PER_HEAD, HELIX_BACKEND_AUTO, HELIX_BACKEND_MPP, HELIX_BACKEND_SGMMA, HELIX_BF16,
+                   HELIX_ERR_SCRATCH_TOO_SMALL, HELIX_ERR_UNSUPPORTED_SHAPE, HELIX_F16, HELIX_F32, HELIX_OK,
+                   HELIX_TENSOR_NULL, HelixScanDesc, HelixTensor)
 
 BACKENDS = {"auto": HELIX_BACKEND_AUTO, "fp32": HELIX_BACKEND_SGMMA, "sgmma": HELIX_BACKEND_SGMMA,
             "bf16": HELIX_BACKEND_MPP, "mpp": HELIX_BACKEND_MPP}
@@ -45,13 +47,12 @@ def tensor_arg(t: torch.Tensor | None) -> HelixTensor:
 
 
 def _scratch_for(device: int, nbytes: int) -> torch.Tensor | None:
-    if nbytes == 0:
-        return None
+    """This thread's scratch on the device, grown to nbytes (0: as it is)."""
     pool = getattr(_scratch, "pool", None)
     if pool is None:
         pool = _scratch.pool = {}
     buf = pool.get(device)
-    if buf is None or buf.numel() < nbytes:
+    if nbytes and (buf is None or buf.numel() < nbytes):
         buf = torch.empty(nbytes, dtype=torch.uint8, device=f"cuda:{device}")
         pool[device] = buf
     return buf
@@ -111,8 +112,6 @@ def ssd_scan(x: torch.Tensor, dt: torch.Tensor, A: torch.Tensor, B: torch.Tensor
             raise ValueError(f"{name} must be {want} on {dev}")
     S, L, H, P = x.shape
     G, N = B.shape[2], B.shape[3]
-    if s0 is None:
-        s0 = torch.zeros((S, H, P, N), dtype=torch.float32, device=dev)
     if y is None:
         y = torch.empty((S, L, H, P), dtype=x.dtype, device=dev)
     elif y.dtype != x.dtype:
@@ -121,22 +120,36 @@ def ssd_scan(x: torch.Tensor, dt: torch.Tensor, A: torch.Tensor, B: torch.Tensor
         s1 = torch.empty((S, H, P, N), dtype=torch.float32, device=dev)
     if ids is not None and (ids.dtype != torch.int32 or not ids.is_contiguous()):
         raise ValueError("ids must be a contiguous int32 tensor")
-    d = make_desc(x, dt, B, C, s0, y, A, backend=backend, multipass=multipass, dt_min=dt_min,
-                  dt_max=dt_max)
-    if tuple(s1.stride()) != tuple(s0.stride()):
+    # No s0: a zero state, of the dense strides, without a tensor of zeros.
+    ss = s0.stride() if s0 is not None else (H * P * N, P * N, N, 1)
+    if s1.stride() != ss:
         raise ValueError("s0 and s1 must share strides")
-    ctx = context(dev.index if dev.index is not None else torch.cuda.current_device())
-    if not ctx.supported(d):
-        raise HelixError(1, f"shape declined: {ctx.backend_desc(d)}")
-    need = ctx.scratch_size(d)
+    sx, sy, sb, sc, sdt = x.stride(), y.stride(), B.stride(), C.stride(), dt.stride()
+    fields = (L, S, H, P, N, G, sx[1], sx[2], sx[3], sb[1], sb[2], sb[3], sc[1], sc[2], sc[3], sdt[1], sdt[2],
+              ss[1], ss[2], ss[3], sy[1], sy[2], sy[3], A.stride(0), sx[0], sb[0], sc[0], sdt[0], ss[0], sy[0],
+              0, HELIX_A_SCALAR_PER_HEAD, IO_DTYPES[x.dtype], HELIX_F32, BACKENDS[backend], bool(multipass))
+    try:
+        d = DESC_STRUCT.pack(*fields, dt_min, dt_max)
+    except OverflowError:   # a bound past float32's range
+        d = DESC_STRUCT.pack(*fields, c_float(dt_min).value, c_float(dt_max).value)
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    ctx = _contexts.get(index) or context(index)
+    st = stream.cuda_stream if stream is not None else torch.cuda.current_stream(dev).cuda_stream
+    lent = scratch
     if scratch is None:
-        scratch = _scratch_for(dev.index, need)
-    elif scratch.numel() * scratch.element_size() < need:
-        raise ValueError(f"scratch needs {need} bytes")
-    st = stream if stream is not None else torch.cuda.current_stream(dev)
-    rc = ctx.encode(st.cuda_stream, d, tensor_arg(s0), tensor_arg(x), tensor_arg(dt),
-                    tensor_arg(A), tensor_arg(B), tensor_arg(C), tensor_arg(ids), tensor_arg(y),
-                    tensor_arg(s1), tensor_arg(scratch))
+        scratch = _scratch_for(index, 0)
+    ptrs = (0 if s0 is None else s0.data_ptr(), x.data_ptr(), dt.data_ptr(), A.data_ptr(), B.data_ptr(), C.data_ptr(),
+            0 if ids is None else ids.data_ptr(), y.data_ptr(), s1.data_ptr())
+    while True:
+        have = 0 if scratch is None else scratch.numel() * scratch.element_size()
+        rc, need = ctx.run(st, d, ARGS_STRUCT.pack(*ptrs, 0 if scratch is None else scratch.data_ptr(), have))
+        if rc != HELIX_ERR_SCRATCH_TOO_SMALL or have >= need:
+            break
+        if lent is not None:
+            raise ValueError(f"scratch needs {need} bytes")
+        scratch = _scratch_for(index, need)
+    if rc == HELIX_ERR_UNSUPPORTED_SHAPE:
+        raise HelixError(1, f"shape declined: {ctx.backend_desc(HelixScanDesc.from_buffer_copy(d))}")
     if rc != HELIX_OK:
         raise HelixError(rc, ctx.last_error())
     return y, s1

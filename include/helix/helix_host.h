@@ -80,6 +80,28 @@ typedef struct {
 helix_status helix_scan_plan_info(helix_ctx* ctx, const helix_scan_desc* d,
                                   helix_plan_info* out);
 
+/* Device pointers of one helix_scan_run call. */
+typedef struct {
+    const void* s0;             /* NULL: every sequence starts from a zero state */
+    const void* x;
+    const void* dt;
+    const void* A;
+    const void* B;
+    const void* C;
+    const void* ids;            /* NULL: identity                                */
+    void*       y;
+    void*       s1;
+    void*       scratch;
+    size_t      scratch_bytes;  /* held by scratch                               */
+} helix_scan_args;
+
+/* helix_scan_supported, helix_scan_scratch_size and helix_scan_encode in one
+ * call, for a host binding whose cost per call counts. *need is the scratch
+ * size; with fewer scratch_bytes it returns HELIX_ERR_SCRATCH_TOO_SMALL and
+ * enqueues nothing. scratch_bytes is taken at its word. */
+helix_status helix_scan_run(helix_ctx* ctx, void* stream, const helix_scan_desc* desc,
+                            const helix_scan_args* args, size_t* need);
+
 /* Size of the fixed scratch helix_scan_encode_noalloc uses on each GPU. */
 #define HELIX_NOALLOC_SCRATCH_BYTES (128u << 20)
 

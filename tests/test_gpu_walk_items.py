@@ -118,3 +118,28 @@ def test_short_scan(gpu, shape, one):
         assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0, name
     same = all(np.array_equal(a, b) for a, b in zip(results["default"][1:], results["one launch" if one else "passes"][1:]))
     assert same
+
+
+NO_STATE = [   # (shape, multipass, backend, knobs): every place that reads s0
+    ((700, 1, 64, 64, 128, 8), True, "fp32", {}),                      # Pass B
+    ((1500, 1, 8, 64, 64, 1), True, "bf16", {"HELIX_SCRATCH_MB": 1}),  # Pass B, many groups
+    ((1024, 4, 40, 64, 128, 1), True, "bf16", {}),                     # the bf16 walk's prologue
+    ((1024, 4, 40, 64, 128, 1), True, "fp32", {}),                     # the fp32 walk's
+    ((600, 1, 16, 64, 128, 2), False, "auto", {}),                     # state tiles in y
+    ((100, 2, 8, 72, 256, 1), True, "auto", {}),                       # one launch per block of state indices
+]
+
+
+@pytest.mark.parametrize("shape,multipass,backend,knobs", NO_STATE, ids=range(len(NO_STATE)))
+def test_ssd_scan_without_state(gpu, shape, multipass, backend, knobs, monkeypatch):
+    """ssd_scan without s0 gives the bits of a state of zeros, with and without ids, twice on one scratch."""
+    from helix_amd import scan
+    p = po.problem_harness(*shape, 818, "long")
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (p.x, p.dt, p.A, p.B, p.C)]
+    monkeypatch.setitem(scan._contexts, torch.cuda.current_device(), ctx_for(gpu, **knobs))
+    zeros = torch.zeros(p.s0.shape, device="cuda")
+    ids = torch.arange(shape[1], dtype=torch.int32, device="cuda").flip(0).contiguous()
+    want = scan.ssd_scan(*t, zeros, backend=backend, multipass=multipass)
+    for i in (None, ids, None):
+        got = scan.ssd_scan(*t, None, i, backend=backend, multipass=multipass)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
