@@ -158,27 +158,6 @@ __device__ __forceinline__ void store_y16(const f32x4 (&acc)[4], const HelixScan
         }
 }
 
-// What y holds at the elements store_y16 would store (fp32 storage), 0 where
-// it would store nothing: for a walk that adds into y (HelixScanParams::y_acc),
-// loaded a chunk's work ahead of the stores so the loads' latency is hidden.
-__device__ __forceinline__ void load_y16(f32x4 (&yv)[4], const HelixScanParams& p, const HelixScanBuffers& b,
-                                         int seq, int h, int t0, int tlen, int p0, int pw, int pp, int q) {
-    const int sy0 = sgpr_fresh((int)p.s_y[0]), sy2 = (int)p.s_y[2];
-    const unsigned bytes = tlen > 0 ? ((tlen - 1) * sy0 + (pw - 1) * sy2 + 1) * 4u : 0u;
-    const helix_rsrc ry = make_rsrc(b.y + seq * p.seq_y + h * p.s_y[1] + (long long)t0 * p.s_y[0] +
-                                        (long long)p0 * p.s_y[2],
-                                    bytes);
-    const int voff = (4 * q * sy0 + pp * sy2) * 4;
-#pragma unroll
-    for (int tb = 0; tb < 4; ++tb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int t = 16 * tb + 4 * q + r;
-            yv[tb][r] = buf_f32(ry, store_off_if_lt(voff, t, tlen, pp, pw), (16 * tb + r) * sy0 * 4);
-        }
-}
-
-
 // The start state R of a walk segment, in the walks' register layout: R[nb][r]
 // = S[16 nb + 4 q + r][p0 + pp] (q = lane / 16, pp = 16 w4 + c16). Without
 // p.fuse_b it is Pass B's S_seg tile of the Pass A segment the walk segment

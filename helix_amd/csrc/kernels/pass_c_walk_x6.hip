@@ -1,5 +1,7 @@
-// pass_c_walk_x6.hip -- the fp32 path's Pass C: the chunk walk on bf16x6 products,
-// four (head, P slab) items of one B/C group per workgroup.
+// pass_c_walk_x6.hip -- Pass C as a chunk walk over four (head, P slab) items of one
+// B/C group per workgroup, up to d_state 128: the fp32 path's on bf16x6 products
+// (helix_scan_walk_x6_*), and the bf16 path's on single bf16 products
+// (helix_scan_walk16_bf16_*; B16 below).
 //
 // Reference counterpart: helix_chunk_out_f32 (src/kernels/
 // helix_scan_multipass.metal:225-361). One workgroup walks a run of chunks
@@ -31,6 +33,12 @@
 // The fp32 path's scan at L=8192 H=64 P=64 N=128 G=8 went from 237 to 199 us, at
 // L=2048 from 75 to 69, at 4 x 1000 tokens of 32 heads of 128 from 128 to 109,
 // against waves of 16 columns, two heads per workgroup, M planes in LDS.
+//
+// The bf16 path's walk (B16) is bound by memory instead: 356 MB at L=8192 H=64
+// P=64 N=128 G=8 in 68 us with the inputs out of the Infinity Cache, 5.2 TB/s
+// where a copy of this card reaches 4.7-5.8 (82 us with 16-column waves and two
+// heads a workgroup, which staged x and its weighted copy through LDS). x loaded
+// a whole chunk ahead, in registers of its own, cost 4 us there.
 //
 // K order: index 16 s + 8 a + 4 b + r of a group of 16 state indices (a, b in
 // {0, 1}) sits at K position 8 b + 4 a + r in the C rows (perm16), so R's result
@@ -330,14 +338,21 @@ __device__ __forceinline__ void wx6_start_state(f32x16 (&R)[NP / 32], const Heli
 // YACC: the walk of a block of state indices after the first (p.y_acc): y of
 // each chunk is loaded with the next chunk's inputs and added to the chunk's
 // result.
-template <int NP, typename IO = float, bool YT = false, bool YACC = false>
+// B16: the bf16 path's walk: every operand rounded once to bf16, one product in
+// place of six, on its Pass A's records (store_decay_record). BIO: the type B
+// and C are read in; __bf16 with fp32 storage when they come from Pass A's bf16
+// copies (the host points B and C there).
+template <int NP, typename IO = float, bool YT = false, bool YACC = false, bool B16 = false, typename BIO = IO>
 __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, const HelixScanBuffers& b) {
     static_assert(NP == 64 || NP == 128, "d_state 64 or 128");
     static_assert(sizeof(IO) == 4 || !(YT || YACC), "state tiles in y and sums into y: fp32 storage");
     constexpr int HB  = HELIX_HB;              // items per workgroup, two waves each
     constexpr int NT  = NP / 32;               // 32-row state tiles of R
     constexpr int KS  = NP / 16;               // K steps over the state (G3)
-    constexpr int NPL = WX6Planes<IO>::value;  // planes of B and C
+    constexpr int NPL = B16 ? 1 : WX6Planes<IO>::value;  // planes of B and C
+    constexpr int NPX = B16 ? 1 : 3;           // planes of x, R and M
+    static_assert(!B16 || !YT, "the form without scratch is fp32-accurate");
+    static_assert(B16 || __is_same(BIO, IO), "bf16 copies of B and C: the bf16 path");
     constexpr int RSC = WX6_RSC<NP>, RSJ = WX6_RSJ, RSM = WX6_RSM;
     constexpr int PL_C = HELIX_CS * RSC, PL_B = NP * RSJ;   // one plane, elements
     constexpr int L = NP / 32;                 // B tokens per thread
@@ -350,7 +365,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
     // sum of two floats (differences of Lcum keep fp32's precision at any
     // magnitude of Lcum).
     __shared__ __attribute__((aligned(16))) float sDt[2][HB][HELIX_CS], sW[2][HB][HELIX_CS], sE[2][HB][HELIX_CS];
-    __shared__ __attribute__((aligned(16))) float sLh[2][HB][HELIX_CS], sLl[2][HB][HELIX_CS];
+    __shared__ __attribute__((aligned(16))) float sLh[2][HB][HELIX_CS], sLl[B16 ? 1 : 2][HB][HELIX_CS];
 
     const int lane = threadIdx.x & 63, wave = wave_uniform(), lo = lane & 31, hi = lane >> 5;
     const int N = p.d_state;
@@ -385,21 +400,22 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
     const int c_end   = min(c_begin + p.walk_len, p.n_cg);
     if (c_begin >= c_end) return;
 
-    const float* __restrict__ rec_h = YT ? nullptr : b.pre + ((long long)seq * p.cpg * p.n_head + h) * (HELIX_CS * 4);
+    constexpr int RECF = B16 ? HELIX_REC_WALK_BYTES / 4 : HELIX_REC64_BYTES / 4;   // floats per record
+    const float* __restrict__ rec_h = YT ? nullptr : b.pre + ((long long)seq * p.cpg * p.n_head + h) * (HELIX_CS * RECF);
     const float* __restrict__ dt_h = b.dt + seq * p.seq_dt + h * p.s_dt[1];
     const float A_h = YT ? b.A[(long long)h * p.s_a] : 0.0f;
     const IO* __restrict__ x_h = reinterpret_cast<const IO*>(b.x) + seq * p.seq_x + h * p.s_x[1] + p0 * p.s_x[2];
-    const IO* __restrict__ B_g = reinterpret_cast<const IO*>(b.B) + seq * p.seq_b + g * p.s_b[1];
-    const IO* __restrict__ C_g = reinterpret_cast<const IO*>(b.C) + seq * p.seq_c + g * p.s_c[1];
+    const BIO* __restrict__ B_g = reinterpret_cast<const BIO*>(b.B) + seq * p.seq_b + g * p.s_b[1];
+    const BIO* __restrict__ C_g = reinterpret_cast<const BIO*>(b.C) + seq * p.seq_c + g * p.s_c[1];
 
     auto tlen_of = [&](int c) { return min(HELIX_CS, p.n_tok - (p.chunk_base + c) * HELIX_CS); };
 
     // Rows past tlen and state indices past d_state take an offset past the
     // resource's range and read 0.
-    WX6Run<IO, 4> rb[L];
-    WX6Run<IO, CE> rc[2];
+    WX6Run<BIO, 4> rb[L];
+    WX6Run<BIO, CE> rc[2];
     auto load_b = [&](int c, int ln) {
-        constexpr int ES = (int)sizeof(IO);
+        constexpr int ES = (int)sizeof(BIO);
         int bn, bt;
         wx6_b_rows<NP>(ln, wave, bn, bt);
         const int tl = tlen_of(c);
@@ -410,7 +426,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
         for (int i = 0; i < L; ++i) rb[i].load(rs, store_off_if_lt(((bt + i) * sb0 + bn) * ES, bt + i, tl, bn, N));
     };
     auto load_c = [&](int c, int ln) {
-        constexpr int ES = (int)sizeof(IO);
+        constexpr int ES = (int)sizeof(BIO);
         int cj, cn0, cpos;
         wx6_c_run<NP>(ln, wave, cj, cn0, cpos);
         const int tl = tlen_of(c);
@@ -445,13 +461,27 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
                                             ((tl - 1) * sdt + 1) * 4u);
             dtraw = buf_f32(rs, min(lane, tl - 1) * sdt * 4, 0);
         } else {
-            const helix_rsrc rs = make_rsrc(rec_h + (long long)c * p.n_head * (HELIX_CS * 4), HELIX_CS * 16u);
-            rec = __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, 0, 0);
+            const helix_rsrc rs = make_rsrc(rec_h + (long long)c * p.n_head * (HELIX_CS * RECF), HELIX_CS * RECF * 4u);
+            if constexpr (B16) {
+                const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(rs, lane * 8, 0, 0);
+                rec = u32x4{w[0], w[1], 0u, 0u};
+            } else {
+                rec = __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, 0, 0);
+            }
         }
     };
     // A chunk's records into buffer par, by one wave of each item.
     auto stage_rec = [&](int tl, int par) {
         if (pt != 1 || !item_ok) return;
+        if constexpr (B16) {
+            const float l2 = as_f32(rec[1]);
+            const float l2_end = __builtin_bit_cast(float, __builtin_amdgcn_readlane((int)rec[1], 63));
+            sDt[par][is][lane] = as_f32(rec[0]);
+            sW[par][is][lane] = __builtin_amdgcn_exp2f(l2_end - l2) * as_f32(rec[0]);
+            sE[par][is][lane] = __builtin_amdgcn_exp2f(l2);
+            sLh[par][is][lane] = l2;
+            return;
+        }
         float dtv, e;
         double lcum;
         if constexpr (YT) {
@@ -470,7 +500,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
         sW[par][is][lane] = exp2_diff(bcast(lcum, 63), lcum) * dtv;
         sE[par][is][lane] = e;
         sLh[par][is][lane] = l2h;
-        sLl[par][is][lane] = (float)(l2 - (double)l2h);
+        if constexpr (!B16) sLl[par][is][lane] = (float)(l2 - (double)l2h);
     };
     auto stage_c = [&](int ln) {
         int cj, cn0, cpos;
@@ -483,7 +513,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
                 unsigned w[2][NPL];
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
-                    if constexpr (NPL == 1)
+                    if constexpr (__is_same(BIO, __bf16))
                         w[e][0] = rc[k].w[2 * m + e];   // bf16 pairs as they are
                     else
                         wx6_split<NPL>(rc[k].at(4 * m + 2 * e), rc[k].at(4 * m + 2 * e + 1), w[e]);
@@ -503,7 +533,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
             unsigned w[L / 2][NPL];
 #pragma unroll
             for (int i = 0; i < L / 2; ++i) {
-                if constexpr (NPL == 1)   // the halves k % 2 of the two tokens' words as one pair
+                if constexpr (__is_same(BIO, __bf16))   // the halves k % 2 of the two tokens' words as one pair
                     w[i][0] = __builtin_amdgcn_perm(rb[2 * i + 1].w[k >> 1], rb[2 * i].w[k >> 1],
                                                     (k & 1) ? 0x07060302u : 0x05040100u);
                 else
@@ -614,11 +644,11 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
         acc[0] = zero16();
         acc[1] = zero16();
         if (item_ok) {
-            auto split_r = [&](int s, bf16x8 (&rp)[3]) {
+            auto split_r = [&](int s, bf16x8 (&rp)[NPX]) {
                 float rv[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) rv[e] = R[s >> 1][8 * (s & 1) + e];
-                wx6_split8<3>(rv, rp);
+                wx6_split8<NPX>(rv, rp);
             };
             auto read_c = [&](int s, bf16x8 (&cv)[2][NPL]) {
 #pragma unroll
@@ -627,7 +657,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
                     for (int pl = 0; pl < NPL; ++pl)
                         cv[tb][pl] = *reinterpret_cast<const bf16x8*>(rC + pl * PL_C + 32 * tb * RSC + 16 * s);
             };
-            bf16x8 cv[2][2][NPL], rp[2][3];
+            bf16x8 cv[2][2][NPL], rp[2][NPX];
             read_c(0, cv[0]);
             split_r(0, rp[0]);
 #pragma unroll
@@ -658,7 +688,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb) {
                 lth[tb] = sLh[par][is][32 * tb + lo];
-                ltl[tb] = sLl[par][is][32 * tb + lo];
+                ltl[tb] = B16 ? 0.0f : sLl[B16 ? 0 : par][is][32 * tb + lo];
             }
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
@@ -669,8 +699,8 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
 #pragma unroll
                     for (int k = 0; k < 4; ++k) v[4 * a + k] = d4[k] * io_widen<IO>(xs[s][4 * a + k]);
                 }
-                bf16x8 x2[3];
-                wx6_split8<3>(v, x2);
+                bf16x8 x2[NPX];
+                wx6_split8<NPX>(v, x2);
                 // M[t][j] = CB[t][j] exp(Lcum_t - Lcum_j), j <= t, of t tile tb
                 // at tokens j = 16 s + 8 hi + e.
                 const int lim = vgpr_fresh(lo - 8 * hi);
@@ -681,16 +711,19 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
                     for (int a = 0; a < 2; ++a) {
                         const f32x4 cb = *reinterpret_cast<const f32x4*>(rCB + 32 * tb * RSM + 16 * s + 4 * a);
                         const f32x4 jh = *reinterpret_cast<const f32x4*>(&sLh[par][is][16 * s + 8 * hi + 4 * a]);
-                        const f32x4 jl = *reinterpret_cast<const f32x4*>(&sLl[par][is][16 * s + 8 * hi + 4 * a]);
+                        f32x4 jl = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if constexpr (!B16) jl = *reinterpret_cast<const f32x4*>(&sLl[par][is][16 * s + 8 * hi + 4 * a]);
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
                             const int e = 4 * a + k;
-                            const float d = cb[k] * __builtin_amdgcn_exp2f((lth[tb] - jh[k]) + (ltl[tb] - jl[k]));
+                            float l = lth[tb] - jh[k];
+                            if constexpr (!B16) l += ltl[tb] - jl[k];
+                            const float d = cb[k] * __builtin_amdgcn_exp2f(l);
                             m[e] = (s >> 1) == tb ? (lim >= 16 * (s & 1) + e ? d : 0.0f) : d;
                         }
                     }
-                    bf16x8 mp[3];
-                    wx6_split8<3>(m, mp);
+                    bf16x8 mp[NPX];
+                    wx6_split8<NPX>(m, mp);
                     acc[tb] = wx6_mfma(mp, x2, acc[tb]);
                 }
             }
@@ -709,8 +742,8 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
 #pragma unroll
                     for (int k = 0; k < 4; ++k) v[4 * a + k] = w4[k] * io_widen<IO>(xs[s][4 * a + k]);
                 }
-                bf16x8 x4[3];
-                wx6_split8<3>(v, x4);
+                bf16x8 x4[NPX];
+                wx6_split8<NPX>(v, x4);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
                     bf16x8 bp[NPL];
@@ -741,7 +774,9 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
             acc[0] += yprev[0];
             acc[1] += yprev[1];
         }
-        if (item_ok) wx6_store_y<IO, HELIX_NT>(acc, p, b, seq, h, t0, tlen, p0, pw, pp, hi);
+        // Reading Pass A's bf16 copies: nt alone (HELIX_NT_L2).
+        constexpr int YAUX = sizeof(IO) == 4 && __is_same(BIO, __bf16) ? HELIX_NT_L2 : HELIX_NT;
+        if (item_ok) wx6_store_y<IO, YAUX>(acc, p, b, seq, h, t0, tlen, p0, pw, pp, hi);
         if (last) break;
         __syncthreads();   // (3)
     }
@@ -773,3 +808,21 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
 
 HELIX_PASS_C_WALK_X6(64)
 HELIX_PASS_C_WALK_X6(128)
+
+// The bf16 path's walk.
+#define HELIX_PASS_C_WALK_BF16(NAME, NP, ...)                                                   \
+    extern "C" __global__ __launch_bounds__(HELIX_HB_THREADS) void helix_scan_walk16_bf16_##NAME##n##NP( \
+        HelixScanParams p, HelixScanBuffers b) {                                                \
+        scan_walk_x6_impl<NP, __VA_ARGS__>(p, b);                                               \
+    }
+#define HELIX_PASS_C_WALK_BF16_ALL(NP)                                                          \
+    HELIX_PASS_C_WALK_BF16(, NP, float, false, false, true)                                     \
+    HELIX_PASS_C_WALK_BF16(bc_, NP, float, false, false, true, __bf16)                          \
+    HELIX_PASS_C_WALK_BF16(bf16io_, NP, __bf16, false, false, true)                             \
+    HELIX_PASS_C_WALK_BF16(f16io_, NP, _Float16, false, false, true)                            \
+    /* The second and later blocks of state indices. */                                         \
+    HELIX_PASS_C_WALK_BF16(acc_, NP, float, false, true, true)                                  \
+    HELIX_PASS_C_WALK_BF16(bc_acc_, NP, float, false, true, true, __bf16)
+
+HELIX_PASS_C_WALK_BF16_ALL(64)
+HELIX_PASS_C_WALK_BF16_ALL(128)

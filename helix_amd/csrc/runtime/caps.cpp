@@ -214,6 +214,7 @@ struct TraitTable {
                         t.np = kNps[k];
                         t.walk = true;
                         t.walk_hpw = HELIX_WALK16_HPW(kNps[k]);
+                        t.walk_hb = hb;
                         t.walk_fuse_b = true;
                         t.bccopy = bc != 0;
                         t.rec_kind = 1;
@@ -568,7 +569,7 @@ double fused_lengths_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, i
                                     (double)std::min(HELIX_HB, ipg - HELIX_HB * ib) / HELIX_HB);
     const double a = dispatch_us(wg, kCostA);
     // Walk: (item block, group, walk, sequence), or (head block, group, slab, walk, sequence).
-    if (tr.walk_hb) {
+    if (tr.walk_hb && !tr.bf16_state) {
         for (size_t i = 0, n = wg.size(); i < n; ++i) {
             const int s = (int)(i / ((size_t)nib * d.n_group) % nseg);
             wg[i].first += kCostWalkHb.o - kCostA.o + kCostWalkHb.g * s;
@@ -603,7 +604,7 @@ int fused_walk_len(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cp
     using Key = std::tuple<int, int, int, int, int, int, int, int>;
     static std::mutex mu;
     static std::map<Key, int> memo;
-    const Key key{d.n_seq, d.n_head, d.head_dim, d.n_group, tr.np, tr.walk_hb ? -1 : tr.walk_hpw, cpg, shortest};
+    const Key key{d.n_seq, d.n_head, d.head_dim, d.n_group, tr.np, tr.bf16_state ? tr.walk_hpw : -1, cpg, shortest};
     {
         std::lock_guard<std::mutex> lk(mu);
         const auto it = memo.find(key);
