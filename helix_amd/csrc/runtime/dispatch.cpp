@@ -19,9 +19,9 @@
 //   Pass C  grid (chunks * n_group * n_hblk * n_seq)    x 256 threads (1-D,
 //           decoded XCD-aware in the kernel); the walking variant runs one
 //           workgroup of 256 * HELIX_WALK_HPW(np) threads per (walk segment,
-//           block of that many heads of a group, P slab, seq) instead (bf16
-//           path), or of 512 threads per (run of chunks, item block of a
-//           group, seq) (fp32 path)
+//           block of that many heads of a group, P slab, seq) instead at
+//           d_state 256, or of 512 threads per (run of chunks, item block of
+//           a group, seq)
 // The ragged-tail padding and the bf16 staging of B and C that the reference
 // runs as separate passes (dispatch.mm:218-245) happen inside the Pass A/C
 // staging here, so there is nothing to launch before the group loop.
@@ -132,8 +132,6 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         return HELIX_ERR_INVALID_ARG;
     }
 
-    // A short scan runs as one launch of the single pass, whatever its plan
-    // (HELIX_ONLY_PASS times the plan's passes).
     // Whether the caller's scratch holds `need` bytes. The reference checks the
     // MTLBuffer length (dispatch.mm:150-153); the HIP analogue is the allocation
     // containing the pointer.
@@ -154,6 +152,8 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
                                    : "multipass requires a scratch buffer of helix_scan_scratch_size() bytes");
         return HELIX_ERR_SCRATCH_TOO_SMALL;
     };
+    // A short scan runs as one launch of the single pass, whatever its plan
+    // (HELIX_ONLY_PASS times the plan's passes).
     const HelixMatmulTraits* const one =
         std::getenv("HELIX_ONLY_PASS") ? nullptr : helix::rt::short_scan_traits(ctx, *d, sel);
     const HelixMatmulTraits* trp = one ? one : &sel;
@@ -518,6 +518,10 @@ extern "C" helix_status helix_scan_encode_noalloc(helix_ctx* ctx, void* stream, 
     // group is refused.
     const size_t need = noalloc_scratch_size(ctx, d);
     if (need > HELIX_NOALLOC_SCRATCH_BYTES) {
+        // 16-bit storage on the fp32 path does without.
+        if (helix::rt::select_traits(ctx, *d).fallback)
+            return encode_core(ctx, static_cast<hipStream_t>(stream), d, s0, x, dt, A, B, C, ids, y, s1,
+                               HELIX_TENSOR_NULL);
         set_error(ctx, "plan needs " + std::to_string(need) + " bytes of scratch at one chunk per group, more than the " +
                            std::to_string((size_t)HELIX_NOALLOC_SCRATCH_BYTES) +
                            " of the fixed scratch (HELIX_NOALLOC_SCRATCH_BYTES); use helix_scan_encode");

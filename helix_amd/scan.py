@@ -146,7 +146,11 @@ def ssd_scan(x: torch.Tensor, dt: torch.Tensor, A: torch.Tensor, B: torch.Tensor
         if rc != HELIX_ERR_SCRATCH_TOO_SMALL or have >= need:
             break
         if lent is not None:
-            raise ValueError(f"scratch needs {need} bytes")
+            # 16-bit storage on the fp32 path does without where it is lent too little.
+            rc, _ = ctx.run(st, d, ARGS_STRUCT.pack(*ptrs, 0, need))
+            if rc == HELIX_ERR_SCRATCH_TOO_SMALL:
+                raise ValueError(f"scratch needs {need} bytes")
+            break
         scratch = _scratch_for(index, need)
     if rc == HELIX_ERR_UNSUPPORTED_SHAPE:
         raise HelixError(1, f"shape declined: {ctx.backend_desc(HelixScanDesc.from_buffer_copy(d))}")

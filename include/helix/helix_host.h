@@ -98,7 +98,8 @@ typedef struct {
 /* helix_scan_supported, helix_scan_scratch_size and helix_scan_encode in one
  * call, for a host binding whose cost per call counts. *need is the scratch
  * size; with fewer scratch_bytes it returns HELIX_ERR_SCRATCH_TOO_SMALL and
- * enqueues nothing. scratch_bytes is taken at its word. */
+ * enqueues nothing. scratch_bytes is taken at its word, but a NULL scratch is
+ * none: a call that can do without runs, any other returns that status. */
 helix_status helix_scan_run(helix_ctx* ctx, void* stream, const helix_scan_desc* desc,
                             const helix_scan_args* args, size_t* need);
 

@@ -1,5 +1,5 @@
-"""The fp32 path's walk over item blocks (pass_c_walk_x6.hip) at the shapes where
-its work split can go wrong: one to five (head, P slab) items per B/C group
+"""The walk over item blocks (pass_c_walk_x6.hip) at the shapes where its work
+split can go wrong: one to five (head, P slab) items per B/C group
 (blocks of four with one to four live items; up to two take their waves a SIMD
 each), slabs and d_state short of their tiles, ragged last chunks, runs of one
 chunk and of several, and the state carried through the groups of a small
@@ -12,8 +12,8 @@ import pytest
 import torch
 
 from oracle import pyoracle as po
-from helix_amd.desc import HELIX_BACKEND_SGMMA, HELIX_BF16, HELIX_F16, HELIX_OK, HELIX_TENSOR_NULL
-from gpu_harness import F32_ABS, F32_REL, T, ctx_for, run
+from helix_amd.desc import HELIX_BACKEND_MPP, HELIX_BACKEND_SGMMA, HELIX_BF16, HELIX_F16, HELIX_OK, HELIX_TENSOR_NULL
+from gpu_harness import BF16_ABS, BF16_REL, F32_ABS, F32_REL, T, ctx_for, run
 from test_gpu_io import TORCH, U, rounded
 
 pytestmark = pytest.mark.gpu
@@ -41,6 +41,22 @@ def test_item_blocks(gpu, shape, knobs):
     assert b"helix_scan_walk_x6_n" in ctx.plan_info(d).kernel_c
     _, y, s1 = run(ctx, p, d)
     assert po.allclose_ratio(y, y_ref, F32_REL, F32_ABS) <= 1.0
+    assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
+
+
+@pytest.mark.parametrize("copies", ["0", "1"], ids=["rows", "copies"])
+@pytest.mark.parametrize("shape,knobs", SHAPES, ids=["x".join(map(str, s)) + ("k" if k else "") for s, k in SHAPES])
+def test_item_blocks_bf16(gpu, shape, knobs, copies):
+    """The bf16 path's instantiations, on the caller's rows of B and C and on Pass A's bf16 copies."""
+    p = po.problem_harness(*shape, 515, "long")
+    p.s0 = (np.random.default_rng(5).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
+    y_ref, s_ref = po.scan(p, use_ids=False)
+    ctx = ctx_for(gpu, HELIX_WALK_BCCOPY=copies, **knobs)
+    d = p.d.copy()
+    d.backend, d.multipass = HELIX_BACKEND_MPP, True
+    assert (b"helix_scan_walk16_bf16_bc_n" if copies == "1" else b"helix_scan_walk16_bf16_n") in ctx.plan_info(d).kernel_c
+    _, y, s1 = run(ctx, p, d)
+    assert po.allclose_ratio(y, y_ref, BF16_REL, BF16_ABS) <= 1.0
     assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
 
 
@@ -88,6 +104,39 @@ def test_16bit_storage(gpu, shape, pad, io):
         torch.cuda.synchronize()
         assert po.allclose_ratio(y.float().cpu().numpy(), y_ref, F32_REL + U[io], F32_ABS) <= 1.0, route
         assert po.allclose_ratio(s1.cpu().numpy(), s_ref, F32_REL, F32_ABS) <= 1.0, route
+
+
+@pytest.mark.parametrize("io", [HELIX_BF16, HELIX_F16], ids=["bf16", "f16"])
+def test_16bit_storage_lent_little(gpu, io):
+    """A tensor too small for the passes, lent to ssd_scan: the single pass's bits, as without scratch; a path
+    that needs its scratch still refuses it."""
+    from helix_amd import scan
+    p = po.problem_harness(513, 1, 5, 72, 120, 1, 616, "long")
+    x, dt, A, B, C = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (p.x, p.dt, p.A, p.B, p.C))
+    x, B, C = (t.to(TORCH[io]) for t in (x, B, C))
+    little = torch.empty(64, dtype=torch.uint8, device="cuda")
+    want = scan.ssd_scan(x, dt, A, B, C, backend="fp32", multipass=False)
+    got = scan.ssd_scan(x, dt, A, B, C, backend="fp32", scratch=little)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    with pytest.raises(ValueError):
+        scan.ssd_scan(x, dt, A, B, C, backend="bf16", scratch=little)
+
+
+def test_16bit_storage_past_fixed_scratch(gpu):
+    """helix_scan_encode_noalloc where one chunk per group exceeds its scratch: the single pass's bits."""
+    from helix_amd import scan
+    S, L, H, P, N = 65, 65, 64, 64, 128
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x, B, C = (torch.randn(S, L, k, n, generator=g, device="cuda").to(torch.bfloat16) for k, n in ((H, P), (1, N), (1, N)))
+    dt = torch.randn(S, L, H, generator=g, device="cuda")
+    A = -1.0 - torch.rand(H, generator=g, device="cuda")
+    s0 = torch.randn(S, H, P, N, generator=g, device="cuda")
+    y, s1 = torch.empty_like(x), torch.empty_like(s0)
+    d = scan.make_desc(x, dt, B, C, s0, y, A, backend="fp32")
+    rc = gpu.encode_noalloc(torch.cuda.current_stream().cuda_stream, d, *map(T, (s0, x, dt, A, B, C, None, y, s1)))
+    assert rc == HELIX_OK, gpu.last_error()
+    want = scan.ssd_scan(x, dt, A, B, C, s0, backend="fp32", multipass=False)
+    assert torch.equal(y, want[0]) and torch.equal(s1, want[1])
 
 
 # Short scans: at the limit of the one-launch route on each path (caps.cpp,
