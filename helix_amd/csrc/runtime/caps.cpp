@@ -167,7 +167,7 @@ struct TraitTable {
                 t.k_chunk_state = kernel("helix_chunk_state_hb_x6agg_r64_n" + np);
                 t.k_chunk_out = kernel("helix_scan_walk_x6_n" + np);
                 t.k_chunk_out_acc = kernel("helix_scan_walk_x6_acc_n" + np);
-                t.mfma_c = "v_mfma_f32_16x16x32_bf16 (bf16x6 split operands)";
+                t.mfma_c = "v_mfma_f32_32x32x16_bf16 (bf16x6 split operands)";
                 t.walk = true;
                 t.walk_hb = true;
                 t.walk_fuse_b = true;
@@ -210,7 +210,7 @@ struct TraitTable {
                         t.bf16_state = true;
                         t.mfma_a = s6 ? "v_mfma_f32_32x32x16_bf16 (bf16x6 split operands)"
                                       : "v_mfma_f32_32x32x16_bf16 (bf16x3 split operands)";
-                        t.mfma_c = "v_mfma_f32_16x16x32_bf16";
+                        t.mfma_c = hb ? "v_mfma_f32_32x32x16_bf16" : "v_mfma_f32_16x16x32_bf16";
                         t.np = kNps[k];
                         t.walk = true;
                         t.walk_hpw = HELIX_WALK16_HPW(kNps[k]);
