@@ -233,6 +233,7 @@ struct TraitTable {
                     t.mfma_a = io ? "v_mfma_f32_32x32x16_f16 (one scaled fp16 plane of B, two of x: two products)"
                                   : "v_mfma_f32_32x32x16_f16 (two scaled fp16 planes, three products)";
                 }
+        for (int k = 0; k < 2; ++k) h3[0][1][k].nocopy = &h3[0][0][k];
         // What helix_ctx_backend_desc reports for a descriptor run as blocks
         // of state indices on these kernels.
         auto blocks_name = [&](HelixMatmulTraits& t) {
@@ -265,14 +266,9 @@ bool bccopy_on(const helix_tuning& tu, const helix_scan_desc& d, bool block) {
     const long K = (long)(d.n_head / d.n_group) * ((d.head_dim + HELIX_HD - 1) / HELIX_HD);
     // The head-block Pass A (d_state <= 128) can copy at every shape (one
     // wave per 8-token block of a chunk and group, pass_a_hb.hip). The copies
-    // pay off when many walk workgroups read a chunk's rows (measured at
-    // configs 4a and 4b, 80 and 27 heads per group: 45 and 56 us faster);
-    // at 8 (config 2) the walk reading the fp32 rows itself is 3 us faster.
-    // Blocks of state indices: at config 2's shape with d_state 256 in two
-    // blocks of 128, the walks reading their columns of the caller's rows took
-    // 81 and 103 us, on the copies 69 and 79 us, for 15 us more per Pass A
-    // (0.279 against 0.273 ms a scan; 9 us and 0.297 against 0.280 ms with
-    // the six-product Pass A).
+    // paid off while a walk workgroup read a chunk's rows for two heads: with
+    // more than eight items per group, and for blocks of state indices. The plan
+    // keeps room for them there; what the encoder runs is no_copies' choice.
     if (d.d_state <= 128) return tu.bccopy == 1 || K > 8 || block;
     return (64 + K - 1) / K * (d.d_state / 4) <= 2 * 256;
 }
@@ -444,6 +440,17 @@ const HelixMatmulTraits& select_traits_unblocked(const helix_ctx* ctx, const hel
     // keeps the six.
     if (k < 2 && tu.passa_split != 3 && tu.passa_f16 != 0) return tt.h3[io][bc][k];
     return tt.bf16[io][tu.passa_split == 3 ? 0 : 1][bc][k];
+}
+
+// A walk workgroup reads a chunk's rows of B and C once for four items, and
+// copies cost Pass A more than they save the walk: without / with them, inputs
+// out of the Infinity Cache, 4096 tokens at d_state 256 158.8 / 168.7 us (8 x 1024
+// tokens of 80 heads 393 / 407), 8 x 4096 tokens of 80 heads 507 / 514 and of 27
+// heads of 192 509 / 514, 2 x 2000 of 48 heads in four groups 84.3 / 87.7, 8192 of
+// 24 heads 83.8 / 85.5, 4 x 1000 of 8 heads of 128 38.4 / 39.5, 2 x 4096 of 64 heads
+// at d_state 64 100.6 / 103.5; slower at no shape measured.
+const HelixMatmulTraits& no_copies(const helix_ctx* ctx, const HelixMatmulTraits& tr) {
+    return tr.nocopy && tuning_of(ctx).planned ? *tr.nocopy : tr;
 }
 
 const HelixMatmulTraits* short_scan_traits(const helix_ctx* ctx, const helix_scan_desc& d,

@@ -251,8 +251,12 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         return no_scratch();
     }
 
-    hipFunction_t fA = fn(tr.k_chunk_state), fB = fn(tr.k_state_scan),
-                  fC = fn(y_acc && tr.k_chunk_out_acc ? tr.k_chunk_out_acc : tr.k_chunk_out);
+    // y over B or C: the walk must read Pass A's copies.
+    const bool keep_copies = tr.nocopy && y_overlaps_others(*d, dptr(y), dptr(x), dptr(dt), dptr(A), dptr(B), dptr(C),
+                                                            dptr(s0), dptr(ids), dptr(s1));
+    const HelixMatmulTraits& kt = keep_copies ? tr : helix::rt::no_copies(ctx, tr);
+    hipFunction_t fA = fn(kt.k_chunk_state), fB = fn(kt.k_state_scan),
+                  fC = fn(y_acc && kt.k_chunk_out_acc ? kt.k_chunk_out_acc : kt.k_chunk_out);
     if (!fA || !fB || !fC) {
         set_error(ctx, "kernel not resolved in code object");
         return HELIX_ERR_PIPELINE;
@@ -373,7 +377,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
             // absolute row t0 lands on the group's row t0 - 64 base.
             HelixScanParams pc = params;
             HelixScanBuffers bc = bufs;
-            if (tr.bccopy) {
+            if (kt.bccopy) {
                 const long long gn = (long long)d->n_group * d->d_state;
                 for (long long* s3 : {pc.s_b, pc.s_c}) {
                     s3[0] = gn;

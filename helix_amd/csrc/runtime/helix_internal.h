@@ -94,6 +94,9 @@ struct HelixMatmulTraits {
     bool          walk_hb;
     // Pass A writes bf16 copies of B and C that the walking Pass C reads.
     bool          bccopy;
+    // The kernels the encoder runs on a bccopy plan, without the copies (null:
+    // the plan's own; no_copies in caps.cpp).
+    const HelixMatmulTraits* nocopy;
     // The walking Pass C can run Pass B's segment scan in its prologue
     // (HelixScanParams::fuse_b); the encoder then skips Pass B's launch
     // whenever the plan has a single group.
@@ -170,6 +173,10 @@ bool one_launch_scan(const helix_scan_desc& d, bool fp32_path);
 // 128 and no tuning override. Null otherwise.
 const HelixMatmulTraits* short_scan_traits(const helix_ctx* ctx, const helix_scan_desc& d,
                                            const HelixMatmulTraits& tr);
+
+// The kernels the encoder runs on a plan of `tr`: those without bf16 copies of B
+// and C up to d_state 128 and no tuning override, else `tr` itself.
+const HelixMatmulTraits& no_copies(const helix_ctx* ctx, const HelixMatmulTraits& tr);
 
 // Whether the walking Pass C runs Pass B's segment scan itself (no Pass B
 // launch): a single-group plan of at most four segments on a kernel that can;

@@ -75,7 +75,8 @@ typedef struct {
 /* The plan of the passes. A scan of a few chunks is encoded as one launch of
  * the single pass instead, whatever its plan, where that is faster (scalar A,
  * d_state up to 128 or blocks of it, no tuning variable set); its scratch then
- * stays unused. */
+ * stays unused. Likewise a plan with bf16 copies of B and C up to d_state 128 (or
+ * blocks of it) runs the same kernels without them, and bccopy_bytes stay unused. */
 /* Returns HELIX_ERR_UNSUPPORTED_SHAPE when the descriptor is declined. */
 helix_status helix_scan_plan_info(helix_ctx* ctx, const helix_scan_desc* d,
                                   helix_plan_info* out);

@@ -169,6 +169,22 @@ def test_short_scan(gpu, shape, one):
     assert same
 
 
+@pytest.mark.parametrize("shape", [(900, 2, 9, 64, 128, 1), (700, 1, 5, 136, 64, 1), (900, 1, 4, 64, 256, 2)],
+                         ids=["nine items", "three slabs", "state blocks"])
+def test_copy_plan_runs_without_copies(gpu, shape):
+    """Plans with bf16 copies of B and C: the bits of the plan without them."""
+    p = po.problem_harness(*shape, 919, "long")
+    d = p.d.copy()
+    d.backend, d.multipass = HELIX_BACKEND_MPP, True
+    assert gpu.plan_info(d).bccopy_bytes > 0
+    _, y, s1 = run(gpu, p, d)
+    _, y0, s0 = run(ctx_for(gpu, HELIX_WALK_BCCOPY="0"), p, d)
+    assert np.array_equal(y, y0) and np.array_equal(s1, s0)
+    y_ref, s_ref = po.scan(p, use_ids=False)
+    assert po.allclose_ratio(y, y_ref, BF16_REL, BF16_ABS) <= 1.0
+    assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
+
+
 NO_STATE = [   # (shape, multipass, backend, knobs): every place that reads s0
     ((700, 1, 64, 64, 128, 8), True, "fp32", {}),                      # Pass B
     ((1500, 1, 8, 64, 64, 1), True, "bf16", {"HELIX_SCRATCH_MB": 1}),  # Pass B, many groups
