@@ -438,8 +438,8 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
     };
     // K step s (tokens 16 s + 8 hi + e) of chunk c's x, in storage form. Rows
     // past tlen read 0 (past the resource's range) or, with strides under which
-    // a token row is shorter than the slab, another element of the chunk: dt is
-    // 0 for them either way.
+    // a token row is shorter than the slab, another element of the buffer, which
+    // mask_x clears.
     typename IoWord<IO>::type xs[4][8];
     auto load_x = [&](int c, int s) {
         const int tl = tlen_of(c);
@@ -449,6 +449,18 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
         const int xv = min(pp, pw - 1) * sx2 + 8 * hi * sx0;
 #pragma unroll
         for (int e = 0; e < 8; ++e) xs[s][e] = io_load_word<IO>(rx, xv, (16 * s + e) * sx0);
+    };
+    // dt is 0 past tlen, but 0 times an Inf or NaN of the caller's padding is
+    // not, and an MFMA spreads it over the tile's rows. Only a ragged chunk of
+    // such strides comes here: a weight that ignores what it multiplies
+    // (mul_legacy) would also ignore it at a token whose dt is exactly 0.
+    auto mask_x = [&](int tl, int hi) {
+        if (tl >= HELIX_CS || (int)p.s_x[0] > (pw - 1) * (int)p.s_x[2]) return;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (16 * s + 8 * hi + e >= tl) xs[s][e] = 0;
     };
     // The decay record of token lane (store_decay_record64: dt, exp(Lcum), Lcum
     // in fp64), or with YT the token's dt.
@@ -761,6 +773,8 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
             stage_rec(tlen_of(c + 1), par ^ 1);
             load_rec(cnn);
             __builtin_amdgcn_sched_barrier(0);
+        } else {
+            mask_x(tlen, hi);   // only a sequence's last chunk is ragged
         }
         if (item_ok) g2();
         if (!last && item_ok) {
