@@ -121,6 +121,10 @@ HELIX_DEV int wx6_jb(int idx) {
     return idx - tb * (tb + 1) / 2;
 }
 
+// Lcum log2(e) as a walk keeps it: fp64, or as the bf16 path's records have it.
+template <bool B16> struct WX6Lcum { typedef double type; };
+template <> struct WX6Lcum<true> { typedef float type; };
+
 constexpr int WX6_RSJ = HELIX_CS + 8;              // B^T rows (elements)
 constexpr int WX6_RSM = HELIX_CS + 4;              // CB rows (floats)
 template <int NP> constexpr int WX6_RSC = NP + 8;  // C rows (elements)
@@ -361,11 +365,13 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
     __shared__ __attribute__((aligned(16))) __bf16 sBt[NPL * PL_B];
     __shared__ __attribute__((aligned(16))) float sCB[HELIX_CS * RSM];
     // Decay records of the chunk's and the next chunk's tokens, by parity: dt
-    // (0 past tlen), exp(L_end - Lcum) dt, exp(Lcum), and Lcum log2(e) as the
-    // sum of two floats (differences of Lcum keep fp32's precision at any
-    // magnitude of Lcum).
+    // (0 past tlen), exp(L_end - Lcum) dt, exp(Lcum), and Lcum log2(e) in fp64
+    // (B16: fp32, as its records have it): differences of Lcum keep fp32's
+    // precision at any magnitude, and are exact where every Lcum is past
+    // fp32's range (A at the lowest float, a state without memory).
     __shared__ __attribute__((aligned(16))) float sDt[2][HB][HELIX_CS], sW[2][HB][HELIX_CS], sE[2][HB][HELIX_CS];
-    __shared__ __attribute__((aligned(16))) float sLh[2][HB][HELIX_CS], sLl[B16 ? 1 : 2][HB][HELIX_CS];
+    using LcumT = typename WX6Lcum<B16>::type;
+    __shared__ __attribute__((aligned(16))) LcumT sL2[2][HB][HELIX_CS];
 
     const int lane = threadIdx.x & 63, wave = wave_uniform(), lo = lane & 31, hi = lane >> 5;
     const int N = p.d_state;
@@ -491,7 +497,7 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
             sDt[par][is][lane] = as_f32(rec[0]);
             sW[par][is][lane] = __builtin_amdgcn_exp2f(l2_end - l2) * as_f32(rec[0]);
             sE[par][is][lane] = __builtin_amdgcn_exp2f(l2);
-            sLh[par][is][lane] = l2;
+            sL2[par][is][lane] = l2;
             return;
         }
         float dtv, e;
@@ -506,13 +512,10 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
             e = as_f32(rec[1]);
             lcum = __builtin_bit_cast(double, (unsigned long long)rec[2] | ((unsigned long long)rec[3] << 32));
         }
-        const double l2 = lcum * 1.4426950408889634074;
-        const float l2h = (float)l2;
         sDt[par][is][lane] = dtv;
         sW[par][is][lane] = exp2_diff(bcast(lcum, 63), lcum) * dtv;
         sE[par][is][lane] = e;
-        sLh[par][is][lane] = l2h;
-        if constexpr (!B16) sLl[par][is][lane] = (float)(l2 - (double)l2h);
+        sL2[par][is][lane] = lcum * 1.4426950408889634074;
     };
     auto stage_c = [&](int ln) {
         int cj, cn0, cpos;
@@ -696,12 +699,9 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
         const float* const rCB = sCB + lo * RSM + 8 * hi;     // row lo of a tile of CB
         const __bf16* const rB = sBt + lo * RSJ + 8 * hi;     // operand row lo of B^T
         auto g2 = [&] {
-            float lth[2], ltl[2];
+            LcumT lt[2];
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb) {
-                lth[tb] = sLh[par][is][32 * tb + lo];
-                ltl[tb] = B16 ? 0.0f : sLl[B16 ? 0 : par][is][32 * tb + lo];
-            }
+            for (int tb = 0; tb < 2; ++tb) lt[tb] = sL2[par][is][32 * tb + lo];
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 float v[8];
@@ -722,15 +722,13 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
 #pragma unroll
                     for (int a = 0; a < 2; ++a) {
                         const f32x4 cb = *reinterpret_cast<const f32x4*>(rCB + 32 * tb * RSM + 16 * s + 4 * a);
-                        const f32x4 jh = *reinterpret_cast<const f32x4*>(&sLh[par][is][16 * s + 8 * hi + 4 * a]);
-                        f32x4 jl = {0.0f, 0.0f, 0.0f, 0.0f};
-                        if constexpr (!B16) jl = *reinterpret_cast<const f32x4*>(&sLl[par][is][16 * s + 8 * hi + 4 * a]);
+                        LcumT lj[4];
+                        __builtin_memcpy(lj, __builtin_assume_aligned(&sL2[par][is][16 * s + 8 * hi + 4 * a], 16),
+                                         sizeof(lj));
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
                             const int e = 4 * a + k;
-                            float l = lth[tb] - jh[k];
-                            if constexpr (!B16) l += ltl[tb] - jl[k];
-                            const float d = cb[k] * __builtin_amdgcn_exp2f(l);
+                            const float d = cb[k] * __builtin_amdgcn_exp2f((float)(lt[tb] - lj[k]));
                             m[e] = (s >> 1) == tb ? (lim >= 16 * (s & 1) + e ? d : 0.0f) : d;
                         }
                     }

@@ -1,6 +1,6 @@
 """Inputs at the edge of what the walks (pass_c_walk_x6.hip) take: x and y with
 tokens inside channels, padded with NaN, and a ragged last chunk, on every
-route. Against the fp64 oracle, to the bounds of the parity and storage suites:
+route; decays whose sums leave fp32's range, at fp32 accuracy. Against the fp64 oracle, to the bounds of the parity and storage suites:
 y on the fp32 path at the fp32 per-element bound (plus its rounding to 16-bit
 storage), on the bf16 path at the bf16 bound, s1 at the fp32 bound."""
 from __future__ import annotations
@@ -68,3 +68,25 @@ def test_tokens_inside_channels(gpu, route):
     torch.cuda.synchronize()
     check(p, y, s1, io, backend == "auto" and multipass)
     assert dense or torch.isnan(yb[..., L:]).all()
+
+
+@pytest.mark.parametrize("route", [r for r in ROUTES if r[1] == "fp32" or not r[2]],
+                         ids=lambda r: f"{r[0]}-{r[1]}-{IDS[r[3]]}-n{r[4]}")
+def test_lowest_decay(gpu, route):
+    """Heads without memory between ordinary ones: the sums of dt A over a chunk pass fp32's range from the first
+    tokens on (A at the lowest float), in the chunk's later tokens only (-1e37), or not at all (-1e30)."""
+    label, backend, multipass, io, N = route
+    S, L, H, P = 2, 714, 16, 128 if label == "tiles in y" else 72
+    p = po.problem_harness(L, S, H, P, N, 1, 4321, "long")
+    p = rounded(p, io) if io != HELIX_F32 else p
+    p.A[::4] = np.finfo(np.float32).min
+    p.A[1::4] = -1e37
+    p.A[2::4] = -1e30
+    p.dt += 6.0     # dt of about 0.6
+    x, B, C = up(p.x, TORCH[io]), up(p.B, TORCH[io]), up(p.C, TORCH[io])
+    d = make_desc(x, up(p.dt), B, C, up(p.s0), x, up(p.A), backend=backend, multipass=multipass)
+    info = gpu.plan_info(d)
+    assert b"walk" in info.kernel_c if label != "one launch" else info.kernel_c is None
+    y, s1 = ssd_scan(x, up(p.dt), up(p.A), B, C, up(p.s0), backend=backend, multipass=multipass)
+    torch.cuda.synchronize()
+    check(p, y, s1, io, False)
