@@ -8,8 +8,10 @@ only; all arithmetic runs in the HIP kernels of libhelix.so.
 """
 from __future__ import annotations
 
+import contextlib
 import math
 import threading
+from collections import OrderedDict
 from ctypes import c_float
 
 import torch
@@ -26,8 +28,12 @@ IO_DTYPES = {torch.float32: HELIX_F32, torch.bfloat16: HELIX_BF16, torch.float16
 
 _ctx_lock = threading.Lock()
 _contexts: dict[int, Context] = {}
-# Scratch is per thread and device, grown monotonically, as the ggml bridge
-# keeps it (ggml-helix.cpp:94-130): concurrent encoders must not share one.
+# Scratch is kept per thread, device and stream (the last SCRATCH_STREAMS that
+# a thread used), grown monotonically: scans that may run at the same time must
+# not share one. Each buffer is allocated under its own stream, so one that is
+# replaced or dropped goes back to the allocator for later work of that stream
+# only.
+SCRATCH_STREAMS = 8
 _scratch = threading.local()
 
 
@@ -46,16 +52,39 @@ def tensor_arg(t: torch.Tensor | None) -> HelixTensor:
     return HelixTensor(t.data_ptr(), 0)
 
 
-def _scratch_for(device: int, nbytes: int) -> torch.Tensor | None:
-    """This thread's scratch on the device, grown to nbytes (0: as it is)."""
+def _scratch_for(device: int, st: int, nbytes: int, stream: torch.cuda.Stream | None = None) -> torch.Tensor | None:
+    """This thread's scratch on the device for the stream of handle st, grown to nbytes (0: as it is). stream: the
+    stream object where it may not be the current one."""
     pool = getattr(_scratch, "pool", None)
     if pool is None:
-        pool = _scratch.pool = {}
-    buf = pool.get(device)
+        pool = _scratch.pool = OrderedDict()
+    key = (device, st)
+    buf = pool.get(key)
+    if buf is not None:
+        pool.move_to_end(key)
     if nbytes and (buf is None or buf.numel() < nbytes):
-        buf = torch.empty(nbytes, dtype=torch.uint8, device=f"cuda:{device}")
-        pool[device] = buf
+        with _under(device, st, stream):
+            buf = torch.empty(nbytes, dtype=torch.uint8, device=f"cuda:{device}")
+        pool[key] = buf
+        if len(pool) > SCRATCH_STREAMS:
+            pool.popitem(last=False)
     return buf
+
+
+def _capturing(device: int, st: int, stream) -> bool:
+    if stream is None:
+        return torch.cuda.is_current_stream_capturing()
+    with _under(device, st, stream):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def _under(device: int, st: int, stream):
+    """The context in which torch allocates for the stream."""
+    if stream is None:
+        return contextlib.nullcontext()
+    if not isinstance(stream, torch.cuda.Stream):
+        stream = torch.cuda.ExternalStream(st, device=device) if st else torch.cuda.default_stream(device)
+    return torch.cuda.stream(stream)
 
 
 def make_desc(x: torch.Tensor, dt: torch.Tensor, B: torch.Tensor, C: torch.Tensor,
@@ -136,8 +165,10 @@ def ssd_scan(x: torch.Tensor, dt: torch.Tensor, A: torch.Tensor, B: torch.Tensor
     ctx = _contexts.get(index) or context(index)
     st = stream.cuda_stream if stream is not None else torch.cuda.current_stream(dev).cuda_stream
     lent = scratch
-    if scratch is None:
-        scratch = _scratch_for(index, 0)
+    # Work under capture gets memory of the graph's own, which no later call touches.
+    capturing = lent is None and _capturing(index, st, stream)
+    if lent is None and not capturing:
+        scratch = _scratch_for(index, st, 0)
     ptrs = (0 if s0 is None else s0.data_ptr(), x.data_ptr(), dt.data_ptr(), A.data_ptr(), B.data_ptr(), C.data_ptr(),
             0 if ids is None else ids.data_ptr(), y.data_ptr(), s1.data_ptr())
     while True:
@@ -151,7 +182,11 @@ def ssd_scan(x: torch.Tensor, dt: torch.Tensor, A: torch.Tensor, B: torch.Tensor
             if rc == HELIX_ERR_SCRATCH_TOO_SMALL:
                 raise ValueError(f"scratch needs {need} bytes")
             break
-        scratch = _scratch_for(index, need)
+        if capturing:
+            with _under(index, st, stream):
+                scratch = torch.empty(need, dtype=torch.uint8, device=dev)
+        else:
+            scratch = _scratch_for(index, st, need, stream)
     if rc == HELIX_ERR_UNSUPPORTED_SHAPE:
         raise HelixError(1, f"shape declined: {ctx.backend_desc(HelixScanDesc.from_buffer_copy(d))}")
     if rc != HELIX_OK:
