@@ -62,16 +62,20 @@ ByteRange byte_range(const void* base, long long n_seq, long long seq_stride,
 // or writes besides y once its first launch has written state tiles into y:
 // x, dt, A, B, C, s1, ids, and s0 (its rows 0 .. n_seq - 1 without ids; with
 // ids the rows read are not known to the host and s0 is left out).
+// x_in_place: y at x's address with x's strides is no overlap with x.
 bool y_overlaps_others(const helix_scan_desc& d, const void* y, const void* x, const void* dt, const void* A,
-                       const void* B, const void* C, const void* s0, const void* ids, const void* s1) {
+                       const void* B, const void* C, const void* s0, const void* ids, const void* s1,
+                       bool x_in_place = false) {
     const long long T = d.n_tok, S = d.n_seq;
     const size_t es = d.io_dtype == HELIX_F32 ? 4 : 2;   // x, B, C and y
     const ByteRange ry = byte_range(y, S, d.seq_y, {{T, d.s_y[0]}, {d.n_head, d.s_y[1]}, {d.head_dim, d.s_y[2]}}, es);
     auto state = [&](const void* p) {
         return byte_range(p, S, d.seq_s, {{d.n_head, d.s_s[0]}, {d.head_dim, d.s_s[1]}, {d.d_state, d.s_s[2]}}, 4);
     };
+    const bool skip_x = x_in_place && x == y && d.seq_x == d.seq_y && std::equal(d.s_x, d.s_x + 3, d.s_y);
     const ByteRange others[] = {
-        byte_range(x, S, d.seq_x, {{T, d.s_x[0]}, {d.n_head, d.s_x[1]}, {d.head_dim, d.s_x[2]}}, es),
+        skip_x ? ByteRange{}
+               : byte_range(x, S, d.seq_x, {{T, d.s_x[0]}, {d.n_head, d.s_x[1]}, {d.head_dim, d.s_x[2]}}, es),
         byte_range(dt, S, d.seq_dt, {{T, d.s_dt[0]}, {d.n_head, d.s_dt[1]}}, 4),
         byte_range(A, 1, 0, {{d.n_head, d.s_a}}, 4),
         byte_range(B, S, d.seq_b, {{T, d.s_b[0]}, {d.n_group, d.s_b[1]}, {d.d_state, d.s_b[2]}}, es),
@@ -153,9 +157,16 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         return HELIX_ERR_SCRATCH_TOO_SMALL;
     };
     // A short scan runs as one launch of the single pass, whatever its plan
-    // (HELIX_ONLY_PASS times the plan's passes).
-    const HelixMatmulTraits* const one =
+    // (HELIX_ONLY_PASS times the plan's passes). Not where y overlaps what
+    // other workgroups still read: each walks the sequence on its own, while
+    // the passes have read dt, and B and C where the plan copies them, before
+    // the first y is written. y in x's place is read by its own workgroup.
+    const HelixMatmulTraits* one =
         std::getenv("HELIX_ONLY_PASS") ? nullptr : helix::rt::short_scan_traits(ctx, *d, sel);
+    if (one && !sel.k_single &&
+        y_overlaps_others(*d, dptr(y), dptr(x), dptr(dt), dptr(A), dptr(B), dptr(C), dptr(s0), dptr(ids), dptr(s1),
+                          /*x_in_place=*/true))
+        one = nullptr;
     const HelixMatmulTraits* trp = one ? one : &sel;
     // It needs no scratch, but the caller's contract is the plan's.
     if (one && !sel.k_single && !sel.fallback &&

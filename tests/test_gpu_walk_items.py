@@ -169,6 +169,30 @@ def test_short_scan(gpu, shape, one):
     assert same
 
 
+@pytest.mark.parametrize("over", ["C", "dt", "x"])
+def test_short_scan_y_over_input(gpu, over):
+    """A short scan whose y lies over C or dt runs the passes, which have read both before y is written (C as Pass A's
+    bf16 copy); over x, in x's strides, the one launch. Bits of the same route with a y of its own."""
+    from helix_amd import scan
+    L, S, H, P, N, G = 300, 1, 16, 64, 128, 1
+    p = po.problem_harness(L, S, H, P, N, G, 929, "long")
+    x, dt, A, B, C, s0 = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (p.x, p.dt, p.A, p.B, p.C, p.s0))
+    route = gpu if over == "x" else ctx_for(gpu, HELIX_WALK_BCCOPY="1")
+    d = p.d.copy()
+    d.backend, d.multipass = HELIX_BACKEND_MPP, True
+    _, y_want, s_want = run(route, p, d)
+    y = x.clone() if over == "x" else torch.full_like(x, float("nan"))
+    if over == "x":
+        x = y
+    elif over == "C":       # the first N columns of y's rows
+        C = y.view(S, L, 1, H * P)[..., :N].copy_(C)
+    else:                   # a column of H of them
+        dt = y.view(S, L, H * P)[..., :H].copy_(dt)
+    _, s1 = scan.ssd_scan(x, dt, A, B, C, s0, backend="bf16", y=y)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), y_want) and np.array_equal(s1.cpu().numpy(), s_want)
+
+
 @pytest.mark.parametrize("shape", [(900, 2, 9, 64, 128, 1), (700, 1, 5, 136, 64, 1), (900, 1, 4, 64, 256, 2)],
                          ids=["nine items", "three slabs", "state blocks"])
 def test_copy_plan_runs_without_copies(gpu, shape):
