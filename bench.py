@@ -100,6 +100,7 @@ class Variant:
         assert ctx.supported(self.d), ctx.backend_desc(self.d)
         self.kernel = ctx.backend_desc(self.d)
         self.plan = ctx.plan_info(self.d)
+        self.runs = ctx.run_info(self.d)   # what of the plan is launched
         self.scratch = torch.empty(max(1, ctx.scratch_size(self.d)), dtype=torch.uint8,
                                    device=x.device)
         self.args = [tensor_arg(t) for t in (s0, x, dt, A, B, C)]
@@ -250,7 +251,7 @@ def pass_us(passes, stat="median"):
     return {k: max(0.0, dist(ts)[stat] - x) * 1e3 for k, ts in passes.items() if k != "X"}
 
 
-def pass_algorithmic_bytes(plan):
+def pass_algorithmic_bytes(plan, runs):
     """Bytes each pass must move once at config 2 on the bf16 path (the
     scratch it writes or reads included, since the pass cannot avoid it)."""
     L, S, H, P, N, G = (CFG[k] for k in "LSHPNG")
@@ -260,15 +261,15 @@ def pass_algorithmic_bytes(plan):
     state = S * H * P * N * 4
     # With bf16 copies of B and C, Pass A also reads C and writes both copies,
     # and Pass C reads the copies instead.
-    cp = plan.bccopy_bytes
+    cp = plan.bccopy_bytes if runs.copies else 0
     # With Pass B run by the walking Pass C (no kernel_b), Pass C also reads s0
     # and writes s1; the segment aggregates are read once either way. Pass A
     # writes the per-token decay records, which Pass C reads instead of dt.
     fused = not plan.kernel_b
     rec = plan.rec_bytes
-    # Pass B stores, and a walking Pass C reads, the start states of the walks
-    # only (one per walk_len chunks); off the walk, every segment's.
-    starts = state * plan.walks_per_group if plan.walk_len != plan.seg_len else plan.s_seg_bytes
+    # Pass B stores, and a walking Pass C reads, the start states of its runs
+    # only (one per run_len chunks); off the walk, every segment's.
+    starts = state * runs.runs_per_group if runs.run_len > plan.seg_len else plan.s_seg_bytes
     return {
         "A": x + dt + bc + plan.s_local_bytes + plan.s_seg_bytes + ((bc + cp) if cp else 0) + rec,
         "B": 0 if fused else plan.s_seg_bytes + starts + 2 * state,
@@ -607,7 +608,7 @@ def main():
         peak_c = PEAK_BF16_MFMA if v.name == "bf16" else PEAK_FP32_MFMA
         t_roof = max(F_A / PEAK_FP32_MFMA + F_C / peak_c, bytes_alg / PEAK_HBM)
         results[v.name] = dict(ms=ms, d=d, wall_ms=wall, passes=passes, in_scan=in_scan, t_roof=t_roof, place=place,
-                               kernel=v.kernel, plan=v.plan)
+                               kernel=v.kernel, plan=v.plan, runs=v.runs)
 
     # Dominant kernel of the headline (bf16) path and its roofline. Every pass
     # is HBM-bound at this shape (Pass C: ~0.49 GB against ~6 us of bf16 MFMA
@@ -620,10 +621,11 @@ def main():
     pa = pass_us(r["passes"])                   # median kernel time per pass (split encodes), us
     pin = r["in_scan"]                          # mean time per pass inside whole scans, us
     plan = r["plan"]
-    pass_bytes = pass_algorithmic_bytes(plan)
+    runs = r["runs"]
+    pass_bytes = pass_algorithmic_bytes(plan, runs)
     # Pass B has no kernel of its own when the walking Pass C runs its scan
-    # (plan.kernel_b is null): its bytes and time are then Pass C's.
-    kernels = {"A": plan.kernel_a, "B": plan.kernel_b, "C": plan.kernel_c}
+    # (kernel_b is null): its bytes and time are then Pass C's.
+    kernels = {"A": runs.kernel_a, "B": runs.kernel_b, "C": runs.kernel_c}
     live = [k for k in "ABC" if kernels[k]]
     dom = max(live, key=lambda k: pin[k])
     kname = kernels[dom].decode()

@@ -27,7 +27,8 @@ ABI_SYMBOLS = (
     "helix_scan_encode",
     "helix_scan_encode_into",
 )
-HOST_SYMBOLS = ("helix_ctx_create_host", "helix_scan_plan_info", "helix_scan_run", "helix_scan_encode_noalloc")
+HOST_SYMBOLS = ("helix_ctx_create_host", "helix_scan_plan_info", "helix_scan_run_info", "helix_scan_run",
+                "helix_scan_encode_noalloc")
 # include/helix/helix_host.h HELIX_PASS_B_*: where Pass B's segment scan runs
 PASS_B_LAUNCHED, PASS_B_IN_C = 0, 1
 # include/helix/helix_host.h HELIX_NOALLOC_SCRATCH_BYTES
@@ -60,6 +61,19 @@ class HelixPlanInfo(ctypes.Structure):
         ("pass_b", c_int32),
         ("state_in_y", c_int32),
         ("state_blocks", c_int32),
+    ]
+
+
+class HelixRunInfo(ctypes.Structure):
+    _fields_ = [
+        ("one_launch", c_int32),
+        ("copies", c_int32),
+        ("run_len", c_int32),
+        ("runs_per_group", c_int32),
+        ("kernel_a", ctypes.c_char_p),
+        ("kernel_b", ctypes.c_char_p),
+        ("kernel_c", ctypes.c_char_p),
+        ("kernel_1pass", ctypes.c_char_p),
     ]
 
 
@@ -119,6 +133,8 @@ def lib():
     L.helix_scan_run.restype = c_int
     L.helix_scan_plan_info.argtypes = [c_void_p, dp, POINTER(HelixPlanInfo)]
     L.helix_scan_plan_info.restype = c_int
+    L.helix_scan_run_info.argtypes = [c_void_p, dp, POINTER(HelixRunInfo)]
+    L.helix_scan_run_info.restype = c_int
     _lib = L
     return L
 
@@ -177,6 +193,13 @@ class Context:
     def plan_info(self, d: HelixScanDesc) -> HelixPlanInfo:
         info = HelixPlanInfo()
         st = lib().helix_scan_plan_info(self.handle, ctypes.byref(d), ctypes.byref(info))
+        if st != HELIX_OK:
+            raise HelixError(st, "descriptor declined")
+        return info
+
+    def run_info(self, d: HelixScanDesc) -> HelixRunInfo:
+        info = HelixRunInfo()
+        st = lib().helix_scan_run_info(self.handle, ctypes.byref(d), ctypes.byref(info))
         if st != HELIX_OK:
             raise HelixError(st, "descriptor declined")
         return info

@@ -644,3 +644,36 @@ extern "C" helix_status helix_scan_plan_info(helix_ctx* ctx, const helix_scan_de
     out->pass_b = fuse_b ? HELIX_PASS_B_IN_C : HELIX_PASS_B_LAUNCHED;
     return HELIX_OK;
 }
+
+extern "C" helix_status helix_scan_run_info(helix_ctx* ctx, const helix_scan_desc* d, helix_run_info* out) {
+    if (!ctx || !d || !out) return HELIX_ERR_INVALID_ARG;
+    if (!helix_scan_supported(ctx, d)) return HELIX_ERR_UNSUPPORTED_SHAPE;
+    std::memset(out, 0, sizeof(*out));
+    // As encode_one decides.
+    const helix_scan_desc pd = helix::rt::plan_desc(ctx, *d);
+    const HelixMatmulTraits* tr = &helix::rt::select_traits(ctx, *d);
+    helix::rt::MultipassPlan pl;
+    const HelixMatmulTraits* const one = helix::rt::short_scan_traits(ctx, pd, *tr);
+    if (one) {
+        tr = one;
+    } else if (tr->k_single) {
+        const HelixMatmulTraits* ytr = nullptr;
+        pl = helix::rt::plan_ytile(ctx, pd, *tr, &ytr);
+        if (ytr) tr = ytr;
+    } else {
+        pl = helix::rt::plan_multipass(ctx, pd, *tr);
+    }
+    if (tr->k_single) {
+        out->one_launch = 1;
+        out->kernel_1pass = tr->k_single;
+        return HELIX_OK;
+    }
+    const HelixMatmulTraits& kt = helix::rt::no_copies(ctx, *tr);
+    out->copies = kt.bccopy ? 1 : 0;
+    out->run_len = kt.walk ? pl.run_len : 0;
+    out->runs_per_group = kt.walk ? (pl.chunks_per_group + pl.run_len - 1) / pl.run_len : 0;
+    out->kernel_a = kt.k_chunk_state;
+    out->kernel_b = helix::rt::fuse_b_on(ctx, *tr, pl) ? nullptr : kt.k_state_scan;
+    out->kernel_c = kt.k_chunk_out;
+    return HELIX_OK;
+}

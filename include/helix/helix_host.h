@@ -36,7 +36,7 @@ typedef struct {
     uint64_t total_bytes;       /* == helix_scan_scratch_size()                  */
     uint64_t s_local_bytes;     /* per-chunk states                              */
     uint64_t s_seg_bytes;       /* segment aggregates / segment initial states   */
-    int32_t  launches;          /* kernel launches per encode                    */
+    int32_t  launches;          /* kernel launches per encode of the plan        */
     int32_t  np;                /* d_state padding of the selected kernels       */
     const char* kernel_a;       /* code-object names of the Pass A, B and C      */
     const char* kernel_b;       /* kernels (static strings)                      */
@@ -44,8 +44,9 @@ typedef struct {
     const char* kernel_1pass;   /* the single-pass kernel, else NULL             */
     uint64_t bccopy_bytes;      /* bf16 copies of B and C Pass A writes for C    */
     uint64_t rec_bytes;         /* per-token decay records Pass A writes for C   */
-    int32_t  walk_len;          /* chunks per walking Pass C workgroup (a
-                                   multiple of seg_len; seg_len off the walk)    */
+    int32_t  walk_len;          /* the most chunks a walking Pass C workgroup
+                                   takes (a multiple of seg_len; seg_len off the
+                                   walk); helix_run_info has what it takes       */
     int32_t  walks_per_group;
     int32_t  pass_b;            /* where Pass B's segment scan runs: one of
                                    HELIX_PASS_B_* (kernel_b is NULL unless it
@@ -72,14 +73,33 @@ typedef struct {
 #define HELIX_PASS_B_LAUNCHED 0   /* kernel_b, between Pass A and Pass C         */
 #define HELIX_PASS_B_IN_C     1   /* the walking Pass C's prologue               */
 
-/* The plan of the passes. A scan of a few chunks is encoded as one launch of
- * the single pass instead, whatever its plan, where that is faster (scalar A,
- * d_state up to 128 or blocks of it, no tuning variable set); its scratch then
- * stays unused. Likewise a plan with bf16 copies of B and C up to d_state 128 (or
- * blocks of it) runs the same kernels without them, and bccopy_bytes stay unused. */
-/* Returns HELIX_ERR_UNSUPPORTED_SHAPE when the descriptor is declined. */
+/* The plan of the passes, which scratch is sized for; helix_scan_run_info says
+ * what of it is launched. Returns HELIX_ERR_UNSUPPORTED_SHAPE when the descriptor
+ * is declined. */
 helix_status helix_scan_plan_info(helix_ctx* ctx, const helix_scan_desc* d,
                                   helix_plan_info* out);
+
+/* What helix_scan_encode launches for `d`, per block of state indices, with a y
+ * that overlaps nothing else. A scan of a few chunks runs as one launch of the
+ * single pass, whatever its plan, where that is faster (scalar A, d_state up to
+ * 128 or blocks of it, no tuning variable set); its scratch stays unused. A plan
+ * with bf16 copies of B and C up to d_state 128 (or blocks of it) runs the same
+ * kernels without them, and bccopy_bytes stay unused (a y over B or C keeps the
+ * copies). */
+typedef struct {
+    int32_t  one_launch;        /* 1: kernel_1pass alone                         */
+    int32_t  copies;            /* 1: Pass A writes bf16 copies of B and C       */
+    int32_t  run_len;           /* chunks per workgroup of a walking Pass C: a
+                                   multiple of seg_len, at most walk_len; 0 off
+                                   the walk                                      */
+    int32_t  runs_per_group;    /* such runs per sequence and chunk group        */
+    const char* kernel_a;       /* NULL where not launched                       */
+    const char* kernel_b;
+    const char* kernel_c;
+    const char* kernel_1pass;
+} helix_run_info;
+
+helix_status helix_scan_run_info(helix_ctx* ctx, const helix_scan_desc* d, helix_run_info* out);
 
 /* Device pointers of one helix_scan_run call. */
 typedef struct {

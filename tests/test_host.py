@@ -646,6 +646,46 @@ def test_tiny_budget_forces_many_groups(host):
     assert tuned(HELIX_SCRATCH_MB=None).plan_info(mp(shape)).n_groups == 1
 
 
+def _runs(d):
+    """Everything helix_scan_run_info reports of a descriptor on an untuned host context."""
+    r = abi.Context(host_only=True).run_info(d)
+    return {k: getattr(r, k) for k, _ in r._fields_}
+
+
+@pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
+def test_run_info(host, backend):
+    # The plan's kernels and runs where the plan is what is launched ...
+    d, k = mp(CONFIG_SHAPES["cfg2"], backend), host.plan_info(mp(CONFIG_SHAPES["cfg2"], backend))
+    assert _runs(d) == {"one_launch": 0, "copies": 0, "run_len": 8, "runs_per_group": 16, "kernel_a": k.kernel_a,
+                        "kernel_b": k.kernel_b, "kernel_c": k.kernel_c, "kernel_1pass": None}
+    assert (k.walk_len, k.walks_per_group) == (16, 8)
+    # ... the kernels without copies on a plan with them, alone and in blocks of state indices ...
+    for shape in (CONFIG_SHAPES["cfg4a"], (4096, 1, 64, 64, 256, 8)):
+        d, k = mp(shape, backend), host.plan_info(mp(shape, backend))
+        r = host.run_info(d)
+        assert (k.bccopy_bytes > 0) == (backend == HELIX_BACKEND_MPP)
+        assert r.copies == 0 and b"_bc_" not in r.kernel_a + r.kernel_c
+        assert r.kernel_c == k.kernel_c.replace(b"_bc_", b"_") and r.run_len * r.runs_per_group >= k.n_chunks
+    # ... and the single pass where a short scan is one launch of it.
+    r = host.run_info(mp((67, 1, 64, 64, 128, 8), backend))
+    assert (r.one_launch, r.kernel_1pass, r.kernel_a, r.run_len) == (1, b"helix_scan_1pass_f32_n128", None, 0)
+    # A tuning variable keeps the plan.
+    c = tuned(HELIX_FUSE_B="0")
+    r = c.run_info(mp((67, 1, 64, 64, 128, 8), backend))
+    assert r.one_launch == 0 and r.kernel_b == b"helix_state_scan_f32"
+    r = c.run_info(mp(CONFIG_SHAPES["cfg4a"], backend))
+    assert r.copies == (backend == HELIX_BACKEND_MPP) and r.kernel_c == c.plan_info(mp(CONFIG_SHAPES["cfg4a"], backend)).kernel_c
+
+
+def test_run_info_single_pass(host):
+    d = desc_init(*CONFIG_SHAPES["cfg2"])
+    d.multipass = False
+    r = host.run_info(d)
+    assert (r.one_launch, r.kernel_c, r.run_len) == (0, b"helix_scan_walk_x6_y_n128", 8)
+    r = tuned(HELIX_1PASS_Y="0").run_info(d)
+    assert (r.one_launch, r.kernel_1pass, r.kernel_c) == (1, b"helix_scan_1pass_f32_n128", None)
+
+
 def test_scratch_zero_for_single_pass(host):
     d = mp(CONFIG_SHAPES["cfg1"])
     d.multipass = False
