@@ -683,7 +683,7 @@ void layout(const helix_tuning& tu, const helix_scan_desc& d, const HelixMatmulT
     pl->segs_per_group = (cpg + pl->seg_len - 1) / pl->seg_len;
     pl->walks_per_group = (cpg + pl->walk_len - 1) / pl->walk_len;
     pl->run_len = pl->walk_len;
-    if (tr.walk_hb) {
+    if (tr.walk_hb && tu.walk_len <= 0) {
         // The walk with HELIX_HB items per workgroup, one workgroup per CU, has
         // half the workgroups of the two-head walks that walk_len is chosen
         // for: the run of whole Pass A segments with the fewest chunk steps

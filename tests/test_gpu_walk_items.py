@@ -14,7 +14,7 @@ import torch
 from oracle import pyoracle as po
 from helix_amd.desc import HELIX_BACKEND_MPP, HELIX_BACKEND_SGMMA, HELIX_BF16, HELIX_F16, HELIX_OK, HELIX_TENSOR_NULL
 from gpu_harness import BF16_ABS, BF16_REL, F32_ABS, F32_REL, T, ctx_for, run
-from test_gpu_io import TORCH, U, rounded
+from test_gpu_io import TORCH, U, check, rounded, run_io
 
 pytestmark = pytest.mark.gpu
 
@@ -24,8 +24,8 @@ SHAPES = [
     ((333, 2, 2, 128, 128, 2), {}),                     # one head of two slabs
     ((449, 1, 6, 64, 64, 2), {}),                       # three items
     ((513, 1, 5, 72, 120, 1), {}),                      # ten items, an 8-channel last slab
-    ((1025, 1, 5, 64, 96, 1), {"HELIX_WALK_LEN": 8, "HELIX_SEG_LEN": 4}),   # five items, runs of 4 or 8, one token last
-    ((640, 1, 4, 64, 128, 1), {"HELIX_WALK_LEN": 3, "HELIX_SEG_LEN": 1}),   # runs of 1 to 3 over ten chunks
+    ((1025, 1, 5, 64, 96, 1), {"HELIX_WALK_LEN": 8, "HELIX_SEG_LEN": 4}),   # five items, runs of 8, one token last
+    ((640, 1, 4, 64, 128, 1), {"HELIX_WALK_LEN": 3, "HELIX_SEG_LEN": 1}),   # runs of 3 over ten chunks, the last of 1
     ((1500, 2, 3, 64, 128, 1), {"HELIX_SCRATCH_MB": 1}),                    # carried through several groups
 ]
 
@@ -39,6 +39,7 @@ def test_item_blocks(gpu, shape, knobs):
     d = p.d.copy()
     d.backend, d.multipass = HELIX_BACKEND_SGMMA, True
     assert b"helix_scan_walk_x6_n" in ctx.plan_info(d).kernel_c
+    assert ctx.run_info(d).run_len == knobs.get("HELIX_WALK_LEN", 1)
     _, y, s1 = run(ctx, p, d)
     assert po.allclose_ratio(y, y_ref, F32_REL, F32_ABS) <= 1.0
     assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
@@ -55,6 +56,7 @@ def test_item_blocks_bf16(gpu, shape, knobs, copies):
     d = p.d.copy()
     d.backend, d.multipass = HELIX_BACKEND_MPP, True
     assert (b"helix_scan_walk16_bf16_bc_n" if copies == "1" else b"helix_scan_walk16_bf16_n") in ctx.plan_info(d).kernel_c
+    assert ctx.run_info(d).run_len == knobs.get("HELIX_WALK_LEN", 1)
     _, y, s1 = run(ctx, p, d)
     assert po.allclose_ratio(y, y_ref, BF16_REL, BF16_ABS) <= 1.0
     assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
@@ -104,6 +106,47 @@ def test_16bit_storage(gpu, shape, pad, io):
         torch.cuda.synchronize()
         assert po.allclose_ratio(y.float().cpu().numpy(), y_ref, F32_REL + U[io], F32_ABS) <= 1.0, route
         assert po.allclose_ratio(s1.cpu().numpy(), s_ref, F32_REL, F32_ABS) <= 1.0, route
+
+
+# Pass A segments and walk runs of several chunks: state carried from chunk to
+# chunk in both, planes and records staged for a next chunk, runs of one and of
+# two segments, ragged last chunks of one token and of four.
+RUNS = [
+    ((1025, 1, 5, 72, 120, 1), {"HELIX_WALK_LEN": 6, "HELIX_SEG_LEN": 3}),
+    ((900, 2, 6, 64, 64, 2), {"HELIX_WALK_LEN": 4, "HELIX_SEG_LEN": 4}),
+]
+
+
+@pytest.mark.parametrize("io", [HELIX_BF16, HELIX_F16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("shape,knobs", RUNS, ids=["x".join(map(str, s)) for s, _ in RUNS])
+def test_16bit_storage_runs(gpu, shape, knobs, backend, io):
+    p = rounded(po.problem_harness(*shape, 617, "long"), io)
+    p.s0 = (np.random.default_rng(6).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
+    y_ref, s_ref = po.scan(p, use_ids=False)
+    ctx = ctx_for(gpu, **knobs)
+    d = p.d.copy()
+    d.io_dtype, d.backend, d.multipass = io, backend, True
+    assert ctx.run_info(d).run_len == knobs["HELIX_WALK_LEN"] and ctx.plan_info(d).seg_len == knobs["HELIX_SEG_LEN"]
+    desc, y, s1 = run_io(ctx, p, io, backend, True)
+    check(io, desc, y, s1, y_ref, s_ref)
+
+
+@pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("N", [136, 256])
+def test_state_block_runs(gpu, N, backend):
+    """The walk that adds into y, over runs of several chunks."""
+    p = po.problem_harness(1025, 1, 5, 72, N, 1, 618, "long")
+    p.s0 = (np.random.default_rng(6).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
+    y_ref, s_ref = po.scan(p, use_ids=False)
+    ctx = ctx_for(gpu, HELIX_WALK_LEN=6, HELIX_SEG_LEN=3, HELIX_F32_WALK="1")
+    d = p.d.copy()
+    d.backend, d.multipass = backend, True
+    assert ctx.plan_info(d).state_blocks == 2 and ctx.run_info(d).run_len == 6
+    _, y, s1 = run(ctx, p, d)
+    rel, ab = (BF16_REL, BF16_ABS) if backend == HELIX_BACKEND_MPP else (F32_REL, F32_ABS)
+    assert po.allclose_ratio(y, y_ref, rel, ab) <= 1.0
+    assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
 
 
 @pytest.mark.parametrize("io", [HELIX_BF16, HELIX_F16], ids=["bf16", "f16"])

@@ -677,6 +677,14 @@ def test_run_info(host, backend):
     assert r.copies == (backend == HELIX_BACKEND_MPP) and r.kernel_c == c.plan_info(mp(CONFIG_SHAPES["cfg4a"], backend)).kernel_c
 
 
+@pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("walk,seg", [(8, 4), (3, 1), (6, 6)])
+def test_walk_len_sets_the_runs(walk, seg, backend):
+    c = tuned(HELIX_WALK_LEN=walk, HELIX_SEG_LEN=seg, HELIX_F32_WALK="1")
+    r = c.run_info(mp((1025, 1, 5, 64, 96, 1), backend))
+    assert (r.run_len, r.runs_per_group) == (walk, -(-17 // walk))
+
+
 def test_run_info_single_pass(host):
     d = desc_init(*CONFIG_SHAPES["cfg2"])
     d.multipass = False
