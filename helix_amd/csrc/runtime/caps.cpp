@@ -341,7 +341,7 @@ helix_tuning tuning_from_env() {
     if (yt >= 0) t.ytile = yt > 0 ? 1 : 0;
     const int sb = env_switch("HELIX_STATE_BLOCKS");
     if (sb >= 0) t.state_blocks = sb > 0 ? 1 : 0;
-    for (const char* k : {"HELIX_SCRATCH_MB", "HELIX_PASSA_SPLIT", "HELIX_PASSA_F16", "HELIX_FUSE_B",
+    for (const char* k : {"HELIX_PASSA_SPLIT", "HELIX_PASSA_F16", "HELIX_FUSE_B",
                           "HELIX_WALK_BCCOPY", "HELIX_SEG_LEN", "HELIX_WALK_LEN", "HELIX_HBLK", "HELIX_F32_WALK",
                           "HELIX_1PASS_Y", "HELIX_STATE_BLOCKS"})
         if (std::getenv(k)) t.planned = false;

@@ -36,8 +36,9 @@ struct helix_tuning {
     int  f32_walk    = -1;     // HELIX_F32_WALK=0 / 1: the fp32 path's chunk-parallel Pass C / walk
                                // (on per-chunk states stored by Pass A) at d_state 128
     int  ytile       = -1;     // HELIX_1PASS_Y=0: the single pass in its one-launch form only
-    bool planned     = true;   // none of the overrides (this struct, FORCE_BACKEND aside) is set:
-                               // a short scan may run as one launch (one_launch_scan)
+    bool planned     = true;   // none of the measurement overrides (this struct, the scratch limit and
+                               // FORCE_BACKEND aside) is set: a short scan may run as one launch
+                               // (one_launch_scan), a plan with copies without them (no_copies)
     int  state_blocks = -1;    // HELIX_STATE_BLOCKS=0|1: d_state 129..256 (fp32 storage,
                                // scalar A) as blocks of at most 128 state indices, or not
 };

@@ -62,6 +62,10 @@ SHAPES = [
     (2048, 1, 8, 64, 128, 2, "L=2048 realistic prefill"),
 ]
 
+# A tuning variable at its default keeps the passes where a short scan would run
+# as one launch of the single pass.
+PASSES = {"HELIX_STATE_BLOCKS": "1"}
+
 MODES = [
     # (label, backend, scratch_mb, memory, extra environment, multipass)
     ("1pass", HELIX_BACKEND_AUTO, None, "short", {}, False),
@@ -71,9 +75,9 @@ MODES = [
     # in y, test_gpu_single_y.py).
     ("1pass/1launch/long", HELIX_BACKEND_AUTO, None, "long", {"HELIX_1PASS_Y": "0"}, False),
     ("fp32", HELIX_BACKEND_SGMMA, None, "short", {}, True),
-    ("fp32/sm", HELIX_BACKEND_SGMMA, 1, "short", {}, True),
+    ("fp32/sm", HELIX_BACKEND_SGMMA, 1, "short", PASSES, True),
     ("fp32/long", HELIX_BACKEND_SGMMA, None, "long", {}, True),
-    ("fp32/sm/long", HELIX_BACKEND_SGMMA, 1, "long", {}, True),
+    ("fp32/sm/long", HELIX_BACKEND_SGMMA, 1, "long", PASSES, True),
     # The fp32 path's chunk-parallel Pass C on per-chunk states stored by
     # Pass A, which d_state <= 128 replaces with the walk wherever the plan
     # walks more than one chunk.
@@ -87,9 +91,9 @@ MODES = [
     ("fp32/walk/sm", HELIX_BACKEND_SGMMA, 1, "short", {"HELIX_F32_WALK": "1"}, True),
     ("fp32/chunk/sm", HELIX_BACKEND_SGMMA, 1, "short", {"HELIX_F32_WALK": "0"}, True),
     ("bf16", HELIX_BACKEND_MPP, None, "short", {}, True),
-    ("bf16/sm", HELIX_BACKEND_MPP, 1, "short", {}, True),
+    ("bf16/sm", HELIX_BACKEND_MPP, 1, "short", PASSES, True),
     ("bf16/long", HELIX_BACKEND_MPP, None, "long", {}, True),
-    ("bf16/sm/long", HELIX_BACKEND_MPP, 1, "long", {}, True),
+    ("bf16/sm/long", HELIX_BACKEND_MPP, 1, "long", PASSES, True),
     # The walk with Pass B launched on its own, and with Pass B's segment scan
     # run in its prologue (by default: single-group plans of at most four
     # segments).

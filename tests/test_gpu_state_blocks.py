@@ -189,9 +189,10 @@ def test_blocks_up_to_256_copies_ids_and_groups(gpu, heads):
     p, d = _problem(shape, 5164)
     d.backend = HELIX_BACKEND_MPP
     p.ids = np.array([2, 0, 1], np.int32)
-    small = ctx_for(gpu, HELIX_SCRATCH_MB="1")
+    small = ctx_for(gpu, HELIX_SCRATCH_MB="1", HELIX_WALK_BCCOPY="1")
     info = small.plan_info(d)
     assert info.state_blocks == 2 and info.n_groups > 1 and info.bccopy_bytes > 0
+    assert small.run_info(d).copies == 1
     y_ref, s_ref = po.scan(p, use_ids=True, threads=0)
     _, y, s1 = run(small, p, desc=d, use_ids=True)
     ry = po.allclose_ratio(y, y_ref, BF16_REL, BF16_ABS)

@@ -669,6 +669,10 @@ def test_run_info(host, backend):
     # ... and the single pass where a short scan is one launch of it.
     r = host.run_info(mp((67, 1, 64, 64, 128, 8), backend))
     assert (r.one_launch, r.kernel_1pass, r.kernel_a, r.run_len) == (1, b"helix_scan_1pass_f32_n128", None, 0)
+    # A scratch limit changes neither.
+    c = tuned(HELIX_SCRATCH_MB="64")
+    assert c.run_info(mp((67, 1, 64, 64, 128, 8), backend)).one_launch == 1
+    assert c.run_info(mp(CONFIG_SHAPES["cfg4a"], backend)).copies == 0
     # A tuning variable keeps the plan.
     c = tuned(HELIX_FUSE_B="0")
     r = c.run_info(mp((67, 1, 64, 64, 128, 8), backend))
