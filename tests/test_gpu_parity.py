@@ -60,6 +60,10 @@ SHAPES = [
     (256, 4, 4, 64, 128, 1, "n_seq=4 batched"),
     (1024, 1, 2, 64, 128, 1, "L=1024 sixteen chunks"),
     (2048, 1, 8, 64, 128, 2, "L=2048 realistic prefill"),
+    # Past the lengths that run as one launch of the single pass by default.
+    (700, 2, 6, 72, 96, 2, "L=700 head_dim=72 d_state=96"),
+    (513, 1, 16, 64, 64, 1, "L=513 d_state=64 sixteen heads"),
+    (520, 1, 4, 64, 256, 2, "L=520 d_state=256"),
 ]
 
 # A tuning variable at its default keeps the passes where a short scan would run
@@ -140,6 +144,8 @@ def test_shape_matrix(gpu, shape, mode):
     assert ctx.supported(d), ctx.backend_desc(d)
     is_bf16 = ctx.select_backend(d) == HELIX_BACKEND_MPP
     s_rel, s_abs = s1_tolerance(ctx, d)
+    if multipass and shape[0] > 400:
+        assert ctx.run_info(d).one_launch == 0
     if scratch_mb:
         assert not multipass or ctx.plan_info(d).n_groups > 1 or shape[0] <= 256
     _, y, s1 = run(ctx, p, desc=d)

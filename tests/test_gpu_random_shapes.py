@@ -27,11 +27,13 @@ pytestmark = pytest.mark.gpu
 BUDGET = 1.5e8   # L * S * H * P * N per case
 
 
-def _shapes(n: int, seed: int):
+def _shapes(n: int, seed: int, shortest: int = 1):
     rng = np.random.default_rng(seed)
     out = []
     while len(out) < n:
         L = int(rng.choice([int(rng.integers(1, 130)), int(rng.integers(130, 1500))]))
+        if L < shortest:
+            continue
         S = int(rng.integers(1, 4))
         G = int(rng.choice([1, 2, 4]))
         H = G * int(rng.integers(1, 13))
@@ -43,7 +45,10 @@ def _shapes(n: int, seed: int):
     return out
 
 
-CASES = _shapes(24, 20261202)
+# Half of the first cases are short enough to run as one launch of the single
+# pass by default; none of the others is.
+PASSES_FROM = 500
+CASES = _shapes(24, 20261202) + _shapes(12, 20261204, PASSES_FROM)
 PATHS = [("bf16", HELIX_BACKEND_MPP, True), ("fp32", HELIX_BACKEND_SGMMA, True), ("single", HELIX_BACKEND_AUTO, False)]
 
 
@@ -58,6 +63,7 @@ def test_random_shape(gpu, case, path):
     d.multipass = multipass
     d.backend = backend
     assert gpu.supported(d), gpu.backend_desc(d)
+    assert not (multipass and L >= PASSES_FROM and gpu.run_info(d).one_launch)
     y_ref, s_ref = po.scan(p, threads=0)
     _, y, s1 = run(gpu, p, desc=d)
     rel, ab = (BF16_REL, BF16_ABS) if label == "bf16" else (F32_REL, F32_ABS)

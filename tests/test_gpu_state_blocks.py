@@ -201,12 +201,16 @@ def test_blocks_up_to_256_copies_ids_and_groups(gpu, heads):
     assert ry <= 1.0 and rs <= 1.0, (ry, rs)
 
 
-def test_blocks_up_to_256_noalloc(gpu):
-    # The bf16 path's blocks, copies included, in the library's fixed scratch.
+@pytest.mark.parametrize("copies", [False, True], ids=["rows", "copies"])
+def test_blocks_up_to_256_noalloc(gpu, copies):
+    # The bf16 path's blocks in the library's fixed scratch, with room for the
+    # copies that the default leaves unused, and with the copies.
     shape = (700, 2, 4, 64, 256, 2, "noalloc, N=256")
     p, d = _problem(shape, 5165)
     d.backend = HELIX_BACKEND_MPP
-    assert gpu.plan_info(d).bccopy_bytes > 0
+    if copies:
+        gpu = ctx_for(gpu, HELIX_WALK_BCCOPY="1")
+    assert gpu.plan_info(d).bccopy_bytes > 0 and gpu.run_info(d).copies == copies and not gpu.run_info(d).one_launch
     y_ref, s_ref = po.scan(p, threads=0)
     dev = {k: upload(getattr(p, k)) for k in ("s0", "x", "dt", "A", "B", "C")}
     y = torch.full(p.y_shape(), float("nan"), device="cuda")
