@@ -462,10 +462,11 @@ const HelixMatmulTraits* short_scan_traits(const helix_ctx* ctx, const helix_sca
 }
 
 // The walk's prologue loads up to segs_per_group segment aggregates per
-// workgroup, four at a time; past four segments the second round of loads
-// costs more than Pass B's own launch (config 2, 8 segments: 149 vs 142 us;
-// configs 4a/4b, 4 segments, fused against launched: 624 vs 635 and 668 vs
-// 681 us).
+// workgroup, two at a time. Past four segments that cost more than Pass B's own
+// launch in the walk of two heads per workgroup, four aggregates in flight
+// (config 2, 8 segments: 149 vs 142 us; configs 4a/4b, 4 segments, fused against
+// launched: 624 vs 635 and 668 vs 681 us); not measured again on the walk of
+// HELIX_HB items.
 constexpr int kFuseBMaxSegs = 4;
 
 bool fuse_b_on(const helix_ctx* ctx, const HelixMatmulTraits& tr, const MultipassPlan& plan) {
@@ -479,7 +480,8 @@ bool fuse_b_on(const helix_ctx* ctx, const HelixMatmulTraits& tr, const Multipas
 
 namespace {
 
-// Chunks per walk segment for a group of `cpg` chunks (the walking Pass C;
+// Chunks per walk segment for a group of `cpg` chunks (the walking Pass C, which
+// layout() cuts into shorter runs where it takes HELIX_HB items per workgroup;
 // also Pass A's segment on the per-item kernels): enough segments that there
 // are ~kTargetWgA (seq, head, P slab) items x segments, and no more (a longer
 // walk keeps more of the chunk recurrence in registers and shortens Pass B), up
@@ -514,9 +516,10 @@ int choose_walk_len(const helix_scan_desc& d, int cpg) {
 // one chunk step per lat + k * load microseconds, load being the running
 // workgroups over the chip (each weighted by the share of its heads or items
 // that are real). lat and k, and a fixed cost per workgroup (o, plus g per
-// segment aggregate a walk's prologue folds in), were fitted to Pass A and the
-// bf16 walk timed at 19 lengths on S=8 L=4096 H=80 P=64 and H=27 P=192 (N=128):
-// rms errors 1.8 and 2.0 %. Without the per-engine round robin the Pass A fit
+// segment aggregate a walk's prologue folds in), were fitted to Pass A and to the
+// bf16 path's walk of two heads per workgroup (since replaced up to d_state 128)
+// timed at 19 lengths on S=8 L=4096 H=80 P=64 and H=27 P=192 (N=128): rms errors
+// 1.8 and 2.0 %. Without the per-engine round robin the Pass A fit
 // misses by up to 17 %: at H=27 and two segments, one engine in each XCD got
 // six long and five short workgroups, ran three shorts in a row, and Pass A
 // took the time of one 64-chunk segment.
@@ -524,6 +527,9 @@ struct DispatchCost {
     double lat, k, o, g;
 };
 constexpr DispatchCost kCostA{3.0, 0.009, 2.0, 0.0};
+// The two-head walk, which also prices the bf16 path's walk of HELIX_HB items:
+// about twice its workgroups on half the items each. The lengths it picks were
+// compared on the two-head walk only.
 constexpr DispatchCost kCostWalk{2.25, 0.007, 0.5, 0.5};
 // The fp32 path's walk of HELIX_HB items: 13.5 us a chunk step over the whole
 // chip at L=8192 H=64 P=64 N=128 G=8 (256 workgroups), with the bf16 walk's
@@ -575,7 +581,8 @@ double fused_lengths_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, i
                     wg.emplace_back(seg_steps(s) + kCostA.o,
                                     (double)std::min(HELIX_HB, ipg - HELIX_HB * ib) / HELIX_HB);
     const double a = dispatch_us(wg, kCostA);
-    // Walk: (item block, group, walk, sequence), or (head block, group, slab, walk, sequence).
+    // The fp32 path's walk: (item block, group, walk, sequence). The bf16 path's is
+    // priced as (head block, group, slab, walk, sequence), kCostWalk's grid.
     if (tr.walk_hb && !tr.bf16_state) {
         for (size_t i = 0, n = wg.size(); i < n; ++i) {
             const int s = (int)(i / ((size_t)nib * d.n_group) % nseg);

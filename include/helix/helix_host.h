@@ -139,8 +139,9 @@ helix_status helix_scan_run(helix_ctx* ctx, void* stream, const helix_scan_desc*
  * scan whose plan under the context's budget needs more scratch is cut into
  * more super-chunk groups (carried through s1, as with a lower
  * HELIX_SCRATCH_MB), and only a scan that does not fit at one chunk per group
- * returns HELIX_ERR_SCRATCH_TOO_SMALL, before anything is enqueued; the
- * single pass needs none. No part of the array needs to start at zero: every
+ * returns HELIX_ERR_SCRATCH_TOO_SMALL, before anything is enqueued (with 16-bit
+ * storage on the fp32 path it runs as the single pass); the single pass needs
+ * none. No part of the array needs to start at zero: every
  * region a kernel reads is written earlier in the same encode.
  *
  * Every call on one GPU shares that GPU's array and it keeps the last call's
