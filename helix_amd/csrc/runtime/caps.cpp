@@ -507,130 +507,164 @@ int choose_walk_len(const helix_scan_desc& d, int cpg) {
     return (int)std::max<long>(1, std::min<long>(len, cpg));
 }
 
-// Dispatch model of a one-workgroup-per-CU launch on MI355X, used to pick
-// the walk length when every walk's start state comes from the walk's own
-// prologue (fused Pass B). Workgroup b runs on XCD b % 8 (the kernels decode
-// their logical id with xcd_logical_id); in each XCD, four shader engines of
-// eight CUs take the XCD's workgroups round-robin, in dispatch order, and a
-// workgroup waits for a CU of its own engine. Every running workgroup moves
-// one chunk step per lat + k * load microseconds, load being the running
-// workgroups over the chip (each weighted by the share of its heads or items
-// that are real). lat and k, and a fixed cost per workgroup (o, plus g per
-// segment aggregate a walk's prologue folds in), were fitted to Pass A and to the
-// bf16 path's walk of two heads per workgroup (since replaced up to d_state 128)
-// timed at 19 lengths on S=8 L=4096 H=80 P=64 and H=27 P=192 (N=128): rms errors
-// 1.8 and 2.0 %. Without the per-engine round robin the Pass A fit
-// misses by up to 17 %: at H=27 and two segments, one engine in each XCD got
-// six long and five short workgroups, ran three shorts in a row, and Pass A
-// took the time of one 64-chunk segment.
+// Dispatch model of Pass A and the walk on HELIX_HB items, one workgroup per CU on
+// MI355X. Workgroup b runs on XCD b % 8 (the kernels decode their logical id with
+// xcd_logical_id); in each XCD, four shader engines of eight CUs take the XCD's
+// workgroups round-robin, in dispatch order, and a workgroup waits for a CU of
+// its own engine. Every running workgroup moves one chunk step per lat + k * load
+// microseconds, load being the running workgroups over the chip (each weighted by
+// the share of its items that are real); o is a fixed cost per workgroup and g
+// one per segment aggregate that a walk's prologue folds in, in chunk steps.
 struct DispatchCost {
     double lat, k, o, g;
 };
-constexpr DispatchCost kCostA{3.0, 0.009, 2.0, 0.0};
-// The two-head walk, which also prices the bf16 path's walk of HELIX_HB items:
-// about twice its workgroups on half the items each. The lengths it picks were
-// compared on the two-head walk only.
-constexpr DispatchCost kCostWalk{2.25, 0.007, 0.5, 0.5};
-// The fp32 path's walk of HELIX_HB items: 13.5 us a chunk step over the whole
-// chip at L=8192 H=64 P=64 N=128 G=8 (256 workgroups), with the bf16 walk's
-// proportions.
-constexpr DispatchCost kCostWalkHb{7.5, 0.0235, 0.5, 0.5};
+struct PlanCost {
+    DispatchCost a, c;
+};
+// lat, k and o fitted to each pass timed alone at up to fourteen lengths on
+// thirteen shapes (600 to 8192 tokens, 1 to 8 sequences of 16 to 96 heads, some of
+// several slabs), inputs out of the Infinity Cache: rms errors 4-6 % each, no
+// sign of a bias in length. By kernels: d_state up to 64, up to 128.
+constexpr double kFoldG = 0.4;
+constexpr PlanCost kCostBf16F32[2]  = {{{2.22, 0.00354, 1.5, 0}, {4.15, 0.0101, 0.5, kFoldG}},
+                                       {{2.69, 0.00426, 2.0, 0}, {4.55, 0.0114, 0.75, kFoldG}}};
+constexpr PlanCost kCostBf16Io16[2] = {{{2.27, 0.00112, 1.5, 0}, {4.27, 0.00357, 0.75, kFoldG}},
+                                       {{2.46, 0.00092, 3.0, 0}, {4.79, 0.00468, 1.0, kFoldG}}};
+constexpr PlanCost kCostF32[2]      = {{{2.32, 0.00373, 1.5, 0}, {8.77, 0.0109, 0.25, kFoldG}},
+                                       {{3.45, 0.00417, 2.0, 0}, {11.6, 0.0166, 0.25, kFoldG}}};
+constexpr PlanCost kCostF32Bf16[2]  = {{{2.14, 0.00106, 1.5, 0}, {7.23, 0.00304, 0.5, kFoldG}},
+                                       {{2.36, 0.00102, 3.0, 0}, {8.62, 0.00474, 0.75, kFoldG}}};
+constexpr PlanCost kCostF32F16[2]   = {{{2.20, 0.0015, 1.5, 0}, {8.0, 0.0045, 0.5, kFoldG}},
+                                       {{2.90, 0.00283, 2.0, 0}, {10.8, 0.00735, 0.5, kFoldG}}};
+constexpr PlanCost kCostY[2]        = {{{2.29, 0.00328, 2.0, 0}, {9.04, 0.00986, 0.5, 0}},
+                                       {{3.42, 0.00488, 2.0, 0}, {12.0, 0.0148, 0.5, 0}}};
 constexpr int kXcds = 8, kEnginesPerXcd = 4, kCusPerEngine = 8;
+constexpr long kCus = kXcds * kEnginesPerXcd * kCusPerEngine;
 
-// Microseconds for workgroups given in logical-id order as (chunk steps,
-// weight). Every running workgroup advances at the same rate, so each
-// engine's queue is list-scheduled at unit speed (the order of events does not
-// depend on the rate) to the makespan T in chunk steps; the chip is busy
-// throughout, and the integral of lat + k * load over T is
-// lat * T + k * sum(weight * steps).
-double dispatch_us(const std::vector<std::pair<double, double>>& wg, const DispatchCost& c) {
-    const size_t n = wg.size();
-    const size_t per = n / kXcds;
+const PlanCost& plan_cost(const helix_scan_desc& d, const HelixMatmulTraits& tr) {
+    const int n = tr.np > 64 ? 1 : 0;
+    if (tr.bf16_state) return d.io_dtype == HELIX_F32 ? kCostBf16F32[n] : kCostBf16Io16[n];
+    if (tr.rec_kind == 0) return kCostY[n];   // state tiles in y
+    return d.io_dtype == HELIX_F32 ? kCostF32[n] : d.io_dtype == HELIX_BF16 ? kCostF32Bf16[n] : kCostF32F16[n];
+}
+
+// The workgroups of either launch over a group of cpg chunks in runs of len, in
+// their kernels' logical order (item block, group, run, sequence).
+struct PlanGrid {
+    long per_run;    // item blocks x groups
+    int  nib, cpg, len, n_run, n_seq;
+    double last;     // share of the last item block's items that are real
+
+    PlanGrid(const helix_scan_desc& d, int cpg_, int len_) : cpg(cpg_), len(len_) {
+        const int ipg = d.n_head / d.n_group * ((d.head_dim + HELIX_HD - 1) / HELIX_HD);
+        nib = (ipg + HELIX_HB - 1) / HELIX_HB;
+        per_run = (long)nib * d.n_group;
+        n_run = (cpg + len - 1) / len;
+        n_seq = d.n_seq;
+        last = (double)(ipg - HELIX_HB * (nib - 1)) / HELIX_HB;
+    }
+    long total() const { return per_run * n_run * n_seq; }
+    int run_of(long wid) const { return (int)(wid / per_run % n_run); }
+    double steps(int r, const DispatchCost& c, bool fold) const {
+        return std::min(len, cpg - r * len) + c.o + (fold ? c.g * r : 0.0);
+    }
+    // The chunk steps of every workgroup, weighted.
+    double work(const DispatchCost& c, bool fold) const {
+        const double w = (double)per_run / nib * (nib - 1 + last);
+        return w * n_seq * (cpg + n_run * c.o + (fold ? c.g * 0.5 * n_run * (n_run - 1) : 0.0));
+    }
+    // No schedule is shorter than its longest workgroup, or than all of them spread evenly.
+    double makespan_bound(const DispatchCost& c, bool fold) const {
+        const double longest = std::max(steps(0, c, fold), steps(n_run - 1, c, fold));
+        return std::max(longest, (cpg + n_run * c.o) * per_run * n_seq / kCus);
+    }
+};
+
+// Makespan in chunk steps. Every running workgroup advances at the same rate, so
+// each engine's queue is list-scheduled at unit speed (the order of events does
+// not depend on the rate). Past 64 rounds of workgroups how the last one falls is
+// a small part of the time.
+double makespan(const PlanGrid& g, const DispatchCost& c, bool fold) {
+    const long n = g.total();
+    if (n > 64 * kCus) return g.makespan_bound(c, fold) + 0.5 * g.len;
+    const long per = n / kXcds;
     double cu[kXcds * kEnginesPerXcd][kCusPerEngine] = {};
-    double T = 0.0, work = 0.0;
-    for (size_t b = 0; b < n; ++b) {
-        const size_t x = b % kXcds, j = b / kXcds;
-        const size_t wid = b < per * kXcds ? x * per + j : b;
+    double T = 0.0;
+    for (long b = 0; b < n; ++b) {
+        const long x = b % kXcds, j = b / kXcds;
+        const long wid = b < per * kXcds ? x * per + j : b;
         double* e = cu[x * kEnginesPerXcd + j % kEnginesPerXcd];
         int m = 0;
         for (int i = 1; i < kCusPerEngine; ++i)
             if (e[i] < e[m]) m = i;
-        e[m] += wg[wid].first;
+        e[m] += g.steps(g.run_of(wid), c, fold);
         T = std::max(T, e[m]);
-        work += wg[wid].first * wg[wid].second;
     }
-    return c.lat * T + c.k * work;
+    return T;
 }
 
-// Pass A (head-block kernel) and the walk with segments = walks of `len`
-// chunks over a single group of `cpg` chunks: the workgroups of both launches
-// in their kernels' logical order, priced by dispatch_us.
-double fused_lengths_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, int len) {
-    const int nseg = (cpg + len - 1) / len;
-    const int nslab = (d.head_dim + HELIX_HD - 1) / HELIX_HD;
-    const int hpg = d.n_head / d.n_group;
-    auto seg_steps = [&](int s) { return (double)std::min(len, cpg - s * len); };
-    std::vector<std::pair<double, double>> wg;
-    // Pass A: (item block, group, segment, sequence), item = (head, P slab).
-    const int ipg = hpg * nslab, nib = (ipg + HELIX_HB - 1) / HELIX_HB;
-    wg.reserve((size_t)d.n_seq * nseg * d.n_group * nib);
-    for (int seq = 0; seq < d.n_seq; ++seq)
-        for (int s = 0; s < nseg; ++s)
-            for (int g = 0; g < d.n_group; ++g)
-                for (int ib = 0; ib < nib; ++ib)
-                    wg.emplace_back(seg_steps(s) + kCostA.o,
-                                    (double)std::min(HELIX_HB, ipg - HELIX_HB * ib) / HELIX_HB);
-    const double a = dispatch_us(wg, kCostA);
-    // The fp32 path's walk: (item block, group, walk, sequence). The bf16 path's is
-    // priced as (head block, group, slab, walk, sequence), kCostWalk's grid.
-    if (tr.walk_hb && !tr.bf16_state) {
-        for (size_t i = 0, n = wg.size(); i < n; ++i) {
-            const int s = (int)(i / ((size_t)nib * d.n_group) % nseg);
-            wg[i].first += kCostWalkHb.o - kCostA.o + kCostWalkHb.g * s;
-        }
-        return a + dispatch_us(wg, kCostWalkHb);
-    }
-    const int hpw = tr.walk_hpw ? tr.walk_hpw : HELIX_WALK_HPW(tr.np);
-    const int npair = (hpg + hpw - 1) / hpw;
-    wg.clear();
-    for (int seq = 0; seq < d.n_seq; ++seq)
-        for (int s = 0; s < nseg; ++s)
-            for (int sl = 0; sl < nslab; ++sl)
-                for (int g = 0; g < d.n_group; ++g)
-                    for (int pr = 0; pr < npair; ++pr)
-                        wg.emplace_back(seg_steps(s) + kCostWalk.o + kCostWalk.g * s,
-                                        (double)std::min(hpw, hpg - hpw * pr) / hpw);
-    return a + dispatch_us(wg, kCostWalk);
+// Microseconds of a group of cpg chunks in segments = runs of len chunks. The
+// chip is busy throughout, so the integral of lat + k * load over a launch is
+// lat * T + k * work. A launch of Pass B reads every segment's aggregate and
+// writes every run's start state and s1 (fitted to whole scans less the other
+// two passes). bound: with the makespans' lower bounds instead.
+double plan_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, int len, bool fold, bool bound) {
+    const PlanCost& pc = plan_cost(d, tr);
+    const PlanGrid g(d, cpg, len);
+    const double mb = 1e-6 * d.n_seq * d.n_head * ((d.head_dim + HELIX_HD - 1) / HELIX_HD) * 64.0 * tr.np * sizeof(float);
+    double us = fold ? 0.0 : 2.0 + mb * (0.34 * g.n_run + 0.15);
+    us += pc.a.k * g.work(pc.a, false) + pc.c.k * g.work(pc.c, fold);
+    us += pc.a.lat * (bound ? g.makespan_bound(pc.a, false) : makespan(g, pc.a, false));
+    us += pc.c.lat * (bound ? g.makespan_bound(pc.c, fold) : makespan(g, pc.c, fold));
+    return us;
 }
 
-// The walk length (= Pass A's segment) with the least modelled time among
-// those of at most kFuseBMaxSegs walks, from `shortest` up. Memoized: the
-// plan is remade on every encode.
-int fused_walk_len(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, int shortest) {
-    // Past 64 rounds of one-workgroup-per-CU walks, how the last round falls
-    // is a small part of the time, and pricing every length would make the
-    // first plan of a large batch slow: keep the default length.
-    const long hpg = d.n_head / d.n_group;
-    const long hpw = tr.walk_hpw ? tr.walk_hpw : HELIX_WALK_HPW(tr.np);
-    const long walk_wg = (long)d.n_seq * d.n_group * ((hpg + hpw - 1) / hpw) *
-                         ((d.head_dim + HELIX_HD - 1) / HELIX_HD) * ((cpg + shortest - 1) / shortest);
-    if (walk_wg > 64L * kXcds * kEnginesPerXcd * kCusPerEngine) return shortest;
-    using Key = std::tuple<int, int, int, int, int, int, int, int>;
+// The chunks per Pass A segment and walk run with the least modelled time, and that
+// time, over a group of cpg chunks. fold: whether the plan may fold Pass B into the
+// walk where there are few enough segments. len: this length and no other
+// (0: any). Memoized: the plan is remade on every encode.
+//
+// Against every length timed on 36 shapes over both paths, all storage types and
+// the form without scratch, the choice was within 0.3 % of the best on average
+// (4 % at most). The lengths that the walk of two heads per workgroup had were
+// 23 % off (4 x 1392 tokens of 64 heads of 80, bf16 storage: runs of 22 and 194 us
+// against 11 and 117; 7059 tokens of 32 heads: 108 us against 68).
+struct PlanChoice {
+    int len;
+    double us;
+};
+bool folds(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, int len) {
+    // A one-chunk run on the fp32 path with fp32 storage keeps Pass B's launch:
+    // the plan of a walk there has walk_len > 1.
+    return tr.walk_fuse_b && (cpg + len - 1) / len <= kFuseBMaxSegs &&
+           (len > 1 || tr.bf16_state || d.io_dtype != HELIX_F32);
+}
+PlanChoice best_plan(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, bool fold, int len) {
+    using Key = std::tuple<const PlanCost*, int, int, int, int, int, bool, int>;
     static std::mutex mu;
-    static std::map<Key, int> memo;
-    const Key key{d.n_seq, d.n_head, d.head_dim, d.n_group, tr.np, tr.bf16_state ? tr.walk_hpw : -1, cpg, shortest};
+    static std::map<Key, PlanChoice> memo;
+    const Key key{&plan_cost(d, tr), d.n_seq, d.n_head, d.head_dim, d.n_group, cpg, fold, len};
     {
         std::lock_guard<std::mutex> lk(mu);
         const auto it = memo.find(key);
         if (it != memo.end()) return it->second;
     }
-    int best = shortest;
-    double best_us = fused_lengths_us(d, tr, cpg, shortest);
-    for (int len = shortest + 1; len <= cpg; ++len) {
-        const double us = fused_lengths_us(d, tr, cpg, len);
-        if (us < best_us) {
-            best_us = us;
-            best = len;
+    auto us = [&](int l, bool bound) { return plan_us(d, tr, cpg, l, fold && folds(d, tr, cpg, l), bound); };
+    PlanChoice best{len, 0.0};
+    if (len > 0) {
+        best.us = us(len, false);
+    } else {
+        // Lengths up to 96 chunks, and the cuts into up to sixteen, by their
+        // lower bounds: few need their schedule.
+        std::vector<std::pair<double, int>> cand;
+        for (int l = 1; l <= std::min(cpg, 96); ++l) cand.emplace_back(us(l, true), l);
+        for (int j = 1; j <= 16; ++j)
+            if ((cpg + j - 1) / j > 96) cand.emplace_back(us((cpg + j - 1) / j, true), (cpg + j - 1) / j);
+        std::sort(cand.begin(), cand.end());
+        for (const auto& [lower, l] : cand) {
+            if (best.len && lower >= best.us) break;
+            const double t = us(l, false);
+            if (!best.len || t < best.us) best = {l, t};
         }
     }
     std::lock_guard<std::mutex> lk(mu);
@@ -639,11 +673,13 @@ int fused_walk_len(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cp
     return best;
 }
 
-// Pass A's segment (seg_len) and the walk's (walk_len, a multiple of it). The
-// head-block Pass A takes the longest divisor of walk_len that still gives
-// ~kTargetWgHb workgroups, so its segments nest in the walk's. HELIX_WALK_LEN
-// sets walk_len, HELIX_SEG_LEN sets seg_len, and walk_len is then rounded to a
-// multiple of it.
+// Pass A's segment (seg_len) and the walk's (walk_len, a multiple of it). On the
+// kernels of HELIX_HB items segments and runs are best_plan's length; walk_len stays
+// a bound of two segments or choose_walk_len's, whichever is longer, where the walk
+// does not fold Pass B in (HELIX_SEG_LEN and HELIX_WALK_LEN nest runs of several
+// segments). The chunk-parallel plan's Pass A takes the longest divisor of
+// walk_len that still gives ~kTargetWgHb workgroups. HELIX_WALK_LEN sets walk_len,
+// HELIX_SEG_LEN sets seg_len, and walk_len is then rounded to a multiple of it.
 void choose_lengths(const helix_tuning& tu, const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg,
                     int* seg_len, int* walk_len) {
     int w = tu.walk_len > 0 ? std::min(tu.walk_len, cpg) : choose_walk_len(d, cpg);
@@ -651,6 +687,14 @@ void choose_lengths(const helix_tuning& tu, const helix_scan_desc& d, const Heli
     if (tu.seg_len > 0) {
         a = std::min(tu.seg_len, cpg);
         w = std::max(a, (w / a) * a);
+    } else if (tr.walk_hb && tu.walk_len <= 0) {
+        const int n_chunks = (d.n_tok + HELIX_CS - 1) / HELIX_CS;
+        const bool fold = tu.fuse_b != 0 && cpg == n_chunks;
+        a = best_plan(d, tr, cpg, fold, 0).len;
+        if (fold && folds(d, tr, cpg, a))
+            w = a;
+        else
+            w = w > 1 ? std::max(2 * a, (w / a) * a) : a;
     } else if (tr.a_hb) {
         const long per_seg = item_blocks(d);
         a = 1;
@@ -661,17 +705,6 @@ void choose_lengths(const helix_tuning& tu, const helix_scan_desc& d, const Heli
                 break;
             }
         }
-        // Walks that are Pass A's segments, few enough for the walk's prologue
-        // to fold them in (fused Pass B), over a single group: a longer walk
-        // may balance the one-workgroup-per-CU launches better. At S=8 L=4096
-        // N=128 the model takes 43-chunk walks at H=80 P=64 and 22 at H=27
-        // P=192, in place of 16: whole scans 605 -> 556 and 649 -> 588 us; on
-        // seven other shapes of 2048-4096 tokens x 4-16 sequences it was 21-78
-        // us faster on the bf16 path and no slower on the fp32 one.
-        const int n_chunks = (d.n_tok + HELIX_CS - 1) / HELIX_CS;
-        if (a == w && tu.walk_len <= 0 && tu.fuse_b != 0 && tr.walk && tr.walk_fuse_b && cpg == n_chunks &&
-            (cpg + w - 1) / w <= kFuseBMaxSegs)
-            a = w = fused_walk_len(d, tr, cpg, w);
     }
     if (!tr.walk) w = a;
     *seg_len = a;
@@ -689,25 +722,7 @@ void layout(const helix_tuning& tu, const helix_scan_desc& d, const HelixMatmulT
     choose_lengths(tu, d, tr, cpg, &pl->seg_len, &pl->walk_len);
     pl->segs_per_group = (cpg + pl->seg_len - 1) / pl->seg_len;
     pl->walks_per_group = (cpg + pl->walk_len - 1) / pl->walk_len;
-    pl->run_len = pl->walk_len;
-    if (tr.walk_hb && tu.walk_len <= 0) {
-        // The walk with HELIX_HB items per workgroup, one workgroup per CU, has
-        // half the workgroups of the two-head walks that walk_len is chosen
-        // for: the run of whole Pass A segments with the fewest chunk steps
-        // over its rounds of workgroups, each costing about 0.6 of a step more
-        // (its start state and first loads). At 24 heads x 2 x 1500 tokens
-        // runs of 1, 2 and 3 chunks are 288, 144 and 96 workgroups.
-        const long wg = item_blocks(d);
-        double best = 0.0;
-        for (int run = pl->seg_len; run <= pl->walk_len; run += pl->seg_len) {
-            const long rounds = (wg * ((cpg + run - 1) / run) + kTargetWgHb - 1) / kTargetWgHb;
-            const double cost = (double)rounds * (run + 0.6);
-            if (run == pl->seg_len || cost <= best) {
-                best = cost;
-                pl->run_len = run;
-            }
-        }
-    }
+    pl->run_len = tr.walk_hb && tu.walk_len <= 0 ? pl->seg_len : pl->walk_len;
     pl->sl_elem_bytes = bf16_state ? 2 : 4;
     pl->sl_elems = (pl->seg_len > 1 && !walk) ? state * (size_t)cpg : 0;
     pl->sg_elems = state * (size_t)pl->segs_per_group;
@@ -813,6 +828,7 @@ MultipassPlan plan_ytile(const helix_ctx* ctx, const helix_scan_desc& d, const H
         if (t2.seg_len <= 0) return pl = MultipassPlan{}, pl;
         layout(t2, d, tr, (int)n_chunks, &pl);
         if (!fits(pl.seg_len)) return pl = MultipassPlan{}, pl;
+        if (tu.walk_len <= 0) pl.run_len = pl.seg_len;
     }
     pl.n_chunks = (int)n_chunks;
     pl.n_groups = 1;

@@ -146,7 +146,7 @@ struct MultipassPlan {
     int    walk_len         = 0;   // chunks per walking Pass C segment (multiple of seg_len)
     int    walks_per_group  = 0;
     int    run_len          = 0;   // chunks per workgroup of the walking Pass C: walk_len, or with walk_hb and no
-                                   // HELIX_WALK_LEN the part of it (whole Pass A segments) that still fills the chip
+                                   // HELIX_WALK_LEN seg_len
     int    hblk             = 0;
     int    n_hblk           = 0;
     size_t sl_elems         = 0;   // s_local elements (0 when seg_len == 1)

@@ -689,6 +689,49 @@ def test_walk_len_sets_the_runs(walk, seg, backend):
     assert (r.run_len, r.runs_per_group) == (walk, -(-17 // walk))
 
 
+# Shapes whose runs the costs of the earlier two-head walk made too long or too
+# short: (shape, backend, io, chunks per segment and run).
+PLANS = [
+    ((1392, 4, 64, 80, 128, 1), HELIX_BACKEND_AUTO, HELIX_BF16, 11),
+    ((1103, 8, 64, 64, 96, 1), HELIX_BACKEND_SGMMA, 0, 9),
+    ((7059, 1, 32, 64, 96, 1), HELIX_BACKEND_AUTO, 0, 4),
+    ((1796, 4, 48, 192, 128, 1), HELIX_BACKEND_AUTO, 0, 10),
+    ((1659, 4, 16, 128, 128, 2), HELIX_BACKEND_SGMMA, HELIX_F16, 4),
+]
+
+
+@pytest.mark.parametrize("shape,backend,io,length", PLANS)
+def test_plan_lengths(host, shape, backend, io, length):
+    d = mp(shape, backend)
+    d.io_dtype = io
+    k, r = host.plan_info(d), host.run_info(d)
+    assert (k.seg_len, r.run_len) == (length, length)
+    assert r.runs_per_group == k.segs_per_group and k.walk_len % k.seg_len == 0
+
+
+def test_plan_lengths_any_shape(host):
+    """Whatever the shape, segments and runs cover the group, walks nest, and Pass B has one place."""
+    rng = np.random.default_rng(7)
+    for _ in range(400):
+        G = int(rng.choice([1, 2, 8]))
+        shape = (int(2 ** rng.uniform(0, 15)), int(rng.integers(1, 9)), G * int(rng.integers(1, 17)),
+                 8 * int(rng.integers(1, 25)), 8 * int(rng.integers(1, 33)), G)
+        for backend, io, multipass in ((HELIX_BACKEND_MPP, 0, True), (HELIX_BACKEND_SGMMA, 0, True),
+                                       (HELIX_BACKEND_SGMMA, HELIX_F16, True), (HELIX_BACKEND_AUTO, 0, False)):
+            d = mp(shape, backend)
+            d.io_dtype, d.multipass = io, multipass
+            k, r = host.plan_info(d), host.run_info(d)
+            if r.one_launch:
+                continue
+            assert k.total_bytes == host.scratch_size(d)
+            assert 1 <= k.seg_len <= k.chunks_per_group and k.segs_per_group == -(-k.chunks_per_group // k.seg_len)
+            if r.run_len:
+                assert r.run_len % k.seg_len == 0 and r.run_len <= k.walk_len and k.walk_len % k.seg_len == 0
+            assert (r.kernel_b is None) == (k.pass_b == abi.PASS_B_IN_C)
+            if r.kernel_b is None:
+                assert k.n_groups == 1 and k.segs_per_group <= 4 and r.run_len == k.seg_len
+
+
 def test_run_info_single_pass(host):
     d = desc_init(*CONFIG_SHAPES["cfg2"])
     d.multipass = False
