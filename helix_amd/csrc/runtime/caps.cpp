@@ -315,9 +315,14 @@ namespace helix::rt {
 // a little more than the bf16 path's. Measured at 64..640 tokens x 1..8
 // sequences of 8..80 heads, 27 heads of 192: at the limits below 18-31 us
 // against 18-42, one step past them 18-38 against 17-44.
-bool one_launch_scan(const helix_scan_desc& d, bool fp32_path) {
+namespace {
+long one_launch_units(const helix_scan_desc& d) {
     const long wg = (long)d.n_seq * d.n_head * ((d.head_dim + HELIX_HD - 1) / HELIX_HD) * 4;
-    const long u = (wg + 255) / 256 * ((d.n_tok + HELIX_CS - 1) / HELIX_CS + 1);
+    return (wg + 255) / 256 * ((d.n_tok + HELIX_CS - 1) / HELIX_CS + 1);
+}
+}  // namespace
+bool one_launch_scan(const helix_scan_desc& d, bool fp32_path) {
+    const long u = one_launch_units(d);
     return u <= (d.io_dtype == HELIX_F32 ? 5 : 4) + (d.d_state > 64 ? 1 : 0) + (fp32_path ? 1 : 0);
 }
 
@@ -453,10 +458,16 @@ const HelixMatmulTraits& no_copies(const helix_ctx* ctx, const HelixMatmulTraits
     return tr.nocopy && tuning_of(ctx).planned ? *tr.nocopy : tr;
 }
 
+// The form without scratch keeps its state tiles in y only where that is the
+// faster form: 481 tokens of 16 heads take 79 us with tiles in y (segments must be
+// long enough for a tile) and 34 in one launch, two blocks of 455 tokens x 64 heads
+// x 2 sequences 155 and 136; 1824 tokens of 8 heads 95 and 101.
+bool tiles_in_y_slower(const helix_ctx* ctx, const helix_scan_desc& d, const HelixMatmulTraits& tr);
+
 const HelixMatmulTraits* short_scan_traits(const helix_ctx* ctx, const helix_scan_desc& d,
                                            const HelixMatmulTraits& tr) {
     if (!tuning_of(ctx).planned || d.a_form != HELIX_A_SCALAR_PER_HEAD || d.d_state > HELIX_N_BLOCK ||
-        !one_launch_scan(d, tr.backend == HELIX_BACKEND_SGMMA))
+        !(one_launch_scan(d, tr.backend == HELIX_BACKEND_SGMMA) || tiles_in_y_slower(ctx, d, tr)))
         return nullptr;
     return &table().single[io_index(d.io_dtype)][np_index(d.d_state)];
 }
@@ -837,6 +848,15 @@ MultipassPlan plan_ytile(const helix_ctx* ctx, const helix_scan_desc& d, const H
     pl.n_hblk = d.n_head / d.n_group;
     *tr_out = &tr;
     return pl;
+}
+
+bool tiles_in_y_slower(const helix_ctx* ctx, const helix_scan_desc& d, const HelixMatmulTraits& tr) {
+    const HelixMatmulTraits* ytr = nullptr;
+    if (!tr.k_single) return false;
+    const MultipassPlan pl = plan_ytile(ctx, d, tr, &ytr);
+    // The one launch's time as one_launch_scan has it.
+    return ytr && one_launch_units(d) * (d.d_state > 64 ? 3.7 : 2.8) + 1.0 <
+                      best_plan(d, *ytr, pl.n_chunks, false, pl.seg_len).us;
 }
 
 bool build_params(const helix_scan_desc& d, HelixScanParams* o, std::string* why) {

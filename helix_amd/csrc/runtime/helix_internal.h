@@ -35,7 +35,8 @@ struct helix_tuning {
     int  hblk        = 0;      // HELIX_HBLK: heads per chunk-parallel Pass C workgroup
     int  f32_walk    = -1;     // HELIX_F32_WALK=0 / 1: the fp32 path's chunk-parallel Pass C / walk
                                // (on per-chunk states stored by Pass A) at d_state 128
-    int  ytile       = -1;     // HELIX_1PASS_Y=0: the single pass in its one-launch form only
+    int  ytile       = -1;     // HELIX_1PASS_Y=0 / 1: the single pass in its one-launch form only / with its
+                               // state tiles in y wherever they fit
     bool planned     = true;   // none of the measurement overrides (this struct, the scratch limit and
                                // FORCE_BACKEND aside) is set: a short scan may run as one launch
                                // (one_launch_scan), a plan with copies without them (no_copies)

@@ -73,10 +73,10 @@ PASSES = {"HELIX_STATE_BLOCKS": "1"}
 MODES = [
     # (label, backend, scratch_mb, memory, extra environment, multipass)
     ("1pass", HELIX_BACKEND_AUTO, None, "short", {}, False),
-    ("1pass/long", HELIX_BACKEND_AUTO, None, "long", {}, False),
-    # The single pass in its one-launch form everywhere (by default the
-    # shapes with rows for a state tile run the three passes with the tiles
-    # in y, test_gpu_single_y.py).
+    # The single pass as three passes with the state tiles in y wherever a
+    # shape has the rows for them (test_gpu_single_y.py), and in its
+    # one-launch form everywhere; by default the faster of the two.
+    ("1pass/long", HELIX_BACKEND_AUTO, None, "long", {"HELIX_1PASS_Y": "1"}, False),
     ("1pass/1launch/long", HELIX_BACKEND_AUTO, None, "long", {"HELIX_1PASS_Y": "0"}, False),
     ("fp32", HELIX_BACKEND_SGMMA, None, "short", {}, True),
     ("fp32/sm", HELIX_BACKEND_SGMMA, 1, "short", PASSES, True),

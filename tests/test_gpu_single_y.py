@@ -21,6 +21,13 @@ from gpu_harness import F32_ABS, F32_REL, T, ctx_for, run, upload
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture
+def gpu(gpu):
+    """A context that keeps the tiles-in-y form where one launch would be faster."""
+    return ctx_for(gpu, HELIX_1PASS_Y="1")
+
+
 # (L, S, H, P, N, G, label): every one plans state_in_y.
 Y_SHAPES = [
     (1000, 3, 4, 80, 128, 2, "P=80: a 16-channel last slab, 513-row tiles"),
@@ -51,7 +58,7 @@ def test_state_in_y_parity(gpu, shape):
     p, d = _problem(shape, 4343)
     info = gpu.plan_info(d)
     assert (info.state_in_y, info.launches, info.total_bytes) == (1, 3, 0)
-    assert gpu.scratch_size(d) == 0
+    assert gpu.scratch_size(d) == 0 and gpu.run_info(d).one_launch == 0
     y_ref, s_ref = po.scan(p, threads=0)
     _, y, s1 = run(gpu, p, desc=d)
     _check(y, s1, y_ref, s_ref, shape[-1])

@@ -11,8 +11,9 @@ import torch
 
 from oracle import pyoracle as po
 from helix_amd.desc import HELIX_BF16, HELIX_F16, HELIX_F32
+from helix_amd import scan
 from helix_amd.scan import make_desc, ssd_scan
-from gpu_harness import BF16_ABS, BF16_REL, F32_ABS, F32_REL
+from gpu_harness import BF16_ABS, BF16_REL, F32_ABS, F32_REL, ctx_for
 from test_gpu_io import TORCH, U, rounded
 
 pytestmark = pytest.mark.gpu
@@ -24,6 +25,14 @@ IDS = {HELIX_F32: "f32", HELIX_BF16: "bf16", HELIX_F16: "f16"}
 
 def up(a, dtype=torch.float32):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda().to(dtype)
+
+
+@pytest.fixture
+def gpu(gpu, monkeypatch):
+    """ssd_scan on a context that keeps the form the route names (HELIX_1PASS_Y=1: tiles in y)."""
+    ctx = ctx_for(gpu, HELIX_1PASS_Y="1")
+    monkeypatch.setitem(scan._contexts, torch.cuda.current_device(), ctx)
+    return ctx
 
 
 def check(p, y, s1, io, bf16):
@@ -62,7 +71,7 @@ def test_tokens_inside_channels(gpu, route):
     dt, A, s0 = up(p.dt), up(p.A), up(p.s0)
     B, C = up(p.B, TORCH[io]), up(p.C, TORCH[io])
     d = make_desc(x, dt, B, C, s0, y, A, backend=backend, multipass=multipass)
-    info = gpu.plan_info(d)
+    info = gpu.run_info(d)
     assert b"walk" in info.kernel_c if label != "one launch" else info.kernel_c is None
     _, s1 = ssd_scan(x, dt, A, B, C, s0, backend=backend, multipass=multipass, y=y)
     torch.cuda.synchronize()
@@ -85,7 +94,7 @@ def test_lowest_decay(gpu, route):
     p.dt += 6.0     # dt of about 0.6
     x, B, C = up(p.x, TORCH[io]), up(p.B, TORCH[io]), up(p.C, TORCH[io])
     d = make_desc(x, up(p.dt), B, C, up(p.s0), x, up(p.A), backend=backend, multipass=multipass)
-    info = gpu.plan_info(d)
+    info = gpu.run_info(d)
     assert b"walk" in info.kernel_c if label != "one launch" else info.kernel_c is None
     y, s1 = ssd_scan(x, up(p.dt), up(p.A), B, C, up(p.s0), backend=backend, multipass=multipass)
     torch.cuda.synchronize()

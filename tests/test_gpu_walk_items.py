@@ -257,7 +257,7 @@ NO_STATE = [   # (shape, multipass, backend, knobs): every place that reads s0
     ((1500, 1, 8, 64, 64, 1), True, "bf16", {"HELIX_SCRATCH_MB": 1}),  # Pass B, many groups
     ((1024, 4, 40, 64, 128, 1), True, "bf16", {}),                     # the bf16 walk's prologue
     ((1024, 4, 40, 64, 128, 1), True, "fp32", {}),                     # the fp32 walk's
-    ((600, 1, 16, 64, 128, 2), False, "auto", {}),                     # state tiles in y
+    ((600, 1, 16, 64, 128, 2), False, "auto", {"HELIX_1PASS_Y": "1"}),  # state tiles in y
     ((100, 2, 8, 72, 256, 1), True, "auto", {}),                       # one launch per block of state indices
 ]
 

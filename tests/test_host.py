@@ -732,6 +732,16 @@ def test_plan_lengths_any_shape(host):
                 assert k.n_groups == 1 and k.segs_per_group <= 4 and r.run_len == k.seg_len
 
 
+def test_single_pass_form(host):
+    """Tiles in y, or one launch where that is faster, unless a tuning variable keeps the plan."""
+    for shape, one in (((481, 1, 16, 64, 128, 2), 1), ((1824, 1, 8, 64, 128, 1), 0), (CONFIG_SHAPES["cfg1"], 0),
+                       ((455, 2, 64, 64, 256, 8), 1)):
+        d = mp(shape)
+        d.multipass = False
+        assert host.plan_info(d).state_in_y == 1 and host.run_info(d).one_launch == one, shape
+        assert tuned(HELIX_1PASS_Y="1").run_info(d).one_launch == 0
+
+
 def test_run_info_single_pass(host):
     d = desc_init(*CONFIG_SHAPES["cfg2"])
     d.multipass = False
