@@ -70,6 +70,7 @@ class HelixRunInfo(ctypes.Structure):
         ("copies", c_int32),
         ("run_len", c_int32),
         ("runs_per_group", c_int32),
+        ("run_items", c_int32),
         ("kernel_a", ctypes.c_char_p),
         ("kernel_b", ctypes.c_char_p),
         ("kernel_c", ctypes.c_char_p),

@@ -122,6 +122,8 @@ typedef struct HelixScanParams {
     int n_walk;           /* walk segments in this group = ceil(n_cg / walk_len) */
     int hblk;             /* heads per Pass C workgroup */
     int n_hblk;           /* head blocks per B/C group */
+    int walk_items;       /* (head, P slab) items per workgroup of the walk that
+                             takes up to HELIX_HB */
     int np;               /* d_state padded to the kernels' tile width (64/128/256) */
     int cpg;              /* chunks per group of the plan (scratch strides) */
     int fuse_b;           /* 1 => no Pass B launch: the walking Pass C forms S_seg

@@ -380,7 +380,8 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
     // sequence), as Pass A's: an XCD's share is whole token rows of one stretch
     // of a sequence, and a group's item blocks share the XCD's L2.
     const int ipg = p.heads_per_group * p.n_pslab;
-    const int nib = (ipg + HB - 1) / HB;
+    const int ipb = p.walk_items;              // items per workgroup, at most HB
+    const int nib = (ipg + ipb - 1) / ipb;
     const unsigned total = (unsigned)p.n_walk * (unsigned)p.n_group * (unsigned)nib * (unsigned)p.n_seq;
     unsigned wid = xcd_logical_id(blockIdx.x, total);
     const int ib  = (int)(wid % (unsigned)nib);       wid /= (unsigned)nib;
@@ -388,14 +389,15 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
     const int seg = (int)(wid % (unsigned)p.n_walk);  wid /= (unsigned)p.n_walk;
     const int seq = (int)wid;
     // This wave's item and 32-column block of its slab. Each SIMD (waves s and
-    // s + 4) holds one item; in a block of at most two items their four waves
-    // take a SIMD each instead. The other waves only stage B and C and take
+    // s + 4) holds one item; in a block of at most two items (also where the plan
+    // asks for two: a grid that would leave half of the CUs idle) their four waves
+    // take a SIMD each instead, and a chunk step takes about 0.8 of the time. The other waves only stage B and C and take
     // their share of G1.
-    const int n_live = min(HB, ipg - ib * HB);
+    const int n_live = min(ipb, ipg - ib * ipb);
     const int is = n_live > 2 ? wave % HB : (wave % HB) >> 1;
     const int pt = n_live > 2 ? wave / HB : wave & 1;
     const bool item_ok = is < n_live && (n_live > 2 || wave < HB);
-    const int ii = ib * HB + min(is, n_live - 1);
+    const int ii = ib * ipb + min(is, n_live - 1);
     const int h = g * p.heads_per_group + ii / p.n_pslab;
     const int slab = ii % p.n_pslab;
     const int p0 = slab * HELIX_HD;

@@ -340,6 +340,7 @@ helix_tuning tuning_from_env() {
     t.seg_len = (int)env_long("HELIX_SEG_LEN", 0);
     t.walk_len = (int)env_long("HELIX_WALK_LEN", 0);
     t.hblk = (int)env_long("HELIX_HBLK", 0);
+    t.walk_items = (int)std::min<long>(env_long("HELIX_WALK_ITEMS", 0), HELIX_HB);
     const int fw = env_switch("HELIX_F32_WALK");
     if (fw >= 0) t.f32_walk = fw > 0 ? 1 : 0;
     const int yt = env_switch("HELIX_1PASS_Y");
@@ -347,7 +348,7 @@ helix_tuning tuning_from_env() {
     const int sb = env_switch("HELIX_STATE_BLOCKS");
     if (sb >= 0) t.state_blocks = sb > 0 ? 1 : 0;
     for (const char* k : {"HELIX_PASSA_SPLIT", "HELIX_PASSA_F16", "HELIX_FUSE_B",
-                          "HELIX_WALK_BCCOPY", "HELIX_SEG_LEN", "HELIX_WALK_LEN", "HELIX_HBLK", "HELIX_F32_WALK",
+                          "HELIX_WALK_BCCOPY", "HELIX_SEG_LEN", "HELIX_WALK_LEN", "HELIX_WALK_ITEMS", "HELIX_HBLK", "HELIX_F32_WALK",
                           "HELIX_1PASS_Y", "HELIX_STATE_BLOCKS"})
         if (std::getenv(k)) t.planned = false;
     return t;
@@ -536,7 +537,7 @@ struct PlanCost {
 // thirteen shapes (600 to 8192 tokens, 1 to 8 sequences of 16 to 96 heads, some of
 // several slabs), inputs out of the Infinity Cache: rms errors 4-6 % each, no
 // sign of a bias in length. By kernels: d_state up to 64, up to 128.
-constexpr double kFoldG = 0.4;
+constexpr double kFoldG = 0.3;
 constexpr PlanCost kCostBf16F32[2]  = {{{2.22, 0.00354, 1.5, 0}, {4.15, 0.0101, 0.5, kFoldG}},
                                        {{2.69, 0.00426, 2.0, 0}, {4.55, 0.0114, 0.75, kFoldG}}};
 constexpr PlanCost kCostBf16Io16[2] = {{{2.27, 0.00112, 1.5, 0}, {4.27, 0.00357, 0.75, kFoldG}},
@@ -559,20 +560,20 @@ const PlanCost& plan_cost(const helix_scan_desc& d, const HelixMatmulTraits& tr)
     return d.io_dtype == HELIX_F32 ? kCostF32[n] : d.io_dtype == HELIX_BF16 ? kCostF32Bf16[n] : kCostF32F16[n];
 }
 
-// The workgroups of either launch over a group of cpg chunks in runs of len, in
-// their kernels' logical order (item block, group, run, sequence).
+// The workgroups of either launch over a group of cpg chunks in runs of len, of
+// `items` items each, in their kernels' logical order (item block, group, run,
+// sequence).
 struct PlanGrid {
     long per_run;    // item blocks x groups
-    int  nib, cpg, len, n_run, n_seq;
-    double last;     // share of the last item block's items that are real
+    int  cpg, len, n_run, n_seq;
+    double weight;   // of a run's workgroups: HELIX_HB items count 1
 
-    PlanGrid(const helix_scan_desc& d, int cpg_, int len_) : cpg(cpg_), len(len_) {
+    PlanGrid(const helix_scan_desc& d, int cpg_, int len_, int items) : cpg(cpg_), len(len_) {
         const int ipg = d.n_head / d.n_group * ((d.head_dim + HELIX_HD - 1) / HELIX_HD);
-        nib = (ipg + HELIX_HB - 1) / HELIX_HB;
-        per_run = (long)nib * d.n_group;
+        per_run = (long)((ipg + items - 1) / items) * d.n_group;
         n_run = (cpg + len - 1) / len;
         n_seq = d.n_seq;
-        last = (double)(ipg - HELIX_HB * (nib - 1)) / HELIX_HB;
+        weight = (double)ipg * d.n_group / HELIX_HB;
     }
     long total() const { return per_run * n_run * n_seq; }
     int run_of(long wid) const { return (int)(wid / per_run % n_run); }
@@ -581,8 +582,7 @@ struct PlanGrid {
     }
     // The chunk steps of every workgroup, weighted.
     double work(const DispatchCost& c, bool fold) const {
-        const double w = (double)per_run / nib * (nib - 1 + last);
-        return w * n_seq * (cpg + n_run * c.o + (fold ? c.g * 0.5 * n_run * (n_run - 1) : 0.0));
+        return weight * n_seq * (cpg + n_run * c.o + (fold ? c.g * 0.5 * n_run * (n_run - 1) : 0.0));
     }
     // No schedule is shorter than its longest workgroup, or than all of them spread evenly.
     double makespan_bound(const DispatchCost& c, bool fold) const {
@@ -614,35 +614,56 @@ double makespan(const PlanGrid& g, const DispatchCost& c, bool fold) {
     return T;
 }
 
+// Items per workgroup of the walk in runs of len chunks: two where that makes no
+// second round of workgroups, for a chunk step then takes about 0.7 of the time on
+// the fp32-accurate walk and 0.77 on the bf16 path's (a SIMD has one working wave
+// instead of two), at somewhat more per workgroup. 1824 tokens of 8 heads with tiles
+// in y 97 -> 78 us, 2048 of 64 heads 94 -> 79, 628 of 24 heads on the bf16 path 33
+// -> 31; past one round 8192 tokens of 64 heads would go from 124 to 144. One item
+// each gains no more.
+int walk_items_for(const helix_scan_desc& d, int cpg, int len) {
+    return PlanGrid(d, cpg, len, 2).total() <= kCus ? 2 : HELIX_HB;
+}
+
 // Microseconds of a group of cpg chunks in segments = runs of len chunks. The
 // chip is busy throughout, so the integral of lat + k * load over a launch is
 // lat * T + k * work. A launch of Pass B reads every segment's aggregate and
-// writes every run's start state and s1 (fitted to whole scans less the other
-// two passes). bound: with the makespans' lower bounds instead.
+// writes every run's start state and s1; folded in, a workgroup's first chunk waits
+// for s0 and the aggregates. bound: with the makespans' lower bounds instead.
 double plan_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, int len, bool fold, bool bound) {
     const PlanCost& pc = plan_cost(d, tr);
-    const PlanGrid g(d, cpg, len);
+    const PlanGrid g(d, cpg, len, HELIX_HB);
+    const int items = walk_items_for(d, cpg, len);
+    const PlanGrid gc(d, cpg, len, items);
+    DispatchCost c = pc.c;
+    if (items < HELIX_HB) {
+        c.lat *= tr.bf16_state ? 0.77 : 0.7;
+        c.o += tr.bf16_state ? 0.4 : 0.25;
+    }
     const double mb = 1e-6 * d.n_seq * d.n_head * ((d.head_dim + HELIX_HD - 1) / HELIX_HD) * 64.0 * tr.np * sizeof(float);
-    double us = fold ? 0.0 : 2.0 + mb * (0.34 * g.n_run + 0.15);
-    us += pc.a.k * g.work(pc.a, false) + pc.c.k * g.work(pc.c, fold);
+    double us = fold ? (tr.np > 64 ? 3.0 : 0.0) : mb * (0.25 * g.n_run + 0.5);
+    us += pc.a.k * g.work(pc.a, false) + c.k * gc.work(c, fold);
     us += pc.a.lat * (bound ? g.makespan_bound(pc.a, false) : makespan(g, pc.a, false));
-    us += pc.c.lat * (bound ? g.makespan_bound(pc.c, fold) : makespan(g, pc.c, fold));
+    us += c.lat * (bound ? gc.makespan_bound(c, fold) : makespan(gc, c, fold));
     return us;
 }
 
-// The chunks per Pass A segment and walk run with the least modelled time, and that
-// time, over a group of cpg chunks. fold: whether the plan may fold Pass B into the
-// walk where there are few enough segments. len: this length and no other
-// (0: any). Memoized: the plan is remade on every encode.
+// The chunks per Pass A segment and walk run with the least modelled time, whether
+// the walk folds Pass B in, and that time, over a group of cpg chunks. fold: whether
+// the plan may fold. len: this length and no other (0: any). Memoized: the plan is
+// remade on every encode.
 //
-// Against every length timed on 36 shapes over both paths, all storage types and
-// the form without scratch, the choice was within 0.3 % of the best on average
-// (4 % at most). The lengths that the walk of two heads per workgroup had were
-// 23 % off (4 x 1392 tokens of 64 heads of 80, bf16 storage: runs of 22 and 194 us
-// against 11 and 117; 7059 tokens of 32 heads: 108 us against 68).
+// Against every length timed on 36 shapes of the whole range over both paths, all
+// storage types and the form without scratch, the choice was within 0.3 % of the
+// best on average (4 % at most). The lengths that the walk of two heads per
+// workgroup had were 23 % off (4 x 1392 tokens of 64 heads of 80, bf16 storage: runs
+// of 22 and 194 us against 11 and 117; 7059 tokens of 32 heads: 108 us against 68).
+// Over 230 scans of 70 to 8000 tokens, most of them short, folded or not and with two
+// items per workgroup or four: 0.7 % on average, 17 % at most.
 struct PlanChoice {
     int len;
     double us;
+    bool fold;
 };
 bool folds(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, int len) {
     // A one-chunk run on the fp32 path with fp32 storage keeps Pass B's launch:
@@ -660,23 +681,26 @@ PlanChoice best_plan(const helix_scan_desc& d, const HelixMatmulTraits& tr, int 
         const auto it = memo.find(key);
         if (it != memo.end()) return it->second;
     }
-    auto us = [&](int l, bool bound) { return plan_us(d, tr, cpg, l, fold && folds(d, tr, cpg, l), bound); };
-    PlanChoice best{len, 0.0};
+    // Lengths up to 96 chunks, and the cuts into up to sixteen, by their lower
+    // bounds: few need their schedule.
+    std::vector<std::tuple<double, int, bool>> cand;
+    auto add = [&](int l) {
+        cand.emplace_back(plan_us(d, tr, cpg, l, false, true), l, false);
+        if (fold && folds(d, tr, cpg, l)) cand.emplace_back(plan_us(d, tr, cpg, l, true, true), l, true);
+    };
     if (len > 0) {
-        best.us = us(len, false);
+        add(len);
     } else {
-        // Lengths up to 96 chunks, and the cuts into up to sixteen, by their
-        // lower bounds: few need their schedule.
-        std::vector<std::pair<double, int>> cand;
-        for (int l = 1; l <= std::min(cpg, 96); ++l) cand.emplace_back(us(l, true), l);
+        for (int l = 1; l <= std::min(cpg, 96); ++l) add(l);
         for (int j = 1; j <= 16; ++j)
-            if ((cpg + j - 1) / j > 96) cand.emplace_back(us((cpg + j - 1) / j, true), (cpg + j - 1) / j);
-        std::sort(cand.begin(), cand.end());
-        for (const auto& [lower, l] : cand) {
-            if (best.len && lower >= best.us) break;
-            const double t = us(l, false);
-            if (!best.len || t < best.us) best = {l, t};
-        }
+            if ((cpg + j - 1) / j > 96) add((cpg + j - 1) / j);
+    }
+    std::sort(cand.begin(), cand.end());
+    PlanChoice best{0, 0.0, false};
+    for (const auto& [lower, l, f] : cand) {
+        if (best.len && lower >= best.us) break;
+        const double t = plan_us(d, tr, cpg, l, f, false);
+        if (!best.len || t < best.us) best = {l, t, f};
     }
     std::lock_guard<std::mutex> lk(mu);
     if (memo.size() > 4096) memo.clear();
@@ -700,12 +724,12 @@ void choose_lengths(const helix_tuning& tu, const helix_scan_desc& d, const Heli
         w = std::max(a, (w / a) * a);
     } else if (tr.walk_hb && tu.walk_len <= 0) {
         const int n_chunks = (d.n_tok + HELIX_CS - 1) / HELIX_CS;
-        const bool fold = tu.fuse_b != 0 && cpg == n_chunks;
-        a = best_plan(d, tr, cpg, fold, 0).len;
-        if (fold && folds(d, tr, cpg, a))
-            w = a;
+        const PlanChoice c = best_plan(d, tr, cpg, tu.fuse_b != 0 && cpg == n_chunks, 0);
+        a = c.len;
+        if (c.fold || (w == 1 && !tr.bf16_state && d.io_dtype == HELIX_F32))
+            w = a;   // the second: HELIX_F32_WALK=1 where the chunk-parallel kernel is planned
         else
-            w = w > 1 ? std::max(2 * a, (w / a) * a) : a;
+            w = std::max(2 * a, (w / a) * a);
     } else if (tr.a_hb) {
         const long per_seg = item_blocks(d);
         a = 1;
@@ -734,6 +758,7 @@ void layout(const helix_tuning& tu, const helix_scan_desc& d, const HelixMatmulT
     pl->segs_per_group = (cpg + pl->seg_len - 1) / pl->seg_len;
     pl->walks_per_group = (cpg + pl->walk_len - 1) / pl->walk_len;
     pl->run_len = tr.walk_hb && tu.walk_len <= 0 ? pl->seg_len : pl->walk_len;
+    pl->walk_items = tu.walk_items > 0 ? tu.walk_items : walk_items_for(d, cpg, pl->run_len);
     pl->sl_elem_bytes = bf16_state ? 2 : 4;
     pl->sl_elems = (pl->seg_len > 1 && !walk) ? state * (size_t)cpg : 0;
     pl->sg_elems = state * (size_t)pl->segs_per_group;
@@ -839,7 +864,10 @@ MultipassPlan plan_ytile(const helix_ctx* ctx, const helix_scan_desc& d, const H
         if (t2.seg_len <= 0) return pl = MultipassPlan{}, pl;
         layout(t2, d, tr, (int)n_chunks, &pl);
         if (!fits(pl.seg_len)) return pl = MultipassPlan{}, pl;
-        if (tu.walk_len <= 0) pl.run_len = pl.seg_len;
+        if (tu.walk_len <= 0) {
+            pl.run_len = pl.seg_len;
+            if (tu.walk_items <= 0) pl.walk_items = walk_items_for(d, (int)n_chunks, pl.run_len);
+        }
     }
     pl.n_chunks = (int)n_chunks;
     pl.n_groups = 1;

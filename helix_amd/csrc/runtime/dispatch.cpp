@@ -278,6 +278,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
     params.np      = tr.np;
     params.seg_len = plan.seg_len;
     params.walk_len = plan.run_len;
+    params.walk_items = plan.walk_items;
     params.hblk    = plan.hblk;
     params.n_hblk  = plan.n_hblk;
     params.sl_cg   = HT;
@@ -320,11 +321,13 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
     const unsigned hpg = (unsigned)(d->n_head / d->n_group);
     const unsigned hpw = tr.walk_hpw > 0 ? (unsigned)tr.walk_hpw : HELIX_WALK_HPW(tr.np);
     const unsigned pairs = (hpg + hpw - 1) / hpw;
-    // Head-block Pass A and walk: item blocks of HELIX_HB (head, P slab) pairs per group.
+    // Head-block Pass A and walk: item blocks of HELIX_HB, or the walk's walk_items, (head, P slab)
+    // pairs per group.
     const long long ipg = (long long)hpg * params.n_pslab;
     const long long nib = (ipg + HELIX_HB - 1) / HELIX_HB;
     auto pass_c_groups = [&](int n_cg, int n_walk) -> long long {
-        if (tr.walk_hb) return (long long)d->n_seq * d->n_group * nib * n_walk;
+        if (tr.walk_hb)
+            return (long long)d->n_seq * d->n_group * ((ipg + plan.walk_items - 1) / plan.walk_items) * n_walk;
         return tr.walk ? (long long)n_walk * d->n_group * pairs * params.n_pslab * d->n_seq
                        : (long long)n_cg * d->n_group * plan.n_hblk * d->n_seq;
     };
@@ -671,6 +674,7 @@ extern "C" helix_status helix_scan_run_info(helix_ctx* ctx, const helix_scan_des
     const HelixMatmulTraits& kt = helix::rt::no_copies(ctx, *tr);
     out->copies = kt.bccopy ? 1 : 0;
     out->run_len = kt.walk ? pl.run_len : 0;
+    out->run_items = kt.walk_hb ? pl.walk_items : 0;
     out->runs_per_group = kt.walk ? (pl.chunks_per_group + pl.run_len - 1) / pl.run_len : 0;
     out->kernel_a = kt.k_chunk_state;
     out->kernel_b = helix::rt::fuse_b_on(ctx, *tr, pl) ? nullptr : kt.k_state_scan;

@@ -37,6 +37,7 @@ struct helix_tuning {
                                // (on per-chunk states stored by Pass A) at d_state 128
     int  ytile       = -1;     // HELIX_1PASS_Y=0 / 1: the single pass in its one-launch form only / with its
                                // state tiles in y wherever they fit
+    int  walk_items  = 0;      // HELIX_WALK_ITEMS=1..4: items per workgroup of the walk with walk_hb
     bool planned     = true;   // none of the measurement overrides (this struct, the scratch limit and
                                // FORCE_BACKEND aside) is set: a short scan may run as one launch
                                // (one_launch_scan), a plan with copies without them (no_copies)
@@ -148,6 +149,7 @@ struct MultipassPlan {
     int    walks_per_group  = 0;
     int    run_len          = 0;   // chunks per workgroup of the walking Pass C: walk_len, or with walk_hb and no
                                    // HELIX_WALK_LEN seg_len
+    int    walk_items       = HELIX_HB;   // items per workgroup of the walk with walk_hb
     int    hblk             = 0;
     int    n_hblk           = 0;
     size_t sl_elems         = 0;   // s_local elements (0 when seg_len == 1)

@@ -93,6 +93,8 @@ typedef struct {
                                    multiple of seg_len, at most walk_len; 0 off
                                    the walk                                      */
     int32_t  runs_per_group;    /* such runs per sequence and chunk group        */
+    int32_t  run_items;         /* (head, 64-channel slab) items per workgroup of
+                                   the walk up to d_state 128; 0 off it          */
     const char* kernel_a;       /* NULL where not launched                       */
     const char* kernel_b;
     const char* kernel_c;

@@ -30,14 +30,20 @@ SHAPES = [
 ]
 
 
+# Items per workgroup: four, and two as a small grid has by default.
+ITEMS = pytest.mark.parametrize("items", ["4", "2"], ids=["four", "two"])
+
+
+@ITEMS
 @pytest.mark.parametrize("shape,knobs", SHAPES, ids=["x".join(map(str, s)) + ("k" if k else "") for s, k in SHAPES])
-def test_item_blocks(gpu, shape, knobs):
+def test_item_blocks(gpu, shape, knobs, items):
     p = po.problem_harness(*shape, 515, "long")
     p.s0 = (np.random.default_rng(5).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
     y_ref, s_ref = po.scan(p, use_ids=False)
-    ctx = ctx_for(gpu, HELIX_F32_WALK="1", **knobs)
+    ctx = ctx_for(gpu, HELIX_F32_WALK="1", HELIX_WALK_ITEMS=items, **knobs)
     d = p.d.copy()
     d.backend, d.multipass = HELIX_BACKEND_SGMMA, True
+    assert ctx.run_info(d).run_items == int(items)
     assert b"helix_scan_walk_x6_n" in ctx.plan_info(d).kernel_c
     assert ctx.run_info(d).run_len == knobs.get("HELIX_WALK_LEN", 1)
     _, y, s1 = run(ctx, p, d)
@@ -45,14 +51,15 @@ def test_item_blocks(gpu, shape, knobs):
     assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
 
 
+@ITEMS
 @pytest.mark.parametrize("copies", ["0", "1"], ids=["rows", "copies"])
 @pytest.mark.parametrize("shape,knobs", SHAPES, ids=["x".join(map(str, s)) + ("k" if k else "") for s, k in SHAPES])
-def test_item_blocks_bf16(gpu, shape, knobs, copies):
+def test_item_blocks_bf16(gpu, shape, knobs, copies, items):
     """The bf16 path's instantiations, on the caller's rows of B and C and on Pass A's bf16 copies."""
     p = po.problem_harness(*shape, 515, "long")
     p.s0 = (np.random.default_rng(5).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
     y_ref, s_ref = po.scan(p, use_ids=False)
-    ctx = ctx_for(gpu, HELIX_WALK_BCCOPY=copies, **knobs)
+    ctx = ctx_for(gpu, HELIX_WALK_BCCOPY=copies, HELIX_WALK_ITEMS=items, **knobs)
     d = p.d.copy()
     d.backend, d.multipass = HELIX_BACKEND_MPP, True
     assert (b"helix_scan_walk16_bf16_bc_n" if copies == "1" else b"helix_scan_walk16_bf16_n") in ctx.plan_info(d).kernel_c
@@ -117,14 +124,15 @@ RUNS = [
 ]
 
 
+@ITEMS
 @pytest.mark.parametrize("io", [HELIX_BF16, HELIX_F16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("shape,knobs", RUNS, ids=["x".join(map(str, s)) for s, _ in RUNS])
-def test_16bit_storage_runs(gpu, shape, knobs, backend, io):
+def test_16bit_storage_runs(gpu, shape, knobs, backend, io, items):
     p = rounded(po.problem_harness(*shape, 617, "long"), io)
     p.s0 = (np.random.default_rng(6).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
     y_ref, s_ref = po.scan(p, use_ids=False)
-    ctx = ctx_for(gpu, **knobs)
+    ctx = ctx_for(gpu, HELIX_WALK_ITEMS=items, **knobs)
     d = p.d.copy()
     d.io_dtype, d.backend, d.multipass = io, backend, True
     assert ctx.run_info(d).run_len == knobs["HELIX_WALK_LEN"] and ctx.plan_info(d).seg_len == knobs["HELIX_SEG_LEN"]
@@ -132,14 +140,15 @@ def test_16bit_storage_runs(gpu, shape, knobs, backend, io):
     check(io, desc, y, s1, y_ref, s_ref)
 
 
+@ITEMS
 @pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("N", [136, 256])
-def test_state_block_runs(gpu, N, backend):
+def test_state_block_runs(gpu, N, backend, items):
     """The walk that adds into y, over runs of several chunks."""
     p = po.problem_harness(1025, 1, 5, 72, N, 1, 618, "long")
     p.s0 = (np.random.default_rng(6).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
     y_ref, s_ref = po.scan(p, use_ids=False)
-    ctx = ctx_for(gpu, HELIX_WALK_LEN=6, HELIX_SEG_LEN=3, HELIX_F32_WALK="1")
+    ctx = ctx_for(gpu, HELIX_WALK_LEN=6, HELIX_SEG_LEN=3, HELIX_F32_WALK="1", HELIX_WALK_ITEMS=items)
     d = p.d.copy()
     d.backend, d.multipass = backend, True
     assert ctx.plan_info(d).state_blocks == 2 and ctx.run_info(d).run_len == 6

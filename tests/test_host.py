@@ -656,7 +656,7 @@ def _runs(d):
 def test_run_info(host, backend):
     # The plan's kernels and runs where the plan is what is launched ...
     d, k = mp(CONFIG_SHAPES["cfg2"], backend), host.plan_info(mp(CONFIG_SHAPES["cfg2"], backend))
-    assert _runs(d) == {"one_launch": 0, "copies": 0, "run_len": 8, "runs_per_group": 16, "kernel_a": k.kernel_a,
+    assert _runs(d) == {"one_launch": 0, "copies": 0, "run_len": 8, "runs_per_group": 16, "run_items": 4, "kernel_a": k.kernel_a,
                         "kernel_b": k.kernel_b, "kernel_c": k.kernel_c, "kernel_1pass": None}
     assert (k.walk_len, k.walks_per_group) == (16, 8)
     # ... the kernels without copies on a plan with them, alone and in blocks of state indices ...
@@ -730,6 +730,19 @@ def test_plan_lengths_any_shape(host):
             assert (r.kernel_b is None) == (k.pass_b == abi.PASS_B_IN_C)
             if r.kernel_b is None:
                 assert k.n_groups == 1 and k.segs_per_group <= 4 and r.run_len == k.seg_len
+
+
+def test_walk_items(host):
+    """Two items per workgroup of the walk where its grid then still fits the 256 CUs once."""
+    for shape, items in (((1024, 1, 64, 64, 128, 8), 2), ((1025, 1, 64, 64, 128, 8), 4), ((628, 1, 24, 64, 128, 1), 2),
+                         (CONFIG_SHAPES["cfg4b"], 4)):
+        d = mp(shape, HELIX_BACKEND_MPP)
+        k, r = host.plan_info(d), host.run_info(d)
+        L, S, H, P, N, G = shape
+        blocks = -(-(H // G * -(-P // 64)) // 2) * G * S * r.runs_per_group
+        assert r.run_items == items and (blocks <= 256) == (items == 2), shape
+    assert tuned(HELIX_WALK_ITEMS="4").run_info(mp((1024, 1, 64, 64, 128, 8), HELIX_BACKEND_MPP)).run_items == 4
+    assert host.run_info(mp((64, 1, 64, 64, 128, 8), HELIX_BACKEND_MPP)).run_items == 0
 
 
 def test_single_pass_form(host):
