@@ -317,25 +317,52 @@ HELIX_DEV float pk_hi(unsigned w) { return __builtin_bit_cast(float, w & 0xffff0
 // matrix pipe. Behind each 16 x 16 x 32 MFMA (18 cycles alone, two waves per
 // SIMD) two dot products took the pair to 39 cycles and four to 48, two and
 // four subtractions to 18 and 27; at config 2's shape the fp32 path's walk took
-// 164 us with the dot products and 161 without.
-HELIX_DEV float sub_lo(float a, unsigned w) { return a - pk_lo(w); }
-HELIX_DEV float sub_hi(float a, unsigned w) { return a - pk_hi(w); }
+// 164 us with the dot products and 161 without. DOT: by the dot product, exact as
+// well, where the splits stand apart from the products and the vector work counts
+// (stage_split8: the d_state 256 Pass A's staging; 8 x 2871 tokens of 24 heads, f16
+// storage, 491 us without and 484 with; the same bits).
+// The (-1, 0) and (0, -1) pairs reach the instruction in a scalar register: the
+// compiler would otherwise encode the first as the inline constant -1.0, which
+// the hardware applies as the fp32 bit pattern 0xbf800000, i.e. the pair (0, -1)
+// (measured).
+HELIX_DEV unsigned bf16_pair_reg(unsigned k) {
+    asm("" : "+s"(k));
+    return k;
+}
+template <bool DOT = false>
+HELIX_DEV float sub_lo(float a, unsigned w) {
+    if constexpr (DOT)
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w),
+                                               __builtin_bit_cast(bf16x2, bf16_pair_reg(0x0000bf80u)), a, false);
+    else
+        return a - pk_lo(w);
+}
+template <bool DOT = false>
+HELIX_DEV float sub_hi(float a, unsigned w) {
+    if constexpr (DOT)
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w),
+                                               __builtin_bit_cast(bf16x2, bf16_pair_reg(0xbf800000u)), a, false);
+    else
+        return a - pk_hi(w);
+}
 
 // Three-way bf16 split of the pair (a, b), each part packed as a pair:
-// 11 VALU operations for two values.
+// 11 VALU operations for two values (DOT: 7).
+template <bool DOT = false>
 HELIX_DEV void split3_pair(float a, float b, unsigned& w0, unsigned& w1, unsigned& w2) {
     w0 = pk_bf16(a, b);
-    const float ra = sub_lo(a, w0), rb = sub_hi(b, w0);
+    const float ra = sub_lo<DOT>(a, w0), rb = sub_hi<DOT>(b, w0);
     w1 = pk_bf16(ra, rb);
-    w2 = pk_bf16(sub_lo(ra, w1), sub_hi(rb, w1));
+    w2 = pk_bf16(sub_lo<DOT>(ra, w1), sub_hi<DOT>(rb, w1));
 }
 
 // Two-way bf16 split of the pair (a, b): v = v0 + v1 + e with |e| <= 2^-18 |v|,
-// 6 VALU operations for two values. Three products a0b0 + a0b1 + a1b0 leave
+// 6 VALU operations for two values (DOT: 4). Three products a0b0 + a0b1 + a1b0 leave
 // out terms of at most 3 * 2^-18 of |ab| (about 1.1e-5).
+template <bool DOT = false>
 HELIX_DEV void split2_pair(float a, float b, unsigned& w0, unsigned& w1) {
     w0 = pk_bf16(a, b);
-    w1 = pk_bf16(sub_lo(a, w0), sub_hi(b, w0));
+    w1 = pk_bf16(sub_lo<DOT>(a, w0), sub_hi<DOT>(b, w0));
 }
 
 // Six-product MFMA of split operands a[3] x b[3], smallest terms first.
@@ -427,9 +454,9 @@ HELIX_DEV void stage_split8(__bf16* planes, int r, int c, const float* v) {
     for (int e = 0; e < 4; ++e) {
         unsigned w[3];
         if constexpr (NS == 3)
-            split3_pair(v[2 * e], v[2 * e + 1], w[0], w[1], w[2]);
+            split3_pair<true>(v[2 * e], v[2 * e + 1], w[0], w[1], w[2]);
         else
-            split2_pair(v[2 * e], v[2 * e + 1], w[0], w[1]);
+            split2_pair<true>(v[2 * e], v[2 * e + 1], w[0], w[1]);
 #pragma unroll
         for (int k = 0; k < NS; ++k) q[k][e] = w[k];
     }
