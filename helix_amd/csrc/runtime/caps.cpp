@@ -537,7 +537,7 @@ struct PlanCost {
 // thirteen shapes (600 to 8192 tokens, 1 to 8 sequences of 16 to 96 heads, some of
 // several slabs), inputs out of the Infinity Cache: rms errors 4-6 % each, no
 // sign of a bias in length. By kernels: d_state up to 64, up to 128.
-constexpr double kFoldG = 0.3;
+constexpr double kFoldG = 0.1;
 constexpr PlanCost kCostBf16F32[2]  = {{{2.22, 0.00354, 1.5, 0}, {4.15, 0.0101, 0.5, kFoldG}},
                                        {{2.69, 0.00426, 2.0, 0}, {4.55, 0.0114, 0.75, kFoldG}}};
 constexpr PlanCost kCostBf16Io16[2] = {{{2.27, 0.00112, 1.5, 0}, {4.27, 0.00357, 0.75, kFoldG}},
@@ -641,7 +641,7 @@ double plan_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, i
         c.o += tr.bf16_state ? 0.4 : 0.25;
     }
     const double mb = 1e-6 * d.n_seq * d.n_head * ((d.head_dim + HELIX_HD - 1) / HELIX_HD) * 64.0 * tr.np * sizeof(float);
-    double us = fold ? (tr.np > 64 ? 3.0 : 0.0) : mb * (0.25 * g.n_run + 0.5);
+    double us = fold ? (tr.np > 64 ? 3.0 : 0.0) : 1.0 + mb * (0.25 * g.n_run + 0.5);
     us += pc.a.k * g.work(pc.a, false) + c.k * gc.work(c, fold);
     us += pc.a.lat * (bound ? g.makespan_bound(pc.a, false) : makespan(g, pc.a, false));
     us += c.lat * (bound ? gc.makespan_bound(c, fold) : makespan(gc, c, fold));
@@ -659,7 +659,7 @@ double plan_us(const helix_scan_desc& d, const HelixMatmulTraits& tr, int cpg, i
 // workgroup had were 23 % off (4 x 1392 tokens of 64 heads of 80, bf16 storage: runs
 // of 22 and 194 us against 11 and 117; 7059 tokens of 32 heads: 108 us against 68).
 // Over 230 scans of 70 to 8000 tokens, most of them short, folded or not and with two
-// items per workgroup or four: 0.7 % on average, 17 % at most.
+// items per workgroup or four: 0.8 % on average, 16 % at most.
 struct PlanChoice {
     int len;
     double us;

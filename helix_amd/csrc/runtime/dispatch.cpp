@@ -169,7 +169,7 @@ helix_status encode_one(helix_ctx* ctx, hipStream_t stream, const helix_scan_des
         one = nullptr;
     const HelixMatmulTraits* trp = one ? one : &sel;
     // It needs no scratch, but the caller's contract is the plan's.
-    if (one && !sel.k_single && !sel.fallback &&
+    if (one && !sel.k_single && !sel.fallback && !scratch_sized &&
         !scratch_fits(helix::rt::plan_multipass(ctx, *d, sel, budget_cap).total_bytes))
         return no_scratch();
     auto fn = [&](const char* name) -> hipFunction_t {
