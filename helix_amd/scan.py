@@ -72,8 +72,6 @@ def _scratch_for(device: int, st: int, nbytes: int, stream: torch.cuda.Stream | 
 
 
 def _capturing(device: int, st: int, stream) -> bool:
-    if stream is None:
-        return torch.cuda.is_current_stream_capturing()
     with _under(device, st, stream):
         return torch.cuda.is_current_stream_capturing()
 
@@ -163,10 +161,11 @@ def ssd_scan(x: torch.Tensor, dt: torch.Tensor, A: torch.Tensor, B: torch.Tensor
         d = DESC_STRUCT.pack(*fields, c_float(dt_min).value, c_float(dt_max).value)
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     ctx = _contexts.get(index) or context(index)
-    st = stream.cuda_stream if stream is not None else torch.cuda.current_stream(dev).cuda_stream
+    st = stream.cuda_stream if stream is not None else torch._C._cuda_getCurrentRawStream(index)
     lent = scratch
     # Work under capture gets memory of the graph's own, which no later call touches.
-    capturing = lent is None and _capturing(index, st, stream)
+    capturing = lent is None and (torch.cuda.is_current_stream_capturing() if stream is None
+                                  else _capturing(index, st, stream))
     if lent is None and not capturing:
         scratch = _scratch_for(index, st, 0)
     ptrs = (0 if s0 is None else s0.data_ptr(), x.data_ptr(), dt.data_ptr(), A.data_ptr(), B.data_ptr(), C.data_ptr(),
