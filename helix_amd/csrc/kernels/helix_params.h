@@ -87,6 +87,13 @@
 #define HELIX_HB 4
 #define HELIX_HB_THREADS (128 * HELIX_HB)
 
+// Whether the runs of an item block follow one another in the walk's logical order,
+// instead of the item blocks of a run (pass_c_walk_x6.hip has the reason): with Pass B
+// folded in, three runs or more, and fewer sequences than XCDs.
+constexpr bool walk_runs_inner(int fuse_b, int n_walk, int n_seq) {
+    return fuse_b != 0 && n_walk > 2 && n_seq < 8;
+}
+
 typedef struct HelixScanParams {
     int n_tok;
     int n_seq;

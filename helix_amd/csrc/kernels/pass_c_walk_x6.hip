@@ -378,16 +378,26 @@ __device__ __forceinline__ void scan_walk_x6_impl(const HelixScanParams& p, cons
 
     // 1-D grid in the logical order (item block, group, walk segment,
     // sequence), as Pass A's: an XCD's share is whole token rows of one stretch
-    // of a sequence, and a group's item blocks share the XCD's L2.
+    // of a sequence, and a group's item blocks share the XCD's L2. With Pass B
+    // folded in, a run reads the aggregates of all runs before it; where an XCD's
+    // share is less than a sequence, the XCDs with the late runs would read them
+    // all while the others have none, so from three runs on the runs of an item
+    // block follow one another there instead and share an XCD (one-chunk runs over
+    // four chunks, 16-bit storage: 194 tokens x 64 heads x 2 sequences 42.3 -> 33.5
+    // us, 245 x 64 heads of 80 44.5 -> 32.6; 2048 x 80 heads x 2 in four runs 97.5 ->
+    // 94.2; with two runs, 0.97 to 1.03 of the time either way).
     const int ipg = p.heads_per_group * p.n_pslab;
     const int ipb = p.walk_items;              // items per workgroup, at most HB
     const int nib = (ipg + ipb - 1) / ipb;
-    const unsigned total = (unsigned)p.n_walk * (unsigned)p.n_group * (unsigned)nib * (unsigned)p.n_seq;
-    unsigned wid = xcd_logical_id(blockIdx.x, total);
-    const int ib  = (int)(wid % (unsigned)nib);       wid /= (unsigned)nib;
-    const int g   = (int)(wid % (unsigned)p.n_group); wid /= (unsigned)p.n_group;
-    const int seg = (int)(wid % (unsigned)p.n_walk);  wid /= (unsigned)p.n_walk;
-    const int seq = (int)wid;
+    const unsigned per_run = (unsigned)nib * (unsigned)p.n_group, per_seq = per_run * (unsigned)p.n_walk;
+    const unsigned wid = xcd_logical_id(blockIdx.x, per_seq * (unsigned)p.n_seq);
+    const bool runs_inner = walk_runs_inner(p.fuse_b, p.n_walk, p.n_seq);
+    const unsigned inner = runs_inner ? (unsigned)p.n_walk : per_run;
+    const unsigned hi_id = wid % per_seq / inner, lo_id = wid % per_seq % inner;
+    const unsigned blk = runs_inner ? hi_id : lo_id;
+    const int seq = (int)(wid / per_seq);
+    const int seg = (int)(runs_inner ? lo_id : hi_id);
+    const int ib  = (int)(blk % (unsigned)nib), g = (int)(blk / (unsigned)nib);
     // This wave's item and 32-column block of its slab. Each SIMD (waves s and
     // s + 4) holds one item; in a block of at most two items (also where the plan
     // asks for two: a grid that would leave half of the CUs idle) their four waves

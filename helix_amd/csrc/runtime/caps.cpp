@@ -562,7 +562,7 @@ const PlanCost& plan_cost(const helix_scan_desc& d, const HelixMatmulTraits& tr)
 
 // The workgroups of either launch over a group of cpg chunks in runs of len, of
 // `items` items each, in their kernels' logical order (item block, group, run,
-// sequence).
+// sequence; or run, item block, group, sequence: walk_runs_inner).
 struct PlanGrid {
     long per_run;    // item blocks x groups
     int  cpg, len, n_run, n_seq;
@@ -576,7 +576,9 @@ struct PlanGrid {
         weight = (double)ipg * d.n_group / HELIX_HB;
     }
     long total() const { return per_run * n_run * n_seq; }
-    int run_of(long wid) const { return (int)(wid / per_run % n_run); }
+    int run_of(long wid, bool fold) const {
+        return (int)((walk_runs_inner(fold, n_run, n_seq) ? wid : wid / per_run) % n_run);
+    }
     double steps(int r, const DispatchCost& c, bool fold) const {
         return std::min(len, cpg - r * len) + c.o + (fold ? c.g * r : 0.0);
     }
@@ -608,7 +610,7 @@ double makespan(const PlanGrid& g, const DispatchCost& c, bool fold) {
         int m = 0;
         for (int i = 1; i < kCusPerEngine; ++i)
             if (e[i] < e[m]) m = i;
-        e[m] += g.steps(g.run_of(wid), c, fold);
+        e[m] += g.steps(g.run_of(wid, fold), c, fold);
         T = std::max(T, e[m]);
     }
     return T;

@@ -140,6 +140,30 @@ def test_16bit_storage_runs(gpu, shape, knobs, backend, io, items):
     check(io, desc, y, s1, y_ref, s_ref)
 
 
+# Folded runs about the line between the two orders of workgroups: two and three
+# runs, seven and eight sequences, grids past a multiple of eight.
+ORDERS = [(1, 1, 2), (1, 1, 3), (2, 2, 4), (7, 1, 3), (8, 1, 3), (3, 2, 5)]   # sequences, chunks per run, runs
+
+
+@ITEMS
+@pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("S,run_len,runs", ORDERS, ids=["x".join(map(str, o)) for o in ORDERS])
+def test_folded_run_order(gpu, S, run_len, runs, backend, items):
+    p = po.problem_harness(64 * run_len * runs - 5, S, 6, 72, 72, 2, 619, "long")
+    p.s0 = (np.random.default_rng(7).standard_normal(p.s0.shape) * 0.2).astype(np.float32)
+    y_ref, s_ref = po.scan(p, use_ids=False)
+    ctx = ctx_for(gpu, HELIX_WALK_LEN=run_len, HELIX_SEG_LEN=run_len, HELIX_FUSE_B="1", HELIX_F32_WALK="1",
+                  HELIX_WALK_ITEMS=items)
+    d = p.d.copy()
+    d.backend, d.multipass = backend, True
+    info = ctx.run_info(d)
+    assert info.kernel_b is None and (info.run_len, info.runs_per_group) == (run_len, runs)
+    _, y, s1 = run(ctx, p, d)
+    rel, ab = (BF16_REL, BF16_ABS) if backend == HELIX_BACKEND_MPP else (F32_REL, F32_ABS)
+    assert po.allclose_ratio(y, y_ref, rel, ab) <= 1.0
+    assert po.allclose_ratio(s1, s_ref, F32_REL, F32_ABS) <= 1.0
+
+
 @ITEMS
 @pytest.mark.parametrize("backend", [HELIX_BACKEND_SGMMA, HELIX_BACKEND_MPP], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("N", [136, 256])
