@@ -3,8 +3,8 @@
 
 One step = one HELIX scan (Pass A, B, C) over BASELINE.json config 2 with
 inputs resident in HBM, on the bf16 path (bf16 Pass C operands; Pass A on
-bf16x6 split products, which keeps the carried state and s1 fp32-accurate as
-the reference requires; fp32 Pass B). The same workload is also timed on the
+three products of scaled fp16 planes, which keeps the carried state and s1
+fp32-accurate as the reference requires; fp32 Pass B). The same workload is also timed on the
 fp32 path. Timing follows
 the reference protocol (docs/BENCHMARKING.md:48-69): wall-clock warm-up of at
 least 800 ms, events on the launch stream, min / median / spread reported.
@@ -657,7 +657,7 @@ def main():
         "data": "synthetic (BASELINE.json distributions; config 2 on torch RNG seed 1002, config i of the per-config report on seed 1000+i)",
         "config": {
             "workload": "config 2: SSD prefill scan S=1 L=8192 H=64 P=64 N=128 G=8 chunk=64, "
-                        "bf16 Pass C operands, Pass A on bf16x6 split products (carried state and "
+                        "bf16 Pass C operands, Pass A on scaled fp16 planes (carried state and "
                         "s1 at the fp32 per-element bound), fp32 Pass B, inputs resident in HBM",
             "kernel": r["kernel"],
             "plan": {"groups": plan.n_groups, "seg_len": plan.seg_len, "hblk": plan.hblk,
